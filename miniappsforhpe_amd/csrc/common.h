@@ -49,6 +49,38 @@ hip_status(hipError_t e)
     return e == hipSuccess ? TTI_OK : (TTI_EHIP_BASE - (int)e);
 }
 
+constexpr int CUS = 256; // compute units of one MI355X
+
+// z planes per thread block of a z-marching kernel: nz planes of `tiles` x-y tiles cut into equal chunks. A block costs
+// its planes plus `warm` (its prologue and the halo planes it recomputes, in planes), and the grid runs in rounds of
+// `slots` resident blocks, so few deep blocks leave CUs idle (a 64^3 volume in chunks of 128 planes is 16 blocks, each
+// marching 72 planes at 2 us) and a round that is barely begun costs a whole one; many shallow ones recompute halos.
+// Returns the depth of the cheapest number of chunks, none deeper than `cap`; a shallower one has to gain 3% over the
+// best so far, because deeper chunks also read less. A last round of at most one block per CU runs its planes faster
+// (2.05 us against 2.43 us with two blocks per CU in the fused forward kernel).
+inline int
+chunk_depth(int nz, long tiles, int slots, float warm, int cap)
+{
+    int best = 0;
+    float cost = 0.0f;
+    for (int c = (nz + cap - 1) / cap;;) {
+        const int bz = (nz + c - 1) / c;
+        if (best && bz < 2)
+            break;
+        const long n = tiles * ((nz + bz - 1) / bz), r = n % slots;
+        const float rounds = (float)(n / slots) + (r == 0 ? 0.0f : r <= CUS && slots > CUS ? 0.85f : 1.0f);
+        const float t = ((float)bz + warm) * rounds;
+        if (!best || t < 0.97f * cost) {
+            cost = t;
+            best = bz;
+        }
+        if (bz < 2)
+            break;
+        c = (nz + bz - 2) / (bz - 1); // the next number of chunks that makes them shallower
+    }
+    return best;
+}
+
 // Status of the last launch on this thread.
 inline int
 launch_status()

@@ -119,14 +119,15 @@ struct Launch
     int ntx, nty, ntz, bz;
 };
 
+// pass 0: forward, 1: adjoint. Chunks of at most zblock planes (0 = 128), by chunk_depth.
 Launch
-plan(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, int bz, int bx, int by)
+plan(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, int zblock, int bx, int by, int pass)
 {
     Launch L;
     const int nx = ixend - ixbeg + 1, ny = iyend - iybeg + 1, nz = izend - izbeg + 1;
-    L.bz = bz > 0 ? bz : 128;
     L.ntx = (nx + bx - 1) / bx;
     L.nty = (ny + by - 1) / by;
+    L.bz = chunk_depth(nz, (long)L.ntx * L.nty, STEP_SLOTS[pass], STEP_WARM, zblock > 0 ? zblock : 128);
     L.ntz = (nz + L.bz - 1) / L.bz;
     const int nt = L.ntx * L.nty * L.ntz;
     L.grid = dim3(((nt + 7) / 8) * 8); // multiple of 8 so the XCD round-robin decode covers every tile
@@ -172,7 +173,7 @@ tti_fused_fwd_step(const float* field1, const float* field2, float* field1_out, 
         return TTI_EINVAL;
     const unsigned src_off = src_index < 0 ? 0xffffffffu : (unsigned)(src_index * 4);
     const Box g{ ixbeg, ixend, iybeg, iyend, izbeg, izend, (long)ldimx, (long)ldimy, free_surface != 0 };
-    const Launch L = plan(ixbeg, ixend, iybeg, iyend, izbeg, izend, zblock, BX, FWD_BY);
+    const Launch L = plan(ixbeg, ixend, iybeg, iyend, izbeg, izend, zblock, BX, FWD_BY, 0);
     const Snap sn = to_snap(snap);
     auto go = [&](auto kernel) {
         kernel<<<L.grid, dim3(BX, FWD_BY), 0, (hipStream_t)stream>>>(
@@ -222,7 +223,7 @@ tti_fused_adj_step(const float* field1, const float* field2, float* field1_out, 
     if (!small_volume(ldimx, ldimy, izend))
         return TTI_EINVAL;
     const Box g{ ixbeg, ixend, iybeg, iyend, izbeg, izend, (long)ldimx, (long)ldimy, free_surface != 0 };
-    const Launch L = plan(ixbeg, ixend, iybeg, iyend, izbeg, izend, zblock, ADJ_AX, ADJ_AY);
+    const Launch L = plan(ixbeg, ixend, iybeg, iyend, izbeg, izend, zblock, ADJ_AX, ADJ_AY, 1);
     const Snap sn = to_snap(snap);
     auto go = [&](auto kernel) {
         kernel<<<L.grid, dim3(ADJ_AX, ADJ_AY), 0, (hipStream_t)stream>>>(

@@ -1263,6 +1263,14 @@ inject_point(float* __restrict__ u, float* __restrict__ w, float* __restrict__ a
 // Host-side argument checks shared by the launchers
 // ------------------------------------------------------------------------------------------------------------------
 
+// Resident blocks on the whole GPU (two 256-thread forward blocks or one 512-thread adjoint block per CU, by their
+// registers) and the cost of a chunk's 8 recomputed planes and prologue, for chunk_depth; [0] forward, [1] adjoint.
+// Measured over z depths of 2 to 256 planes on volumes of 40^3 to 400^3, a step takes 2.43 us (forward, two blocks per
+// CU; 2.05 us one) and 3.2 us (adjoint) per plane and round within 8%. Against 128-plane chunks throughout: 64^3 149 ->
+// 27 us forward and 193 -> 38 us adjoint, 128^3 281 -> 58 and 359 -> 75 us.
+constexpr int STEP_SLOTS[2] = { 2 * CUS, CUS };
+constexpr float STEP_WARM = 9.5f;
+
 // The fused kernels stage tiles with 16-byte loads: the interior must start on a 4-float boundary, rows must be a
 // multiple of 4 floats and every volume 16-byte aligned.
 inline bool
