@@ -30,8 +30,7 @@ struct EttiCoef
 
 static EttiCoef g_etti_coef = {};
 
-constexpr int EBY = 8;   // tile rows per block
-constexpr int EBZ = 64;  // output planes per block for the z-marching kernels
+constexpr int EBY = 8; // tile rows per block
 
 // D+ / D- over a row or column of an LDS tile (stride S) or a register queue (q[4] = centre).
 template <int S>
@@ -573,18 +572,14 @@ etti_grid(int nx, int ny, int nz, int bz)
     return dim3((nx + BX - 1) / BX, (ny + EBY - 1) / EBY, (nz + bz - 1) / bz);
 }
 
-// z planes per block of the z-marching kernels: the deepest of 256 and 128 that still gives 512 blocks (two per CU),
-// else EBZ (fewer recomputed halo planes per output plane, as the type2 launchers choose). With the XCD order,
-// measured at 512^3: velocity 1.70 -> 1.64 ms, strains 1.79 -> 1.76 ms, mixed interpolations 0.54 -> 0.48 ms.
+// Chunks of the z-marching kernels (see stencil_bz; against 64-plane chunks at 64^3: velocity 76 -> 15 us, strains 58 ->
+// 14, mixed interpolations 29 -> 9 us)
+constexpr Chunk VELOCITY_CHUNK{ 2, 2.0f }, STRAIN_CHUNK{ 2, 4.0f }, MIXED_CHUNK{ 4, 9.0f };
+
 int
-etti_bz(int nx, int ny, int nz)
+etti_bz(int nx, int ny, int nz, Chunk k)
 {
-    for (int bz : { 256, 128 }) {
-        const dim3 g = etti_grid(nx, ny, nz, bz);
-        if ((long)g.x * g.y * g.z >= 512)
-            return bz;
-    }
-    return EBZ;
+    return stencil_bz(R, R + nx - 1, R, R + ny - 1, R, R + nz - 1, k, EBY);
 }
 
 // Runs launch() on `stream`; with ms != NULL it also waits for it and adds its event-measured time to *ms, as the
@@ -622,7 +617,7 @@ template <int XS, int YS, int ZS>
 void
 launch_mixed(const float* g, float* xz, float* yz, int nx, int ny, int nz, long ldx, long ldy, hipStream_t s)
 {
-    const int bz = etti_bz(nx, ny, nz);
+    const int bz = etti_bz(nx, ny, nz, MIXED_CHUNK);
     k_etti_mixed<XS, YS, ZS><<<etti_grid(nx, ny, nz, bz), dim3(BX, EBY), 0, s>>>(g, xz, yz, nx, ny, nz, ldx, ldy, bz,
                                                                                 g_etti_coef);
 }
@@ -682,7 +677,7 @@ vPlainLoop(float* f1, float* f2, float* f3, const float* f4, const float* f5, co
     if (!all_set(p, 11) || !dims_ok(nx, ny, nz, ldimx, ldimy) || !quads_ok(ldimx, p + 3, 6))
         return TTI_EINVAL;
     return timed_launch(milliseconds_v, stream, [&] {
-        const int bz = etti_bz(nx, ny, nz);
+        const int bz = etti_bz(nx, ny, nz, VELOCITY_CHUNK);
         k_etti_velocity<<<etti_grid(nx, ny, nz, bz), dim3(BX, EBY), 0, (hipStream_t)stream>>>(
             f1, f2, f3, f4, f5, f6, f7, f8, f9, M22, zprime, nx, ny, nz, ldimx, ldimy, bz, g_etti_coef, 1.01f,
             2.01f);
@@ -698,7 +693,7 @@ vgPlainLoop(const float* f1, const float* f2, const float* f3, float* d4, float*
     if (!all_set(p, 10) || !dims_ok(nx, ny, nz, ldimx, ldimy) || !quads_ok(ldimx, p, 3))
         return TTI_EINVAL;
     return timed_launch(milliseconds_g, stream, [&] {
-        const int bz = etti_bz(nx, ny, nz);
+        const int bz = etti_bz(nx, ny, nz, STRAIN_CHUNK);
         k_etti_strain<<<etti_grid(nx, ny, nz, bz), dim3(BX, EBY), 0, (hipStream_t)stream>>>(
             f1, f2, f3, d4, d5, d6, d7, d8, d9, zprime, nx, ny, nz, ldimx, ldimy, bz, g_etti_coef, 1.01f, 2.02f);
     });

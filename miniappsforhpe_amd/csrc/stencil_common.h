@@ -77,9 +77,8 @@ struct TileQuads
 } // namespace tti
 
 namespace tti {
-constexpr int BYS = 8;         // rows per block of the reference-structure stencil kernels
-constexpr int BYL = 16;        // rows per block of the light ones (forward derivatives, adjoint update)
-constexpr int BZ_DEFAULT = 64; // z planes per block where no choice below applies
+constexpr int BYS = 8;  // rows per block of the reference-structure stencil kernels
+constexpr int BYL = 16; // rows per block of the light ones (forward derivatives, adjoint update)
 
 // Tile of a stencil block in a (gridDim.x, gridDim.y, gridDim.z) launch in XCD order. The dispatcher hands
 // consecutive blocks (x fastest, then y, then z) to the 8 XCDs in turn; here each XCD instead takes a contiguous range
@@ -128,16 +127,20 @@ stencil_grid(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, i
     return dim3((nx + BX - 1) / BX, (ny + by - 1) / by, (nz + bz - 1) / bz);
 }
 
-// z planes per block of the XCD-ordered kernels: the deepest of 256 and 128 planes that still gives 512 blocks (two
-// per CU), else 64. Deeper chunks recompute fewer halo planes (8 per chunk); at 512^3 the kernels take 256.
-inline int
-stencil_bz(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, int by = BYS)
+// What chunk_depth needs of a z-marching kernel: its resident blocks per CU and the planes' worth of a chunk's prologue
+// and recomputed halo, both from its sweep over chunk depths of 2 to 256 planes at 64^3 to 320 x 288 x 240. The deepest
+// chunk is 256 planes (4% more reads at 128; no faster at 512).
+struct Chunk
 {
-    for (int bz : { 256, 128 }) {
-        const dim3 g = stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz, by);
-        if ((long)g.x * g.y * g.z >= 512)
-            return bz;
-    }
-    return BZ_DEFAULT;
+    int per_cu;
+    float warm;
+    int cap = 256;
+};
+
+inline int
+stencil_bz(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, Chunk k, int by = BYS)
+{
+    const dim3 g = stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, 1, by);
+    return chunk_depth((int)g.z, (long)g.x * g.y, k.per_cu * CUS, k.warm, k.cap);
 }
 } // namespace tti

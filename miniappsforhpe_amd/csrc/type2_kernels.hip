@@ -16,6 +16,15 @@
 
 namespace tti {
 
+// {resident blocks per CU, planes' worth of a chunk's prologue and halo, deepest chunk} of the launchers below. Against
+// chunks of 64 planes on grids too small for 512 deeper ones, at 64^3: derivatives 70 -> 30 us (then host time), update
+// 122 -> 21, adjoint derivatives 143 -> 36, adjoint update 70 -> 15, density gradient 149 -> 19 us.
+constexpr Chunk FWD_DRV_CHUNK{ 1, 4.0f }, FWD_UPDATE_CHUNK{ 1, 9.5f }, ADJ_DRV_CHUNK{ 1, 9.0f },
+    RHO_GRAD_CHUNK{ 1, 3.0f };
+// the adjoint update runs in dispatch order, where chunks over 64 planes read more (1.37 ms at 64, 1.43 at 256, 512^3)
+constexpr Chunk ADJ_UPDATE_CHUNK{ 1, 4.0f, 64 };
+
+
 // ------------------------------------------------------------------------------------------------------------------
 // a2: d_a f = b * D-_a f  (kernels/kernel_type2_fwd_drv.cu:148-362; launcher :368-409)
 // ------------------------------------------------------------------------------------------------------------------
@@ -1747,7 +1756,7 @@ launch_fwd_kernel2_drv(const float* field1, const float* field2, const float* Mo
     if (!field1 || !field2 || !Model11 || !dfield1dx || !dfield1dy || !dfield1dz || !dfield2dx || !dfield2dy ||
         !dfield2dz || !ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, BYL);
+    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, FWD_DRV_CHUNK, BYL);
     auto kern = quads_fit(ixbeg, ldimx, { field1, field2 }) ? k_fwd_drv_q<BYL> : k_fwd_drv<BYL>;
     kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz, BYL), dim3(BX, BYL), 0, (hipStream_t)stream>>>(
         field1, field2, Model11, dfield1dx, dfield1dy, dfield1dz, dfield2dx, dfield2dy, dfield2dz, ixbeg, ixend, iybeg,
@@ -1790,7 +1799,7 @@ launch_update_rho_fwd_main_loop_2_1(float* field3, float* field4, const float* f
     const float invdx = (float)(1.0 / dx), invdy = (float)(1.0 / dy), invdz = (float)(1.0 / dz);
     const float invdxdy = (float)(1.0 / (4 * dx * dy)), invdydz = (float)(1.0 / (4 * dy * dz)),
                 invdzdx = (float)(1.0 / (4 * dx * dz));
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend);
+    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, FWD_UPDATE_CHUNK);
     auto kern = quads_fit(ixbeg, ldimx, { field1, field2, field1_dx, field2_dx, field1_dy, field2_dy })
                     ? k_fwd_update_q<BYS>
                     : k_fwd_update<BYS>;
@@ -1824,7 +1833,7 @@ launch_adj_kernel2_drv(float* dfield1dx, float* dfield2dx, float* dfield1dy, flo
                              invdx, invdy, invdz, stream);
     if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend);
+    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, ADJ_DRV_CHUNK);
     const bool q = quads_fit(ixbeg, ldimx,
                              { field1, field2, Model11, model1, model2, model3, model4, model5, model6, model7 });
     auto kern = q ? k_adj_drv_q<BYS> : k_adj_drv<BYS>;
@@ -1860,7 +1869,7 @@ launch_update_adj_kernel_main_3(float* field3, float* field4, const float* field
     if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
     const float invdx = (float)(1.0 / dx), invdy = (float)(1.0 / dy), invdz = (float)(1.0 / dz);
-    const int bz = BZ_DEFAULT; // plain dispatch order, 64-plane chunks: the fastest measured for this kernel
+    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, ADJ_UPDATE_CHUNK, BYL); // plain dispatch order
     const dim3 grid = stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz, BYL);
     const bool q = quads_fit(ixbeg, ldimx, { field1_dx, field2_dx, field1_dy, field2_dy });
     auto kern = sponge_active ? (q ? k_adj_update_q<BYL, true> : k_adj_update<BYL, true>)
@@ -1905,7 +1914,7 @@ launch_update_rho_gradient_rho(float* grad, const float* fwd_field1_dx, const fl
     if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
     const float hx = (float)(1.0 / dx), hy = (float)(1.0 / dy), hz = (float)(1.0 / dz);
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend);
+    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, RHO_GRAD_CHUNK);
     const bool q = quads_fit(ixbeg, ldimx, { fwd_field1_dx, fwd_field2_dx, fwd_field1_dy, fwd_field2_dy, field1, field2,
                                             irho, model1, model2, model3, model4, rx, ry });
     auto kern = q ? k_rho_grad_q<BYS> : k_rho_grad<BYS>;
@@ -1934,7 +1943,7 @@ rho_gradient_f64(double* grad, const float* fwd_field1_dx, const float* fwd_fiel
         grad_ldimx < ixend - ixbeg + 1 || grad_ldimy < iyend - iybeg + 1)
         return TTI_EINVAL;
     const float hx = (float)(1.0 / dx), hy = (float)(1.0 / dy), hz = (float)(1.0 / dz);
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend);
+    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, RHO_GRAD_CHUNK);
     const bool q = quads_fit(ixbeg, ldimx, { fwd_field1_dx, fwd_field2_dx, fwd_field1_dy, fwd_field2_dy, field1, field2,
                                             irho, model1, model2, model3, model4, rx, ry });
     auto kern = q ? k_rho_grad_q<BYS, double> : k_rho_grad<BYS, double>;

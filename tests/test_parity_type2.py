@@ -154,6 +154,37 @@ def test_rho_gradient(shape, rng, cuda):
     assert rel_l2(from_gpu(gg) - g0, go - g0) < 1e-5
 
 
+@pytest.mark.parametrize("shape", [(1030, 140, 21), (65, 9, 1), (5, 3, 2)])
+def test_steps_at_both_ends_of_the_chunk_rule(shape, rng, cuda):
+    """The launchers cut z into the chunks that fill the GPU: 17 x 18 tiles keep 21 planes in one chunk (planes marched
+    past the register queues' length), one or a few planes leave the shortest ones. A forward and an adjoint step."""
+    import torch
+
+    from miniappsforhpe_amd.propagator import TTIPropagator
+
+    G, OG = grid_pair(shape)
+    m = make_models(G, rng)
+    f1, f2, u, w = (f32(rng.standard_normal(G.shape)) for _ in range(4))
+    sp = tuple(rng.uniform(0.9, 1.0, (n, 2)).astype(np.float32) for n in (G.ldx, G.ldy, G.ldz))
+    P = TTIPropagator(G, [to_gpu(x, cuda) for x in m], DX, DY, DZ, 4e-4, sponge=[torch.from_numpy(a) for a in sp],
+                      device=cuda)
+    for step in ("fwd", "adj"):
+        for dst, src in zip((*P.sigma, P.u, P.w), (f1, f2, u, w)):
+            dst.copy_(to_gpu(src, cuda))
+        for t in P.scratch():
+            t.zero_()
+        o = [x.copy() for x in (f1, f2, u, w)]
+        d = [OG.zeros() for _ in range(8)]
+        if step == "fwd":
+            P.step_fwd_plain()
+            O.step_fwd(OG, *o, m, d[:6], sp, O.f32(4e-4), DX, DY, DZ)
+        else:
+            P.step_adj_plain()
+            O.step_adj(OG, *o, m, d, sp, O.f32(4e-4), DX, DY, DZ, sponge_active=True)
+        for name, got, ref in zip(("f1", "f2", "u", "w"), (*P.sigma, P.u, P.w), o):
+            assert rel_l2(from_gpu(got), ref) < 1e-5, (step, name)
+
+
 @pytest.mark.parametrize("shape", SHAPES[:2])
 def test_pointwise_kernels(shape, rng, cuda):
     from miniappsforhpe_amd import ops
