@@ -4,11 +4,66 @@
 #include <cstdint>
 #include <initializer_list>
 
-#include "common.h"
+#include "fd_tables.h"
 
 namespace tti {
 
 constexpr int BX = 64;
+
+// x halo of a quad-staged tile of stencil radius RO: a whole number of quads, so the tile's rows start aligned
+__host__ __device__ constexpr int
+halo_x(int ro)
+{
+    return (ro + 3) / 4 * 4;
+}
+
+// Element offset of plane z, uniform over the wave and opaque to the optimiser: otherwise loop strength reduction turns
+// base + z ldx ldy into one 64-bit per-lane pointer for every volume, two VGPRs each and a 64-bit vector add per plane.
+__device__ __forceinline__ long
+plane_off(int z, long sz)
+{
+    const long v = (long)z * sz;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32));
+    return (long)(((unsigned long)hi << 32) | lo);
+}
+
+// A lane offset, opaque in the block that uses it: instruction selection works block by block and folds a 32-bit offset
+// into a load with a scalar base only where it sees the offset's extension to 64 bits, which is otherwise hoisted out
+// of the loop (and every load then takes a 64-bit vector add).
+__device__ __forceinline__ unsigned
+here(unsigned off)
+{
+    asm volatile("" : "+v"(off));
+    return off;
+}
+
+// Keeps v where it is computed: without it the compiler sinks a plane's sums to the end of the loop body, past the
+// next plane's work, with every LDS word they need held in registers until then.
+__device__ __forceinline__ void
+pin(float& v)
+{
+    asm volatile("" : "+v"(v));
+}
+
+// Words of a plane: `plane` is a scalar (the volume plus a uniform plane or tile-origin offset), `off` a 32-bit byte
+// offset of the lane, so a load needs one address register and no 64-bit vector arithmetic (64-bit offsets made the
+// compiler keep one pointer per volume and lane: 222 VGPRs for the forward update where 18 volumes are touched).
+__device__ __forceinline__ float
+ldp(const float* __restrict__ plane, unsigned off)
+{
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(plane) + off);
+}
+__device__ __forceinline__ float4
+ldp4(const float* __restrict__ plane, unsigned off) // 16-byte aligned
+{
+    return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(plane) + off);
+}
+__device__ __forceinline__ void
+stp(float* __restrict__ plane, unsigned off, float v)
+{
+    *reinterpret_cast<float*>(reinterpret_cast<char*>(plane) + off) = v;
+}
 
 // Cooperative load of one plane tile with halos into LDS. `origin` is the global index of tile element (0, 0), i.e.
 // of the point (x0 - HX, y0 - HY, z). Elements whose tile column is >= xlim or row >= ylim are set to zero (they
@@ -37,9 +92,9 @@ template <int W, int H, int NT>
 struct TileQuads
 {
     static constexpr int QPR = W / 4, NQ = QPR * H, QT = (NQ + NT - 1) / NT;
-    long off[QT]; // element offset from the tile origin within a plane, -1: not loaded
-    int lds[QT];  // first element of the quad in the W x H LDS tile, -1: no quad for this slot
-    int keep[QT]; // elements of the quad inside xlim (0..4)
+    unsigned off[QT]; // byte offset from the tile origin within a plane
+    int lds[QT];      // first element of the quad in the W x H LDS tile, -1: no quad for this slot
+    int keep[QT];     // elements of the quad inside xlim (0..4; 0: not loaded)
 
     __device__ TileQuads(int tid, long ldx, int xlim, int ylim)
     {
@@ -50,15 +105,15 @@ struct TileQuads
             const bool has = q < NQ;
             lds[k] = has ? row * W + lx : -1;
             keep[k] = has && row < ylim ? min(max(xlim - lx, 0), 4) : 0;
-            off[k] = keep[k] > 0 ? (long)row * ldx + lx : -1;
+            off[k] = ((unsigned)row * (unsigned)ldx + (unsigned)lx) * 4u;
         }
     }
     __device__ __forceinline__ void fetch(float4 (&r)[QT], const float* __restrict__ origin) const
     {
 #pragma unroll
         for (int k = 0; k < QT; ++k)
-            if (off[k] >= 0)
-                r[k] = *reinterpret_cast<const float4*>(origin + off[k]);
+            if (keep[k] > 0)
+                r[k] = ldp4(origin, here(off[k]));
     }
     __device__ __forceinline__ void commit(float* tile, const float4 (&r)[QT]) const
     {
@@ -97,22 +152,23 @@ stencil_tile(int& bx, int& by, int& bz)
     bz = t / (gx * gy);
 }
 
-// Validates the ghost requirement of the radius-4 stencils: the interior must sit at least 4 points inside the
+// Validates the ghost requirement of the radius-ro stencils: the interior must sit at least ro points inside the
 // allocated x and y extents (the z extent is the caller's contract, as in the reference launchers).
 inline bool
-ranges_ok(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, int ldimx, int ldimy)
+ranges_ok(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, int ldimx, int ldimy, int ro = R)
 {
-    return ixbeg >= R && iybeg >= R && izbeg >= R && ixend >= ixbeg && iyend >= iybeg && izend >= izbeg &&
-           ixend + R < ldimx && iyend + R < ldimy;
+    return ixbeg >= ro && iybeg >= ro && izbeg >= ro && ixend >= ixbeg && iyend >= iybeg && izend >= izbeg &&
+           ixend + ro < ldimx && iyend + ro < ldimy;
 }
 
-// Whether the quad-staged kernels apply: tile origins (ixbeg - 4 + 64 k) and rows (ldimx) a multiple of 4 floats and
-// every tile source 16-byte aligned, so each tile quad is one aligned float4 load. Otherwise the launchers use the
+// Whether the quad-staged kernels apply: tile origins (ixbeg - 4 or - 8 + 64 k) and rows (ldimx) a multiple of 4 floats and
+// every tile source 16-byte aligned, so each tile quad is one aligned float4 load, and planes of less than 4 GiB, which
+// they address with 32-bit byte offsets. Otherwise the launchers use the
 // element-wise kernels.
 inline bool
-quads_fit(int ixbeg, int ldimx, std::initializer_list<const float*> tiles)
+quads_fit(int ixbeg, int ldimx, int ldimy, std::initializer_list<const float*> tiles)
 {
-    if (ixbeg % 4 || ldimx % 4)
+    if (ixbeg % 4 || ldimx % 4 || (long)ldimx * ldimy >= (1L << 30))
         return false;
     for (const float* p : tiles)
         if (reinterpret_cast<uintptr_t>(p) % 16)

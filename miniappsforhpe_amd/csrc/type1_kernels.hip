@@ -327,7 +327,8 @@ __global__ __launch_bounds__(BX* BY) void k_t1_fwd_q(
     const long sz = ldx * ldy;
     const int xlim = min(W, ixend + R + 1 - (x0 - R));
     const int ylim = min(H, iyend + R + 1 - (y0 - R));
-    const long col = (long)iy * ldx + ix;
+    // byte offset within a plane (inactive lanes: the plane's first word)
+    const unsigned colb = active ? ((unsigned)iy * (unsigned)ldx + (unsigned)ix) * 4u : 0u;
     const int p0 = z0 - R, pend = z1 + R; // tile planes p in [p0, pend), output o = p - R
     const TileQuads<W, H, NT> qt(tid, ldx, xlim, ylim);
     const long org = (long)(y0 - R) * ldx + (x0 - R);
@@ -344,17 +345,17 @@ __global__ __launch_bounds__(BX* BY) void k_t1_fwd_q(
     float pw[9]; // m1..m7, u, w of the output plane being finalised
     auto load_pw = [&](int o) {
         if (active && o >= z0 && o < z1) {
-            const long i = (long)o * sz + col;
-            pw[0] = m1[i];
-            pw[1] = m2[i];
-            pw[2] = m3[i];
-            pw[3] = m4[i];
-            pw[4] = m5[i];
-            pw[5] = m6[i];
-            pw[6] = m7[i];
+            const long i = (long)o * sz;
+            pw[0] = ldp(m1 + i, colb);
+            pw[1] = ldp(m2 + i, colb);
+            pw[2] = ldp(m3 + i, colb);
+            pw[3] = ldp(m4 + i, colb);
+            pw[4] = ldp(m5 + i, colb);
+            pw[5] = ldp(m6 + i, colb);
+            pw[6] = ldp(m7 + i, colb);
             if (MODE != 2) {
-                pw[7] = u[i];
-                pw[8] = w[i];
+                pw[7] = ldp(u + i, colb);
+                pw[8] = ldp(w + i, colb);
             }
         }
     };
@@ -455,9 +456,9 @@ __global__ __launch_bounds__(BX* BY) void k_t1_fwd_q(
                 u[oi] = un;
                 w[oi] = wn;
             } else {
-                const long i = (long)o * sz + col;
-                u[i] = un;
-                w[i] = wn;
+                const long i = (long)o * sz;
+                stp(u + i, colb, un);
+                stp(w + i, colb, wn);
             }
         }
 #pragma unroll
@@ -516,27 +517,29 @@ __global__ __launch_bounds__(BX* BY) void k_t1_adj_q(
     const long sz = ldx * ldy;
     const int xlim = min(W, ixend + R + 1 - (x0 - R));
     const int ylim = min(H, iyend + R + 1 - (y0 - R));
-    const long col = (long)iy * ldx + ix;
+    // byte offset within a plane (inactive lanes: the plane's first word)
+    const unsigned colb = active ? ((unsigned)iy * (unsigned)ldx + (unsigned)ix) * 4u : 0u;
     const int p0 = z0 - R, pend = z1 + R;
 
     const bool qhas = tid < NQ;
     const int qr = tid / QPR, ql = 4 * (tid - qr * QPR);
     const int qkeep = qhas && qr < ylim ? min(max(xlim - ql, 0), 4) : 0;
-    const long qoff = (long)(y0 - R + qr) * ldx + (x0 - R + ql);
+    const unsigned qoff = ((unsigned)qr * (unsigned)ldx + (unsigned)ql) * 4u; // bytes from the tile origin
+    const long org = (long)(y0 - R) * ldx + (x0 - R);
     const bool qrow = qr >= R && qr < R + BY, qcol = ql >= R && ql < R + BX;
     float4 v1, v2, vm1, vm2, vm3, vm4, vm5, vm6, vm7;
     auto fetch = [&](int p) {
         if (qkeep > 0) {
-            const long g = (long)p * sz + qoff;
-            v1 = *reinterpret_cast<const float4*>(f1 + g);
-            v2 = *reinterpret_cast<const float4*>(f2 + g);
-            vm1 = *reinterpret_cast<const float4*>(m1 + g);
-            vm2 = *reinterpret_cast<const float4*>(m2 + g);
-            vm3 = *reinterpret_cast<const float4*>(m3 + g);
-            vm4 = *reinterpret_cast<const float4*>(m4 + g);
-            vm5 = *reinterpret_cast<const float4*>(m5 + g);
-            vm6 = *reinterpret_cast<const float4*>(m6 + g);
-            vm7 = *reinterpret_cast<const float4*>(m7 + g);
+            const long g = (long)p * sz + org;
+            v1 = ldp4(f1 + g, qoff);
+            v2 = ldp4(f2 + g, qoff);
+            vm1 = ldp4(m1 + g, qoff);
+            vm2 = ldp4(m2 + g, qoff);
+            vm3 = ldp4(m3 + g, qoff);
+            vm4 = ldp4(m4 + g, qoff);
+            vm5 = ldp4(m5 + g, qoff);
+            vm6 = ldp4(m6 + g, qoff);
+            vm7 = ldp4(m7 + g, qoff);
         }
     };
     auto commit = [&](int bf) {
@@ -599,8 +602,8 @@ __global__ __launch_bounds__(BX* BY) void k_t1_adj_q(
     float pu = 0.0f, pwv = 0.0f; // u, w of the output plane being finalised
     auto load_pw = [&](int o) {
         if (active && o >= z0 && o < z1) {
-            pu = u[(long)o * sz + col];
-            pwv = w[(long)o * sz + col];
+            pu = ldp(u + (long)o * sz, colb);
+            pwv = ldp(w + (long)o * sz, colb);
         }
     };
 
@@ -690,9 +693,9 @@ __global__ __launch_bounds__(BX* BY) void k_t1_adj_q(
         }
         load_pw(o + 1);
         if (active && o >= z0) {
-            const long i = (long)o * sz + col;
-            u[i] = un;
-            w[i] = wn;
+            const long i = (long)o * sz;
+            stp(u + i, colb, un);
+            stp(w + i, colb, wn);
         }
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -753,7 +756,7 @@ fwd_main_loop_2_1_inner_gpu_launch(float* field3, float* field4, const float* fi
     const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, T1_CHUNK);
     const dim3 grid = stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz);
     hipStream_t s = (hipStream_t)stream;
-    if (quads_fit(ixbeg, ldimx_in, { field1, field2, model1, model2, model3, model4, model5, model6, model7 })) {
+    if (quads_fit(ixbeg, ldimx_in, ldimy_in, { field1, field2, model1, model2, model3, model4, model5, model6, model7 })) {
         auto kern = calc_snap ? k_t1_fwd_q<BYS, 2> : sponge ? k_t1_fwd_q<BYS, 1> : k_t1_fwd_q<BYS, 0>;
         kern<<<grid, dim3(BX, BYS), 0, s>>>(field3, field4, field1, field2, model1, model2, model3, model4, model5,
                                             model6, model7, sponge ? (const ab2*)ABx : nullptr,
@@ -809,7 +812,7 @@ adj_main_loop_2_inner_gpu_launch(float* field3, float* field4, const float* fiel
     const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, T1_CHUNK);
     const dim3 grid = stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz);
     hipStream_t s = (hipStream_t)stream;
-    if (quads_fit(ixbeg, ldimx, { field1, field2, model1, model2, model3, model4, model5, model6, model7 })) {
+    if (quads_fit(ixbeg, ldimx, ldimy, { field1, field2, model1, model2, model3, model4, model5, model6, model7 })) {
         auto kern = sponge ? k_t1_adj_q<BYS, true> : k_t1_adj_q<BYS, false>;
         kern<<<grid, dim3(BX, BYS), 0, s>>>(field3, field4, field1, field2, model1, model2, model3, model4, model5,
                                             model6, model7, sponge ? (const ab2*)ABx : nullptr,

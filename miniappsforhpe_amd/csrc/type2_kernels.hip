@@ -23,7 +23,26 @@ constexpr Chunk FWD_DRV_CHUNK{ 1, 4.0f }, FWD_UPDATE_CHUNK{ 1, 9.5f }, ADJ_DRV_C
     RHO_GRAD_CHUNK{ 1, 3.0f };
 // the adjoint update runs in dispatch order, where chunks over 64 planes read more (1.37 ms at 64, 1.43 at 256, 512^3)
 constexpr Chunk ADJ_UPDATE_CHUNK{ 1, 4.0f, 64 };
+// order 16: 16 halo planes
+constexpr Chunk FWD_DRV16_CHUNK{ 1, 6.0f }, FWD_UPDATE16_CHUNK{ 1, 17.5f }, ADJ_DRV16_CHUNK{ 1, 17.0f },
+    ADJ_UPDATE16_CHUNK{ 1, 6.0f, 64 };
 
+
+// Moves the queue of mixed partial sums one plane on and absorbs the differences d[1..RO] of that plane, in one FMA per
+// slot: afterwards q[j] belongs to output plane p - RO + j (plane p at offset +n feeds output p - n, at -n output p + n
+// with the sign flipped). Slots go upwards, so each is read by its left neighbour before it is written.
+template <int RO>
+__device__ __forceinline__ void
+absorb(float (&q)[2 * RO + 1], const float (&d)[RO + 1])
+{
+#pragma unroll
+    for (int j = 0; j <= 2 * RO; ++j) {
+        const int n = j < RO ? RO - j : j - RO;
+        const float e = j < RO ? FD<RO>::e[n] : -FD<RO>::e[n], next = j < 2 * RO ? q[j + 1] : 0.0f;
+        q[j] = n ? fmaf(e, d[n], next) : next;
+        pin(q[j]);
+    }
+}
 
 // ------------------------------------------------------------------------------------------------------------------
 // a2: d_a f = b * D-_a f  (kernels/kernel_type2_fwd_drv.cu:148-362; launcher :368-409)
@@ -100,7 +119,7 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_drv(const float* __restrict__ f1
 // The same operator with the plane pipeline: the sigma tiles of plane z + 1 are loaded as float4 quads during plane
 // z - 1 and stored into the other LDS buffer during plane z; the column words (sigma at z + 4, b at z + 1) one plane
 // ahead; one barrier per plane. Needs quads_fit (launcher falls back).
-template <int BY>
+template <int BY, int RO>
 __global__ __launch_bounds__(BX* BY) void k_fwd_drv_q(const float* __restrict__ f1, const float* __restrict__ f2,
                                                       const float* __restrict__ b, float* __restrict__ d1x,
                                                       float* __restrict__ d1y, float* __restrict__ d1z,
@@ -109,7 +128,7 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_drv_q(const float* __restrict__ 
                                                       int iyend, int izbeg, int izend, float invdx, float invdy,
                                                       float invdz, long ldx, long ldy, int bz)
 {
-    constexpr int W = BX + 2 * R, H = BY + 2 * R, NT = BX * BY;
+    constexpr int HX = halo_x(RO), W = BX + 2 * HX, H = BY + 2 * RO, NT = BX * BY;
     __shared__ __align__(16) float t1[2][H][W];
     __shared__ __align__(16) float t2[2][H][W];
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
@@ -120,28 +139,29 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_drv_q(const float* __restrict__ 
     const int ix = x0 + tx, iy = y0 + ty;
     const bool active = ix <= ixend && iy <= iyend;
     const long sz = ldx * ldy;
-    const int xlim = min(W, ixend + R + 1 - (x0 - R));
-    const int ylim = min(H, iyend + R + 1 - (y0 - R));
-    const long col = (long)iy * ldx + ix;
+    const int xlim = min(W, ixend + RO + 1 - (x0 - HX));
+    const int ylim = min(H, iyend + RO + 1 - (y0 - RO));
+    // byte offset within a plane (inactive lanes: the plane's first word)
+    const unsigned colb = active ? ((unsigned)iy * (unsigned)ldx + (unsigned)ix) * 4u : 0u;
     const TileQuads<W, H, NT> qt(tid, ldx, xlim, ylim);
-    const long org = (long)(y0 - R) * ldx + (x0 - R);
+    const long org = (long)(y0 - RO) * ldx + (x0 - HX);
     float4 r1[qt.QT], r2[qt.QT];
     auto fetch = [&](int z) {
         qt.fetch(r1, f1 + (long)z * sz + org);
         qt.fetch(r2, f2 + (long)z * sz + org);
     };
 
-    float q1[8], q2[8]; // q[k] = f(z - 4 + k)
+    float q1[2 * RO], q2[2 * RO]; // q[k] = f(z - RO + k)
 #pragma unroll
-    for (int k = 0; k < 7; ++k) {
-        q1[k] = active ? f1[(long)(z0 - 4 + k) * sz + col] : 0.0f;
-        q2[k] = active ? f2[(long)(z0 - 4 + k) * sz + col] : 0.0f;
+    for (int k = 0; k < 2 * RO - 1; ++k) {
+        q1[k] = ldp(f1 + (long)(z0 - RO + k) * sz, colb);
+        q2[k] = ldp(f2 + (long)(z0 - RO + k) * sz, colb);
     }
-    float n1 = 0.0f, n2 = 0.0f, nb = 0.0f; // sigma(z + 3) and b(z) of the next plane
+    float n1 = 0.0f, n2 = 0.0f, nb = 0.0f; // sigma(z + RO - 1) and b(z) of the next plane
     if (active) {
-        n1 = f1[(long)(z0 + 3) * sz + col];
-        n2 = f2[(long)(z0 + 3) * sz + col];
-        nb = b[(long)z0 * sz + col];
+        n1 = ldp(f1 + (long)(z0 + RO - 1) * sz, colb);
+        n2 = ldp(f2 + (long)(z0 + RO - 1) * sz, colb);
+        nb = ldp(b + (long)z0 * sz, colb);
     }
     fetch(z0);
     qt.commit(&t1[0][0][0], r1);
@@ -151,13 +171,13 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_drv_q(const float* __restrict__ 
     __syncthreads();
     for (int z = z0; z < z1; ++z) {
         const int bf = (z - z0) & 1;
-        q1[7] = n1;
-        q2[7] = n2;
+        q1[2 * RO - 1] = n1;
+        q2[2 * RO - 1] = n2;
         const float bb = nb;
         if (active && z + 1 < z1) {
-            n1 = f1[(long)(z + 4) * sz + col];
-            n2 = f2[(long)(z + 4) * sz + col];
-            nb = b[(long)(z + 1) * sz + col];
+            n1 = ldp(f1 + (long)(z + RO) * sz, colb);
+            n2 = ldp(f2 + (long)(z + RO) * sz, colb);
+            nb = ldp(b + (long)(z + 1) * sz, colb);
         }
         if (z + 1 < z1) {
             qt.commit(&t1[bf ^ 1][0][0], r1);
@@ -170,25 +190,25 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_drv_q(const float* __restrict__ 
             const float(*T2)[W] = t2[bf];
             float ax1 = 0, ay1 = 0, az1 = 0, ax2 = 0, ay2 = 0, az2 = 0;
 #pragma unroll
-            for (int n = 1; n <= R; ++n) {
-                const float c = cstg(n);
-                ax1 += c * (T1[ty + R][tx + R + n - 1] - T1[ty + R][tx + R - n]);
-                ay1 += c * (T1[ty + R + n - 1][tx + R] - T1[ty + R - n][tx + R]);
-                az1 += c * (q1[R + n - 1] - q1[R - n]);
-                ax2 += c * (T2[ty + R][tx + R + n - 1] - T2[ty + R][tx + R - n]);
-                ay2 += c * (T2[ty + R + n - 1][tx + R] - T2[ty + R - n][tx + R]);
-                az2 += c * (q2[R + n - 1] - q2[R - n]);
+            for (int n = 1; n <= RO; ++n) {
+                const float c = FD<RO>::c[n];
+                ax1 += c * (T1[ty + RO][tx + HX + n - 1] - T1[ty + RO][tx + HX - n]);
+                ay1 += c * (T1[ty + RO + n - 1][tx + HX] - T1[ty + RO - n][tx + HX]);
+                az1 += c * (q1[RO + n - 1] - q1[RO - n]);
+                ax2 += c * (T2[ty + RO][tx + HX + n - 1] - T2[ty + RO][tx + HX - n]);
+                ay2 += c * (T2[ty + RO + n - 1][tx + HX] - T2[ty + RO - n][tx + HX]);
+                az2 += c * (q2[RO + n - 1] - q2[RO - n]);
             }
-            const long i = (long)z * sz + col;
-            d1x[i] = ax1 * invdx * bb;
-            d1y[i] = ay1 * invdy * bb;
-            d1z[i] = az1 * invdz * bb;
-            d2x[i] = ax2 * invdx * bb;
-            d2y[i] = ay2 * invdy * bb;
-            d2z[i] = az2 * invdz * bb;
+            const long i = (long)z * sz;
+            stp(d1x + i, colb, ax1 * invdx * bb);
+            stp(d1y + i, colb, ay1 * invdy * bb);
+            stp(d1z + i, colb, az1 * invdz * bb);
+            stp(d2x + i, colb, ax2 * invdx * bb);
+            stp(d2y + i, colb, ay2 * invdy * bb);
+            stp(d2z + i, colb, az2 * invdz * bb);
         }
 #pragma unroll
-        for (int k = 0; k < 7; ++k) {
+        for (int k = 0; k < 2 * RO - 1; ++k) {
             q1[k] = q1[k + 1];
             q2[k] = q2[k + 1];
         }
@@ -353,11 +373,16 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_update(
 }
 
 // The same operator with the plane pipeline of the gfx950 stencils: the tiles of plane p + 1 (sigma, and the d_x / d_y
-// tiles of output plane p + 1 - 4) are loaded as float4 quads during plane p - 1 and stored into the other LDS buffer
-// during plane p, the d_z column word and the 11 pointwise words of the next output plane are loaded one plane ahead,
-// and one barrier per plane separates a buffer's last read from its refill. Needs quads_fit (launcher falls back).
-template <int BY>
-__global__ __launch_bounds__(BX* BY) void k_fwd_update_q(
+// tiles of output plane p + 1 - RO) are loaded as float4 quads during plane p - 1 and stored into the other LDS buffer
+// during plane p, the d_z column word and the pointwise words of the next output plane are loaded one plane ahead, and
+// one barrier per plane separates a buffer's last read from its refill. Needs quads_fit (launcher falls back).
+// One thread per column and field (threadIdx.z): the z queues of one field fit 88 VGPRs (124 at RO = 8, where both
+// fields in one thread spilled 93 of 256), so 16 waves are resident per CU instead of 8. u needs V2 and w needs H1 of
+// the other field's thread: they pass through LDS and a plane's update is finished after the barrier that ends it.
+// It is bound by HBM at 512^3 (2.48 ms with one thread per column, 2.53 ms; 80 B a point at the copy rate: 2.16 ms) and
+// by latency below (256^3 335 -> 317 us, 301 x 217 x 190 280 -> 272 us); order 16 at 200 x 168 x 144 419 -> 163 us.
+template <int BY, int RO>
+__global__ __launch_bounds__(2 * BX* BY) void k_fwd_update_q(
     float* __restrict__ u, float* __restrict__ w, const float* __restrict__ d1x, const float* __restrict__ d2x,
     const float* __restrict__ d1y, const float* __restrict__ d2y, const float* __restrict__ d1z,
     const float* __restrict__ d2z, const float* __restrict__ f1, const float* __restrict__ f2,
@@ -367,14 +392,13 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_update_q(
     int izbeg, int izend, long ldx, long ldy, float dt, float invdx, float invdy, float invdz, float invdxdy,
     float invdydz, float invdzdx, int bz)
 {
-    constexpr int W = BX + 2 * R, H = BY + 2 * R, NT = BX * BY;
-    __shared__ __align__(16) float s1[2][H][W]; // sigma at plane p (halo 4 in x and y)
-    __shared__ __align__(16) float s2[2][H][W];
-    __shared__ __align__(16) float x1[2][BY][W]; // d_x at plane o (halo 4 in x)
-    __shared__ __align__(16) float x2[2][BY][W];
-    __shared__ __align__(16) float y1[2][H][BX]; // d_y at plane o (halo 4 in y)
-    __shared__ __align__(16) float y2[2][H][BX];
+    constexpr int HX = halo_x(RO), W = BX + 2 * HX, H = BY + 2 * RO, NT = BX * BY;
+    __shared__ __align__(16) float ls[2][2][H][W];   // [plane parity][field] sigma at plane p (halos in x and y)
+    __shared__ __align__(16) float lx[2][2][BY][W];  // d_x at plane o (halo in x)
+    __shared__ __align__(16) float ly[2][2][H][BX];  // d_y at plane o (halo in y)
+    __shared__ float ex[2][2][BY][BX];               // what the other field's update needs of this one: H1, V2
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
+    const int F = __builtin_amdgcn_readfirstlane(threadIdx.z); // field of this wave
     int bxi, byi, bzi;
     stencil_tile(bxi, byi, bzi);
     const int x0 = ixbeg + bxi * BX, y0 = iybeg + byi * BY, z0 = izbeg + bzi * bz;
@@ -382,190 +406,137 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_update_q(
     const int ix = x0 + tx, iy = y0 + ty;
     const bool active = ix <= ixend && iy <= iyend;
     const long sz = ldx * ldy;
-    const int xlim = min(W, ixend + R + 1 - (x0 - R));
-    const int ylim = min(H, iyend + R + 1 - (y0 - R));
+    const int xlim = min(W, ixend + RO + 1 - (x0 - HX));
+    const int ylim = min(H, iyend + RO + 1 - (y0 - RO));
     const int xlim_c = min(BX, ixend + 1 - x0);
     const int ylim_c = min(BY, iyend + 1 - y0);
-    const long col = (long)iy * ldx + ix;
-    const int p0 = z0 - R, pend = z1 + R; // tile planes p in [p0, pend), output o = p - R
+    // byte offset within a plane (inactive lanes: the plane's first word)
+    const unsigned colb = active ? ((unsigned)iy * (unsigned)ldx + (unsigned)ix) * 4u : 0u;
+    const int p0 = z0 - RO, pend = z1 + RO; // tile planes p in [p0, pend), output o = p - RO
+    // u += dt (m1 H1 + m4 V1 + m2 V2), w += dt (m4 H2 + m3 V2 + m2 H1)
+    const float *const f = F ? f2 : f1, *const dx_ = F ? d2x : d1x, *const dy_ = F ? d2y : d1y,
+                *const dz_ = F ? d2z : d1z, *const mh = F ? m4 : m1, *const mv = F ? m3 : m4;
+    float* const out = F ? w : u;
 
     const TileQuads<W, H, NT> qs(tid, ldx, xlim, ylim);
     const TileQuads<W, BY, NT> qx(tid, ldx, xlim, ylim_c);
     const TileQuads<BX, H, NT> qy(tid, ldx, xlim_c, ylim);
-    const long os = (long)(y0 - R) * ldx + (x0 - R), ox = (long)y0 * ldx + (x0 - R), oy = (long)(y0 - R) * ldx + x0;
-    float4 rs1[qs.QT], rs2[qs.QT], rx1[qx.QT], rx2[qx.QT], ry1[qy.QT], ry2[qy.QT];
+    const long os = (long)(y0 - RO) * ldx + (x0 - HX), ox = (long)y0 * ldx + (x0 - HX), oy = (long)(y0 - RO) * ldx + x0;
+    float4 rs[qs.QT], rx4[qx.QT], ry4[qy.QT];
     auto fetch = [&](int p) {
-        const long pz = (long)p * sz;
-        qs.fetch(rs1, f1 + pz + os);
-        qs.fetch(rs2, f2 + pz + os);
-        if (p - R >= z0) {
-            const long oz = (long)(p - R) * sz;
-            qx.fetch(rx1, d1x + oz + ox);
-            qx.fetch(rx2, d2x + oz + ox);
-            qy.fetch(ry1, d1y + oz + oy);
-            qy.fetch(ry2, d2y + oz + oy);
+        qs.fetch(rs, f + plane_off(p, sz) + os);
+        if (p - RO >= z0) {
+            const long oz = plane_off(p - RO, sz);
+            qx.fetch(rx4, dx_ + oz + ox);
+            qy.fetch(ry4, dy_ + oz + oy);
         }
     };
     auto commit = [&](int p, int b) {
-        qs.commit(&s1[b][0][0], rs1);
-        qs.commit(&s2[b][0][0], rs2);
-        if (p - R >= z0) {
-            qx.commit(&x1[b][0][0], rx1);
-            qx.commit(&x2[b][0][0], rx2);
-            qy.commit(&y1[b][0][0], ry1);
-            qy.commit(&y2[b][0][0], ry2);
+        qs.commit(&ls[b][F][0][0], rs);
+        if (p - RO >= z0) {
+            qx.commit(&lx[b][F][0][0], rx4);
+            qy.commit(&ly[b][F][0][0], ry4);
         }
     };
-    // pointwise words of an output plane: 1/rho, m1..m4, rx, ry, rz, u, w
-    float pw[10];
+    float pw[8]; // pointwise words of an output plane: 1/rho, rx, ry, rz, the three m, u or w
     auto load_pw = [&](int o) {
-        if (active && o >= z0 && o < z1) {
-            const long i = (long)o * sz + col;
-            pw[0] = irho[i];
-            pw[1] = m1[i];
-            pw[2] = m2[i];
-            pw[3] = m3[i];
-            pw[4] = m4[i];
-            pw[5] = rx[i];
-            pw[6] = ry[i];
-            pw[7] = rz[i];
-            pw[8] = u[i];
-            pw[9] = w[i];
+        if (o >= z0 && o < z1) {
+            const long i = plane_off(o, sz);
+            const unsigned c = here(colb);
+            pw[0] = ldp(irho + i, c);
+            pw[1] = ldp(rx + i, c);
+            pw[2] = ldp(ry + i, c);
+            pw[3] = ldp(rz + i, c);
+            pw[4] = ldp(mh + i, c);
+            pw[5] = ldp(mv + i, c);
+            pw[6] = ldp(m2 + i, c);
+            pw[7] = ldp(out + i, c);
         }
     };
 
-    float qzx1[9], qyz1[9], qzx2[9], qyz2[9]; // mixed partial sums: Q[j] <-> output plane p - 4 + j
-    float xy1[5], xy2[5];                     // F_xy delayed: xy[4] = F_xy(p)
-    float dz1[8], dz2[8];                     // dz[k] <-> d_z(p - 7 + k)
+    float qzx[2 * RO + 1], qyz[2 * RO + 1]; // mixed partial sums: Q[j] <-> output plane p - RO + j
+    float xy[RO + 1];                       // F_xy delayed: xy[RO] = F_xy(p)
+    float dz[2 * RO];                       // dz[k] <-> d_z(p - 2 RO + 1 + k)
 #pragma unroll
-    for (int j = 0; j < 9; ++j)
-        qzx1[j] = qyz1[j] = qzx2[j] = qyz2[j] = 0.0f;
+    for (int j = 0; j < 2 * RO + 1; ++j)
+        qzx[j] = qyz[j] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 5; ++j)
-        xy1[j] = xy2[j] = 0.0f;
+    for (int j = 0; j < RO + 1; ++j)
+        xy[j] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        dz1[j] = dz2[j] = 0.0f;
-    float n1z = 0.0f, n2z = 0.0f; // d_z of the next plane
-    if (active) {
-        n1z = d1z[(long)p0 * sz + col];
-        n2z = d2z[(long)p0 * sz + col];
-    }
-    load_pw(p0 - R + 1);
+    for (int j = 0; j < 2 * RO; ++j)
+        dz[j] = 0.0f;
+    float nz = ldp(dz_ + (long)p0 * sz, colb); // d_z of the next plane
+    float part = 0.0f, mc = 0.0f, old = 0.0f;  // own part of the update of the plane before o, m2, u or w there
+    auto finish = [&](int o, int b) {          // plane o, with the other field's part in ex[b]
+        const float r = fmaf(mc, ex[b][F ^ 1][ty][tx], part);
+        if (active)
+            stp(out + plane_off(o, sz), here(colb), fmaf(r, dt, old));
+    };
+    load_pw(p0 - RO + 1);
     fetch(p0);
     commit(p0, 0);
-    if (p0 + 1 < pend)
-        fetch(p0 + 1);
+    fetch(p0 + 1);
     __syncthreads();
 
     for (int p = p0; p < pend; ++p) {
-        const int o = p - R, b = (p - p0) & 1;
-        const bool emit = o >= z0;
-        dz1[7] = n1z;
-        dz2[7] = n2z;
-        if (active && p + 1 < pend) {
-            n1z = d1z[(long)(p + 1) * sz + col];
-            n2z = d2z[(long)(p + 1) * sz + col];
-        }
-        if (p + 1 < pend)
+        const int o = p - RO, b = (p - p0) & 1;
+        dz[2 * RO - 1] = nz;
+        if (p + 1 < pend) {
+            nz = ldp(dz_ + plane_off(p + 1, sz), here(colb));
             commit(p + 1, b ^ 1);
+        }
         if (p + 2 < pend)
             fetch(p + 2);
-        float un = 0.0f, wn = 0.0f;
-        if (active) {
-            const float(*S1)[W] = s1[b];
-            const float(*S2)[W] = s2[b];
+        const float(*S)[W] = ls[b][F];
+        float a = 0, ddx[RO + 1], ddy[RO + 1];
 #pragma unroll
-            for (int j = 0; j < 9; ++j) {
-                const int k = R - j;
-                if (k != 0) {
-                    const int ak = k < 0 ? -k : k;
-                    const float e = ecen(ak);
-                    qzx1[j] += e * (S1[ty + R][tx + R + k] - S1[ty + R][tx + R - k]);
-                    qyz1[j] += e * (S1[ty + R + k][tx + R] - S1[ty + R - k][tx + R]);
-                    qzx2[j] += e * (S2[ty + R][tx + R + k] - S2[ty + R][tx + R - k]);
-                    qyz2[j] += e * (S2[ty + R + k][tx + R] - S2[ty + R - k][tx + R]);
-                }
-            }
-            float a1 = 0, a2 = 0;
-#pragma unroll
-            for (int n = 1; n <= R; ++n) {
-                const float e = ecen(n);
-                a1 += e * ((S1[ty + R + n][tx + R + n] - S1[ty + R - n][tx + R + n]) +
-                           (S1[ty + R - n][tx + R - n] - S1[ty + R + n][tx + R - n]));
-                a2 += e * ((S2[ty + R + n][tx + R + n] - S2[ty + R - n][tx + R + n]) +
-                           (S2[ty + R - n][tx + R - n] - S2[ty + R + n][tx + R - n]));
-            }
-            xy1[4] = a1 * invdxdy;
-            xy2[4] = a2 * invdxdy;
-
-            if (emit) {
-                const float(*X1)[W] = x1[b];
-                const float(*X2)[W] = x2[b];
-                const float(*Y1)[BX] = y1[b];
-                const float(*Y2)[BX] = y2[b];
-                float fxx1 = 0, fxx2 = 0, fyy1 = 0, fyy2 = 0, fzz1 = 0, fzz2 = 0;
-#pragma unroll
-                for (int n = 1; n <= R; ++n) {
-                    const float c = cstg(n);
-                    fxx1 += c * (X1[ty][tx + R + n] - X1[ty][tx + R - n + 1]);
-                    fxx2 += c * (X2[ty][tx + R + n] - X2[ty][tx + R - n + 1]);
-                    fyy1 += c * (Y1[ty + R + n][tx] - Y1[ty + R - n + 1][tx]);
-                    fyy2 += c * (Y2[ty + R + n][tx] - Y2[ty + R - n + 1][tx]);
-                    fzz1 += c * (dz1[3 + n] - dz1[4 - n]);
-                    fzz2 += c * (dz2[3 + n] - dz2[4 - n]);
-                }
-                const float rho = 1.0f / pw[0];
-                fxx1 *= invdx * rho;
-                fxx2 *= invdx * rho;
-                fyy1 *= invdy * rho;
-                fyy2 *= invdy * rho;
-                fzz1 *= invdz * rho;
-                fzz2 *= invdz * rho;
-                const float fzx1 = qzx1[0] * invdzdx, fzx2 = qzx2[0] * invdzdx;
-                const float fyz1 = qyz1[0] * invdydz, fyz2 = qyz2[0] * invdydz;
-                const float fxy1 = xy1[0], fxy2 = xy2[0];
-                const float vx = pw[5], vy = pw[6], vz = pw[7];
-                const float rx2 = vx * vx, ry2 = vy * vy, rz2 = vz * vz;
-                const float rxy = 2.0f * vx * vy, ryz = 2.0f * vy * vz, rzx = 2.0f * vz * vx;
-                const float V1 = rx2 * fxx1 + ry2 * fyy1 + rz2 * fzz1 + rxy * fxy1 + rzx * fzx1 + ryz * fyz1;
-                const float H1 = fxx1 + fyy1 + fzz1 - V1;
-                const float V2 = rx2 * fxx2 + ry2 * fyy2 + rz2 * fzz2 + rxy * fxy2 + rzx * fzx2 + ryz * fyz2;
-                const float H2 = fxx2 + fyy2 + fzz2 - V2;
-                const float mm1 = pw[1], mm2 = pw[2], mm3 = pw[3], mm4 = pw[4];
-                const float r3 = mm1 * H1 + mm4 * V1 + mm2 * V2;
-                const float r4 = mm2 * H1 + mm3 * V2 + mm4 * H2;
-                un = pw[8] + r3 * dt;
-                wn = pw[9] + r4 * dt;
-            }
+        for (int n = 1; n <= RO; ++n) {
+            a += FD<RO>::e[n] * ((S[ty + RO + n][tx + HX + n] - S[ty + RO - n][tx + HX + n]) +
+                                 (S[ty + RO - n][tx + HX - n] - S[ty + RO + n][tx + HX - n]));
+            ddx[n] = S[ty + RO][tx + HX + n] - S[ty + RO][tx + HX - n];
+            ddy[n] = S[ty + RO + n][tx + HX] - S[ty + RO - n][tx + HX];
+            pin(a), pin(ddx[n]), pin(ddy[n]);
         }
-        // the pointwise words of the next output plane (their registers are free now), then this plane's stores
+        absorb<RO>(qzx, ddx);
+        absorb<RO>(qyz, ddy);
+        xy[RO] = a * invdxdy;
+        if (o > z0)
+            finish(o - 1, b ^ 1);
+        if (o >= z0) {
+            const float(*X)[W] = lx[b][F];
+            const float(*Y)[BX] = ly[b][F];
+            float fxx = 0, fyy = 0, fzz = 0;
+#pragma unroll
+            for (int n = 1; n <= RO; ++n) {
+                const float c = FD<RO>::c[n];
+                fxx += c * (X[ty][tx + HX + n] - X[ty][tx + HX - n + 1]);
+                fyy += c * (Y[ty + RO + n][tx] - Y[ty + RO - n + 1][tx]);
+                fzz += c * (dz[RO - 1 + n] - dz[RO - n]);
+            }
+            const float rho = 1.0f / pw[0];
+            fxx *= invdx * rho;
+            fyy *= invdy * rho;
+            fzz *= invdz * rho;
+            const float vx = pw[1], vy = pw[2], vz = pw[3];
+            const float V = vx * vx * fxx + vy * vy * fyy + vz * vz * fzz + 2.0f * vx * vy * xy[0] +
+                            2.0f * vz * vx * (qzx[0] * invdzdx) + 2.0f * vy * vz * (qyz[0] * invdydz);
+            const float Hf = fxx + fyy + fzz - V;
+            ex[b][F][ty][tx] = F ? V : Hf;
+            part = pw[4] * Hf + pw[5] * V;
+            mc = pw[6];
+            old = pw[7];
+        }
         load_pw(o + 1);
-        if (active && emit) {
-            const long i = (long)o * sz + col;
-            u[i] = un;
-            w[i] = wn;
-        }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            qzx1[j] = qzx1[j + 1];
-            qyz1[j] = qyz1[j + 1];
-            qzx2[j] = qzx2[j + 1];
-            qyz2[j] = qyz2[j + 1];
-        }
-        qzx1[8] = qyz1[8] = qzx2[8] = qyz2[8] = 0.0f;
+        for (int j = 0; j < RO; ++j)
+            xy[j] = xy[j + 1];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            xy1[j] = xy1[j + 1];
-            xy2[j] = xy2[j + 1];
-        }
-#pragma unroll
-        for (int j = 0; j < 7; ++j) {
-            dz1[j] = dz1[j + 1];
-            dz2[j] = dz2[j + 1];
-        }
+        for (int j = 0; j < 2 * RO - 1; ++j)
+            dz[j] = dz[j + 1];
         __syncthreads();
     }
+    finish(z1 - 1, (pend - 1 - p0) & 1);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -763,8 +734,11 @@ __global__ __launch_bounds__(BX* BY) void k_adj_drv(
 // The same operator with the plane pipeline: the 10 input fields of the (H x W) tile of plane p + 2 are loaded as
 // float4 quads (one quad per thread) during plane p; during plane p + 1 the quads become the temporaries S_x, S_y,
 // M_xy, M_zx, M_yz (and, on the centre, S_z and b of every column) in the other LDS buffer; one barrier per plane.
-// Needs quads_fit (launcher falls back).
-template <int BY>
+// d_x and d_y of plane p are stored with plane p, d_z RO - 1 planes and the right-hand sides RO planes later, so only
+// S_z, b and the partial sums wait in registers (160 VGPRs, 247 with d_x, d_y and X_xy in delay queues). Needs quads_fit
+// (launcher falls back). 512^3 3.11 -> 3.05 ms, 256^3 420 -> 390 us (72 B a point at the copy rate: 1.94 ms, 243 us; the
+// tile loads 3.2 words per output and field are what it waits for); order 16 at 200 x 168 x 144 11.45 -> 0.23 ms.
+template <int BY, int RO>
 __global__ __launch_bounds__(BX* BY) void k_adj_drv_q(
     float* __restrict__ d1x, float* __restrict__ d2x, float* __restrict__ d1y, float* __restrict__ d2y,
     float* __restrict__ d1z, float* __restrict__ d2z, float* __restrict__ rhs3, float* __restrict__ rhs4,
@@ -774,15 +748,15 @@ __global__ __launch_bounds__(BX* BY) void k_adj_drv_q(
     const float* __restrict__ m7, int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, long ldx,
     long ldy, float invdx, float invdy, float invdz, float invdxy, float invdyz, float invdzx, int bz)
 {
-    constexpr int W = BX + 2 * R, H = BY + 2 * R, QPR = W / 4, NQ = QPR * H;
+    constexpr int HX = halo_x(RO), W = BX + 2 * HX, H = BY + 2 * RO, QPR = W / 4, NQ = QPR * H;
     static_assert(NQ <= BX * BY, "one tile quad per thread");
-    __shared__ __align__(16) float sx1[2][BY][W], sx2[2][BY][W];   // S_x (x halo)
-    __shared__ __align__(16) float sy1[2][H][BX], sy2[2][H][BX];   // S_y (y halo)
-    __shared__ __align__(16) float mxy1[2][H][W], mxy2[2][H][W];   // M_xy (both halos)
-    __shared__ __align__(16) float mzx1[2][BY][W], mzx2[2][BY][W]; // M_zx (x halo)
-    __shared__ __align__(16) float myz1[2][H][BX], myz2[2][H][BX]; // M_yz (y halo)
-    __shared__ __align__(16) float bt[2][BY][BX];                  // b (centre)
-    __shared__ __align__(16) float szt1[2][BY][BX], szt2[2][BY][BX]; // S_z (centre)
+    __shared__ __align__(16) float2 lsx[2][BY][W];  // S_x (x halo)
+    __shared__ __align__(16) float2 lsy[2][H][BX];  // S_y (y halo)
+    __shared__ __align__(16) float2 lmxy[2][H][W];  // M_xy (both halos)
+    __shared__ __align__(16) float2 lmzx[2][BY][W]; // M_zx (x halo)
+    __shared__ __align__(16) float2 lmyz[2][H][BX]; // M_yz (y halo)
+    __shared__ __align__(16) float2 lsz[2][BY][BX]; // S_z (centre)
+    __shared__ __align__(16) float lb[2][BY][BX];   // b (centre)
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
     int bxi, byi, bzi;
     stencil_tile(bxi, byi, bzi);
@@ -791,35 +765,40 @@ __global__ __launch_bounds__(BX* BY) void k_adj_drv_q(
     const int ix = x0 + tx, iy = y0 + ty;
     const bool active = ix <= ixend && iy <= iyend;
     const long sz = ldx * ldy;
-    const int xlim = min(W, ixend + R + 1 - (x0 - R));
-    const int ylim = min(H, iyend + R + 1 - (y0 - R));
-    const long col = (long)iy * ldx + ix;
-    const int p0 = z0 - R, pend = z1 + R; // tile planes p in [p0, pend), output o = p - R
+    const int xlim = min(W, ixend + RO + 1 - (x0 - HX));
+    const int ylim = min(H, iyend + RO + 1 - (y0 - RO));
+    // byte offset within a plane (inactive lanes: the plane's first word)
+    const unsigned colb = active ? ((unsigned)iy * (unsigned)ldx + (unsigned)ix) * 4u : 0u;
+    const int p0 = z0 - RO, pend = z1 + RO; // tile planes
 
-    // this thread's tile quad: row qr, columns ql .. ql + 3 (elements at or beyond xlim / ylim are zero)
+    // this thread's tile quad: row qr, columns ql .. ql + 3 (elements at or beyond xlim / ylim are zero). The planes
+    // outside [z0, z1) feed the z stencils only, which need no corner of the footprint
     const bool qhas = tid < NQ;
     const int qr = tid / QPR, ql = 4 * (tid - qr * QPR);
+    const bool qrow = qr >= RO && qr < RO + BY, qcol = ql >= HX && ql < HX + BX;
     const int qkeep = qhas && qr < ylim ? min(max(xlim - ql, 0), 4) : 0;
-    const long qoff = (long)(y0 - R + qr) * ldx + (x0 - R + ql);
-    const bool qrow = qr >= R && qr < R + BY, qcol = ql >= R && ql < R + BX;
+    const unsigned qoff = ((unsigned)qr * (unsigned)ldx + (unsigned)ql) * 4u; // bytes from the tile origin
+    const long org = (long)(y0 - RO) * ldx + (x0 - HX);
+    auto inside = [&](int p) { return p >= z0 && p < z1; };
     float4 v1, v2, vb, vm1, vm2, vm3, vm4, vm5, vm6, vm7;
     auto fetch = [&](int p) {
-        if (qkeep > 0) {
-            const long g = (long)p * sz + qoff;
-            v1 = *reinterpret_cast<const float4*>(f1 + g);
-            v2 = *reinterpret_cast<const float4*>(f2 + g);
-            vb = *reinterpret_cast<const float4*>(b + g);
-            vm1 = *reinterpret_cast<const float4*>(m1 + g);
-            vm2 = *reinterpret_cast<const float4*>(m2 + g);
-            vm3 = *reinterpret_cast<const float4*>(m3 + g);
-            vm4 = *reinterpret_cast<const float4*>(m4 + g);
-            vm5 = *reinterpret_cast<const float4*>(m5 + g);
-            vm6 = *reinterpret_cast<const float4*>(m6 + g);
-            vm7 = *reinterpret_cast<const float4*>(m7 + g);
+        if (qkeep > 0 && (qrow || qcol || inside(p))) {
+            const long g = (long)p * sz + org;
+            v1 = ldp4(f1 + g, qoff);
+            v2 = ldp4(f2 + g, qoff);
+            vb = ldp4(b + g, qoff);
+            vm1 = ldp4(m1 + g, qoff);
+            vm2 = ldp4(m2 + g, qoff);
+            vm3 = ldp4(m3 + g, qoff);
+            vm4 = ldp4(m4 + g, qoff);
+            vm5 = ldp4(m5 + g, qoff);
+            vm6 = ldp4(m6 + g, qoff);
+            vm7 = ldp4(m7 + g, qoff);
         }
     };
-    auto commit = [&](int bf) {
-        if (!qhas)
+    auto commit = [&](int p, int bf) {
+        const bool in = inside(p);
+        if (!qhas || !(qrow || qcol || in))
             return;
         const float* A1 = &v1.x;
         const float* A2 = &v2.x;
@@ -831,163 +810,152 @@ __global__ __launch_bounds__(BX* BY) void k_adj_drv_q(
         const float* M5 = &vm5.x;
         const float* M6 = &vm6.x;
         const float* M7 = &vm7.x;
-        float s1x[4], s2x[4], s1y[4], s2y[4], a1xy[4], a2xy[4], a1zx[4], a2zx[4], a1yz[4], a2yz[4], s1z[4], s2z[4],
-            bv[4];
+        float l1[4], h1[4], l2[4], h2[4], rho[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            s1x[e] = s2x[e] = s1y[e] = s2y[e] = a1xy[e] = a2xy[e] = 0.0f;
-            a1zx[e] = a2zx[e] = a1yz[e] = a2yz[e] = s1z[e] = s2z[e] = bv[e] = 0.0f;
-            if (e < qkeep) {
-                const AdjTemps t = adj_temps(A1[e], A2[e], M1[e], M2[e], M3[e], M4[e]);
-                const float rho = 1.0f / BB[e];
-                const float vx = M5[e], vy = M6[e], vz = M7[e];
-                s1x[e] = rho * (t.lap1 + vx * vx * t.hz1);
-                s2x[e] = rho * (t.lap2 + vx * vx * t.hz2);
-                s1y[e] = rho * (t.lap1 + vy * vy * t.hz1);
-                s2y[e] = rho * (t.lap2 + vy * vy * t.hz2);
-                a1xy[e] = 2.0f * vx * vy * t.hz1;
-                a2xy[e] = 2.0f * vx * vy * t.hz2;
-                a1zx[e] = 2.0f * vz * vx * t.hz1;
-                a2zx[e] = 2.0f * vz * vx * t.hz2;
-                a1yz[e] = 2.0f * vy * vz * t.hz1;
-                a2yz[e] = 2.0f * vy * vz * t.hz2;
-                s1z[e] = rho * (t.lap1 + vz * vz * t.hz1);
-                s2z[e] = rho * (t.lap2 + vz * vz * t.hz2);
-                bv[e] = BB[e];
-            }
+            const AdjTemps t = adj_temps(A1[e], A2[e], M1[e], M2[e], M3[e], M4[e]);
+            l1[e] = t.lap1;
+            h1[e] = t.hz1;
+            l2[e] = t.lap2;
+            h2[e] = t.hz2;
+            rho[e] = 1.0f / BB[e];
         }
-        auto st = [](float* dst, const float* v) {
-            *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+        // four points of two fields, interleaved: one 8-byte LDS read per stencil tap gives both
+        auto st2 = [&](float2* dst, auto&& f) {
+            float2 v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = e < qkeep ? f(e) : make_float2(0.0f, 0.0f);
+            *reinterpret_cast<float4*>(dst) = make_float4(v[0].x, v[0].y, v[1].x, v[1].y);
+            *reinterpret_cast<float4*>(dst + 2) = make_float4(v[2].x, v[2].y, v[3].x, v[3].y);
         };
-        st(&mxy1[bf][qr][ql], a1xy);
-        st(&mxy2[bf][qr][ql], a2xy);
-        if (qrow) {
-            st(&sx1[bf][qr - R][ql], s1x);
-            st(&sx2[bf][qr - R][ql], s2x);
-            st(&mzx1[bf][qr - R][ql], a1zx);
-            st(&mzx2[bf][qr - R][ql], a2zx);
+        auto S = [&](const float* r) {
+            return [&, r](int e) {
+                const float s = r[e] * r[e];
+                return make_float2(rho[e] * (l1[e] + s * h1[e]), rho[e] * (l2[e] + s * h2[e]));
+            };
+        };
+        auto M = [&](const float* ra, const float* rb) {
+            return [&, ra, rb](int e) {
+                const float s = 2.0f * ra[e] * rb[e];
+                return make_float2(s * h1[e], s * h2[e]);
+            };
+        };
+        if (in) {
+            st2(&lmxy[bf][qr][ql], M(M5, M6));
+            if (qrow)
+                st2(&lsx[bf][qr - RO][ql], S(M5));
+            if (qcol)
+                st2(&lsy[bf][qr][ql - HX], S(M6));
         }
-        if (qcol) {
-            st(&sy1[bf][qr][ql - R], s1y);
-            st(&sy2[bf][qr][ql - R], s2y);
-            st(&myz1[bf][qr][ql - R], a1yz);
-            st(&myz2[bf][qr][ql - R], a2yz);
-        }
+        if (qrow)
+            st2(&lmzx[bf][qr - RO][ql], M(M7, M5));
+        if (qcol)
+            st2(&lmyz[bf][qr][ql - HX], M(M6, M7));
         if (qrow && qcol) {
-            st(&bt[bf][qr - R][ql - R], bv);
-            st(&szt1[bf][qr - R][ql - R], s1z);
-            st(&szt2[bf][qr - R][ql - R], s2z);
+            st2(&lsz[bf][qr - RO][ql - HX], S(M7));
+            *reinterpret_cast<float4*>(&lb[bf][qr - RO][ql - HX]) = vb;
         }
     };
 
-    float qr1[9], qr2[9];                 // partial X_yz + X_zx sums, q[j] <-> output p - 4 + j
-    float dx1[5], dx2[5], dy1[5], dy2[5]; // delayed d_x, d_y (unscaled by b) at planes p-4..p
-    float rxy1[5], rxy2[5];               // delayed X_xy
-    float szq1[9], szq2[9];               // S_z(p - 8 + k)
-    float bq[5];                          // b(p - 4 + k)
+    // right-hand side sums, q[j] <-> plane p - RO + j: X_yz + X_zx of the planes around it, X_xy of the plane itself
+    float q1[2 * RO + 1], q2[2 * RO + 1];
+    float sz1[2 * RO], sz2[2 * RO]; // S_z(p - 2 RO + 1 + k)
+    float bq[RO];                   // b(p - RO + 1 + k)
 #pragma unroll
-    for (int j = 0; j < 9; ++j)
-        qr1[j] = qr2[j] = szq1[j] = szq2[j] = 0.0f;
+    for (int j = 0; j <= 2 * RO; ++j)
+        q1[j] = q2[j] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 5; ++j)
-        dx1[j] = dx2[j] = dy1[j] = dy2[j] = rxy1[j] = rxy2[j] = bq[j] = 0.0f;
+    for (int j = 0; j < 2 * RO; ++j)
+        sz1[j] = sz2[j] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < RO; ++j)
+        bq[j] = 0.0f;
 
     fetch(p0);
-    commit(0);
-    if (p0 + 1 < pend)
-        fetch(p0 + 1);
+    commit(p0, 0);
+    fetch(p0 + 1); // 2 RO + 1 planes at least
     __syncthreads();
-    // The output o = p - 4 needs S_z(o - 4 .. o + 3), absorbed at planes z0 - 4 onwards.
     for (int p = p0; p < pend; ++p) {
-        const int o = p - R, bf = (p - p0) & 1;
+        const int bf = (p - p0) & 1;
         if (p + 1 < pend)
-            commit(bf ^ 1);
+            commit(p + 1, bf ^ 1);
         if (p + 2 < pend)
             fetch(p + 2);
         if (active) {
-            szq1[8] = szt1[bf][ty][tx];
-            szq2[8] = szt2[bf][ty][tx];
-            bq[4] = bt[bf][ty][tx];
-            const float(*SX1)[W] = sx1[bf];
-            const float(*SX2)[W] = sx2[bf];
-            const float(*SY1)[BX] = sy1[bf];
-            const float(*SY2)[BX] = sy2[bf];
-            const float(*MXY1)[W] = mxy1[bf];
-            const float(*MXY2)[W] = mxy2[bf];
-            const float(*MZX1)[W] = mzx1[bf];
-            const float(*MZX2)[W] = mzx2[bf];
-            const float(*MYZ1)[BX] = myz1[bf];
-            const float(*MYZ2)[BX] = myz2[bf];
+            const long ip = (long)p * sz;
+            const float bc = lb[bf][ty][tx];
+            const float2 sc = lsz[bf][ty][tx];
+            sz1[2 * RO - 1] = sc.x;
+            sz2[2 * RO - 1] = sc.y;
+            bq[RO - 1] = bc;
 #pragma unroll
-            for (int j = 0; j < 9; ++j) {
-                const int k = R - j;
-                if (k != 0) {
-                    const int ak = k < 0 ? -k : k;
-                    const float e = ecen(ak);
-                    qr1[j] += invdyz * e * (MYZ1[ty + R + k][tx] - MYZ1[ty + R - k][tx]) +
-                              invdzx * e * (MZX1[ty][tx + R + k] - MZX1[ty][tx + R - k]);
-                    qr2[j] += invdyz * e * (MYZ2[ty + R + k][tx] - MYZ2[ty + R - k][tx]) +
-                              invdzx * e * (MZX2[ty][tx + R + k] - MZX2[ty][tx + R - k]);
+            for (int n = 1; n <= RO; ++n) {
+                const float e = FD<RO>::e[n];
+                const float2 yp = lmyz[bf][ty + RO + n][tx], ym = lmyz[bf][ty + RO - n][tx];
+                const float2 xp = lmzx[bf][ty][tx + HX + n], xm = lmzx[bf][ty][tx + HX - n];
+                const float d1 = invdyz * (yp.x - ym.x) + invdzx * (xp.x - xm.x);
+                const float d2 = invdyz * (yp.y - ym.y) + invdzx * (xp.y - xm.y);
+                q1[RO - n] += e * d1;
+                q1[RO + n] -= e * d1;
+                q2[RO - n] += e * d2;
+                q2[RO + n] -= e * d2;
+            }
+            if (inside(p)) {
+                float ax1 = 0, ax2 = 0, ay1 = 0, ay2 = 0, axy1 = 0, axy2 = 0;
+#pragma unroll
+                for (int n = 1; n <= RO; ++n) {
+                    const float c = FD<RO>::c[n], e = FD<RO>::e[n];
+                    const float2 xp = lsx[bf][ty][tx + HX + n - 1], xm = lsx[bf][ty][tx + HX - n];
+                    const float2 yp = lsy[bf][ty + RO + n - 1][tx], ym = lsy[bf][ty + RO - n][tx];
+                    ax1 += c * (xp.x - xm.x);
+                    ax2 += c * (xp.y - xm.y);
+                    ay1 += c * (yp.x - ym.x);
+                    ay2 += c * (yp.y - ym.y);
+                    const float2 pp = lmxy[bf][ty + RO + n][tx + HX + n], pm = lmxy[bf][ty + RO + n][tx + HX - n];
+                    const float2 mm = lmxy[bf][ty + RO - n][tx + HX - n], mp = lmxy[bf][ty + RO - n][tx + HX + n];
+                    axy1 += e * (pp.x - pm.x + mm.x - mp.x);
+                    axy2 += e * (pp.y - pm.y + mm.y - mp.y);
                 }
+                stp(d1x + ip, colb, ax1 * invdx * bc);
+                stp(d2x + ip, colb, ax2 * invdx * bc);
+                stp(d1y + ip, colb, ay1 * invdy * bc);
+                stp(d2y + ip, colb, ay2 * invdy * bc);
+                q1[RO] += axy1 * invdxy;
+                q2[RO] += axy2 * invdxy;
             }
-            float ax1 = 0, ax2 = 0, ay1 = 0, ay2 = 0, axy1 = 0, axy2 = 0;
-#pragma unroll
-            for (int n = 1; n <= R; ++n) {
-                const float c = cstg(n);
-                ax1 += c * (SX1[ty][tx + R + n - 1] - SX1[ty][tx + R - n]);
-                ax2 += c * (SX2[ty][tx + R + n - 1] - SX2[ty][tx + R - n]);
-                ay1 += c * (SY1[ty + R + n - 1][tx] - SY1[ty + R - n][tx]);
-                ay2 += c * (SY2[ty + R + n - 1][tx] - SY2[ty + R - n][tx]);
-                const float e = ecen(n);
-                axy1 += e * (MXY1[ty + R + n][tx + R + n] - MXY1[ty + R + n][tx + R - n] +
-                             MXY1[ty + R - n][tx + R - n] - MXY1[ty + R - n][tx + R + n]);
-                axy2 += e * (MXY2[ty + R + n][tx + R + n] - MXY2[ty + R + n][tx + R - n] +
-                             MXY2[ty + R - n][tx + R - n] - MXY2[ty + R - n][tx + R + n]);
-            }
-            dx1[4] = ax1 * invdx;
-            dx2[4] = ax2 * invdx;
-            dy1[4] = ay1 * invdy;
-            dy2[4] = ay2 * invdy;
-            rxy1[4] = axy1 * invdxy;
-            rxy2[4] = axy2 * invdxy;
-            if (o >= z0) {
+            if (inside(p - RO + 1)) {
                 float az1 = 0, az2 = 0;
 #pragma unroll
-                for (int n = 1; n <= R; ++n) {
-                    const float c = cstg(n);
-                    az1 += c * (szq1[3 + n] - szq1[4 - n]);
-                    az2 += c * (szq2[3 + n] - szq2[4 - n]);
+                for (int n = 1; n <= RO; ++n) {
+                    const float c = FD<RO>::c[n];
+                    az1 += c * (sz1[RO + n - 1] - sz1[RO - n]);
+                    az2 += c * (sz2[RO + n - 1] - sz2[RO - n]);
                 }
-                const float bo = bq[0];
-                const long i = (long)o * sz + col;
-                d1x[i] = dx1[0] * bo;
-                d2x[i] = dx2[0] * bo;
-                d1y[i] = dy1[0] * bo;
-                d2y[i] = dy2[0] * bo;
-                d1z[i] = az1 * invdz * bo;
-                d2z[i] = az2 * invdz * bo;
-                rhs3[i] = rxy1[0] + qr1[0];
-                rhs4[i] = rxy2[0] + qr2[0];
+                const long i = ip - (RO - 1) * sz;
+                stp(d1z + i, colb, az1 * invdz * bq[0]);
+                stp(d2z + i, colb, az2 * invdz * bq[0]);
+            }
+            if (p - RO >= z0) {
+                const long i = ip - RO * sz;
+                stp(rhs3 + i, colb, q1[0]);
+                stp(rhs4 + i, colb, q2[0]);
             }
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            qr1[j] = qr1[j + 1];
-            qr2[j] = qr2[j + 1];
-            szq1[j] = szq1[j + 1];
-            szq2[j] = szq2[j + 1];
+        for (int j = 0; j < 2 * RO; ++j) {
+            q1[j] = q1[j + 1];
+            q2[j] = q2[j + 1];
         }
-        qr1[8] = qr2[8] = 0.0f;
+        q1[2 * RO] = q2[2 * RO] = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            dx1[j] = dx1[j + 1];
-            dx2[j] = dx2[j + 1];
-            dy1[j] = dy1[j + 1];
-            dy2[j] = dy2[j + 1];
-            rxy1[j] = rxy1[j + 1];
-            rxy2[j] = rxy2[j + 1];
-            bq[j] = bq[j + 1];
+        for (int j = 0; j < 2 * RO - 1; ++j) {
+            sz1[j] = sz1[j + 1];
+            sz2[j] = sz2[j + 1];
         }
+#pragma unroll
+        for (int j = 0; j < RO - 1; ++j)
+            bq[j] = bq[j + 1];
         __syncthreads();
     }
 }
@@ -1084,7 +1052,7 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update(
 // The same operator with the plane pipeline: the d_x / d_y tiles of plane o + 1 are loaded as float4 quads during
 // plane o - 1 and stored into the other LDS buffer during plane o; the d_z column word and the pointwise words
 // (rhs3, rhs4, u, w) of plane o + 1 are loaded during plane o; one barrier per plane. Needs quads_fit.
-template <int BY, bool SPONGE>
+template <int BY, bool SPONGE, int RO>
 __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
     float* __restrict__ u, float* __restrict__ w, const float* __restrict__ d1x, const float* __restrict__ d2x,
     const float* __restrict__ d1y, const float* __restrict__ d2y, const float* __restrict__ d1z,
@@ -1093,7 +1061,7 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
     int iybeg, int iyend, int izbeg, int izend, long ldx, long ldy, float dt, float invdx, float invdy, float invdz,
     int bz)
 {
-    constexpr int W = BX + 2 * R, H = BY + 2 * R, NT = BX * BY;
+    constexpr int HX = halo_x(RO), W = BX + 2 * HX, H = BY + 2 * RO, NT = BX * BY;
     __shared__ __align__(16) float x1[2][BY][W], x2[2][BY][W];
     __shared__ __align__(16) float y1[2][H][BX], y2[2][H][BX];
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
@@ -1106,11 +1074,12 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
     const int ix = x0 + tx, iy = y0 + ty;
     const bool active = ix <= ixend && iy <= iyend;
     const long sz = ldx * ldy;
-    const int xlim = min(W, ixend + R + 1 - (x0 - R));
-    const int ylim = min(H, iyend + R + 1 - (y0 - R));
+    const int xlim = min(W, ixend + RO + 1 - (x0 - HX));
+    const int ylim = min(H, iyend + RO + 1 - (y0 - RO));
     const int xlim_c = min(BX, ixend + 1 - x0);
     const int ylim_c = min(BY, iyend + 1 - y0);
-    const long col = (long)iy * ldx + ix;
+    // byte offset within a plane (inactive lanes: the plane's first word)
+    const unsigned colb = active ? ((unsigned)iy * (unsigned)ldx + (unsigned)ix) * 4u : 0u;
     float axy = 1.0f, bxy = 1.0f;
     if (SPONGE && active) {
         axy = fminf(abx[ix].a, aby[iy].a);
@@ -1118,7 +1087,7 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
     }
     const TileQuads<W, BY, NT> qx(tid, ldx, xlim, ylim_c);
     const TileQuads<BX, H, NT> qy(tid, ldx, xlim_c, ylim);
-    const long ox = (long)y0 * ldx + (x0 - R), oy = (long)(y0 - R) * ldx + x0;
+    const long ox = (long)y0 * ldx + (x0 - HX), oy = (long)(y0 - RO) * ldx + x0;
     float4 rx1[qx.QT], rx2[qx.QT], ry1[qy.QT], ry2[qy.QT];
     auto fetch = [&](int o) {
         const long oz = (long)o * sz;
@@ -1136,24 +1105,24 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
     float pw[4]; // rhs3, rhs4, u, w of the plane being finalised
     auto load_pw = [&](int o) {
         if (active && o < z1) {
-            const long i = (long)o * sz + col;
-            pw[0] = rhs3[i];
-            pw[1] = rhs4[i];
-            pw[2] = u[i];
-            pw[3] = w[i];
+            const long i = (long)o * sz;
+            pw[0] = ldp(rhs3 + i, colb);
+            pw[1] = ldp(rhs4 + i, colb);
+            pw[2] = ldp(u + i, colb);
+            pw[3] = ldp(w + i, colb);
         }
     };
 
-    float dz1[8], dz2[8]; // d_z(o - 3 + k)
+    float dz1[2 * RO], dz2[2 * RO]; // d_z(o - RO + 1 + k)
 #pragma unroll
-    for (int k = 0; k < 7; ++k) {
-        dz1[k] = active ? d1z[(long)(z0 - 3 + k) * sz + col] : 0.0f;
-        dz2[k] = active ? d2z[(long)(z0 - 3 + k) * sz + col] : 0.0f;
+    for (int k = 0; k < 2 * RO - 1; ++k) {
+        dz1[k] = ldp(d1z + (long)(z0 - RO + 1 + k) * sz, colb);
+        dz2[k] = ldp(d2z + (long)(z0 - RO + 1 + k) * sz, colb);
     }
-    float n1 = 0.0f, n2 = 0.0f; // d_z(o + 4) of the next plane
+    float n1 = 0.0f, n2 = 0.0f; // d_z(o + RO) of the next plane
     if (active) {
-        n1 = d1z[(long)(z0 + 4) * sz + col];
-        n2 = d2z[(long)(z0 + 4) * sz + col];
+        n1 = ldp(d1z + (long)(z0 + RO) * sz, colb);
+        n2 = ldp(d2z + (long)(z0 + RO) * sz, colb);
     }
     load_pw(z0);
     fetch(z0);
@@ -1163,11 +1132,11 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
     __syncthreads();
     for (int o = z0; o < z1; ++o) {
         const int bf = (o - z0) & 1;
-        dz1[7] = n1;
-        dz2[7] = n2;
+        dz1[2 * RO - 1] = n1;
+        dz2[2 * RO - 1] = n2;
         if (active && o + 1 < z1) {
-            n1 = d1z[(long)(o + 5) * sz + col];
-            n2 = d2z[(long)(o + 5) * sz + col];
+            n1 = ldp(d1z + (long)(o + RO + 1) * sz, colb);
+            n2 = ldp(d2z + (long)(o + RO + 1) * sz, colb);
         }
         if (o + 1 < z1)
             commit(bf ^ 1);
@@ -1181,14 +1150,14 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
             const float(*Y2)[BX] = y2[bf];
             float fx1 = 0, fx2 = 0, fy1 = 0, fy2 = 0, fz1 = 0, fz2 = 0;
 #pragma unroll
-            for (int n = 1; n <= R; ++n) {
-                const float c = cstg(n);
-                fx1 += c * (X1[ty][tx + R + n] - X1[ty][tx + R - n + 1]);
-                fx2 += c * (X2[ty][tx + R + n] - X2[ty][tx + R - n + 1]);
-                fy1 += c * (Y1[ty + R + n][tx] - Y1[ty + R - n + 1][tx]);
-                fy2 += c * (Y2[ty + R + n][tx] - Y2[ty + R - n + 1][tx]);
-                fz1 += c * (dz1[3 + n] - dz1[4 - n]);
-                fz2 += c * (dz2[3 + n] - dz2[4 - n]);
+            for (int n = 1; n <= RO; ++n) {
+                const float c = FD<RO>::c[n];
+                fx1 += c * (X1[ty][tx + HX + n] - X1[ty][tx + HX - n + 1]);
+                fx2 += c * (X2[ty][tx + HX + n] - X2[ty][tx + HX - n + 1]);
+                fy1 += c * (Y1[ty + RO + n][tx] - Y1[ty + RO - n + 1][tx]);
+                fy2 += c * (Y2[ty + RO + n][tx] - Y2[ty + RO - n + 1][tx]);
+                fz1 += c * (dz1[RO - 1 + n] - dz1[RO - n]);
+                fz2 += c * (dz2[RO - 1 + n] - dz2[RO - n]);
             }
             const float r3 = fx1 * invdx + fy1 * invdy + fz1 * invdz + pw[0];
             const float r4 = fx2 * invdx + fy2 * invdy + fz2 * invdz + pw[1];
@@ -1204,12 +1173,12 @@ __global__ __launch_bounds__(BX* BY) void k_adj_update_q(
         }
         load_pw(o + 1);
         if (active) {
-            const long i = (long)o * sz + col;
-            u[i] = un;
-            w[i] = wn;
+            const long i = (long)o * sz;
+            stp(u + i, colb, un);
+            stp(w + i, colb, wn);
         }
 #pragma unroll
-        for (int k = 0; k < 7; ++k) {
+        for (int k = 0; k < 2 * RO - 1; ++k) {
             dz1[k] = dz1[k + 1];
             dz2[k] = dz2[k + 1];
         }
@@ -1398,14 +1367,16 @@ __global__ __launch_bounds__(BX* BY) void k_rho_grad_q(
     const int ylim = min(H, iyend + R + 1 - (y0 - R));
     const int xlim_c = min(BX, ixend + 1 - x0);
     const int ylim_c = min(BY, iyend + 1 - y0);
-    const long col = (long)iy * ldx + ix;
+    // byte offset within a plane (inactive lanes: the plane's first word)
+    const unsigned colb = active ? ((unsigned)iy * (unsigned)ldx + (unsigned)ix) * 4u : 0u;
 
     // this thread's quad of the S footprint (rows of the tile or columns of the tile; corners are not needed)
     const int qr = tid / QPR, ql = 4 * (tid - qr * QPR);
     const bool qrow = qr >= R && qr < R + BY, qcol = ql >= R && ql < R + BX;
     const bool qhas = tid < NQ && (qrow || qcol);
     const int qkeep = qhas && qr < ylim ? min(max(xlim - ql, 0), 4) : 0;
-    const long qoff = (long)(y0 - R + qr) * ldx + (x0 - R + ql);
+    const unsigned qoff = ((unsigned)qr * (unsigned)ldx + (unsigned)ql) * 4u; // bytes from the tile origin
+    const long org = (long)(y0 - R) * ldx + (x0 - R);
     float4 v1, v2, vb, vm1, vm2, vm3, vm4, vx4, vy4;
     const TileQuads<W, BY, NT> qx(tid, ldx, xlim, ylim_c);
     const TileQuads<BX, H, NT> qy(tid, ldx, xlim_c, ylim);
@@ -1414,16 +1385,16 @@ __global__ __launch_bounds__(BX* BY) void k_rho_grad_q(
     auto fetch = [&](int o) {
         const long oz = (long)o * sz;
         if (qkeep > 0) {
-            const long g = oz + qoff;
-            v1 = *reinterpret_cast<const float4*>(f1 + g);
-            v2 = *reinterpret_cast<const float4*>(f2 + g);
-            vb = *reinterpret_cast<const float4*>(b + g);
-            vm1 = *reinterpret_cast<const float4*>(m1 + g);
-            vm2 = *reinterpret_cast<const float4*>(m2 + g);
-            vm3 = *reinterpret_cast<const float4*>(m3 + g);
-            vm4 = *reinterpret_cast<const float4*>(m4 + g);
-            vx4 = *reinterpret_cast<const float4*>(vrx + g);
-            vy4 = *reinterpret_cast<const float4*>(vry + g);
+            const long g = oz + org;
+            v1 = ldp4(f1 + g, qoff);
+            v2 = ldp4(f2 + g, qoff);
+            vb = ldp4(b + g, qoff);
+            vm1 = ldp4(m1 + g, qoff);
+            vm2 = ldp4(m2 + g, qoff);
+            vm3 = ldp4(m3 + g, qoff);
+            vm4 = ldp4(m4 + g, qoff);
+            vx4 = ldp4(vrx + g, qoff);
+            vy4 = ldp4(vry + g, qoff);
         }
         qx.fetch(rx1, fd1x + oz + ox);
         qx.fetch(rx2, fd2x + oz + ox);
@@ -1481,8 +1452,9 @@ __global__ __launch_bounds__(BX* BY) void k_rho_grad_q(
         float a1, a2, mm1, mm2, mm3, mm4, bb, vz, d1, d2;
     };
     auto col_load = [&](int q) {
-        const long g = (long)q * sz + col;
-        return Col{ f1[g], f2[g], m1[g], m2[g], m3[g], m4[g], b[g], vrz[g], fd1z[g], fd2z[g] };
+        const long g = (long)q * sz;
+        auto w = [&](const float* v) { return ldp(v + g, colb); };
+        return Col{ w(f1), w(f2), w(m1), w(m2), w(m3), w(m4), w(b), w(vrz), w(fd1z), w(fd2z) };
     };
     auto col_sz = [&](const Col& c, float& s1, float& s2) {
         const AdjTemps t = adj_temps(c.a1, c.a2, c.mm1, c.mm2, c.mm3, c.mm4);
@@ -1504,17 +1476,12 @@ __global__ __launch_bounds__(BX* BY) void k_rho_grad_q(
     if (active) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const long g = (long)(z0 - 4 + k) * sz + col;
-            const AdjTemps t = adj_temps(f1[g], f2[g], m1[g], m2[g], m3[g], m4[g]);
-            const float rho = 1.0f / b[g];
-            const float vz = vrz[g];
-            szq1[k] = rho * (t.lap1 + vz * vz * t.hz1);
-            szq2[k] = rho * (t.lap2 + vz * vz * t.hz2);
+            col_sz(col_load(z0 - 4 + k), szq1[k], szq2[k]);
         }
 #pragma unroll
         for (int k = 0; k < 7; ++k) {
-            fzq1[k] = fd1z[(long)(z0 - 3 + k) * sz + col];
-            fzq2[k] = fd2z[(long)(z0 - 3 + k) * sz + col];
+            fzq1[k] = ldp(fd1z + (long)(z0 - 3 + k) * sz, colb);
+            fzq2[k] = ldp(fd2z + (long)(z0 - 3 + k) * sz, colb);
         }
         nc = col_load(z0 + 4);
         g0 = grad[((long)(z0 - izbeg) * gldy + (iy - iybeg)) * gldx + (ix - ixbeg)];
@@ -1746,6 +1713,17 @@ launch_fwd_kernel2_drv(const float* field1, const float* field2, const float* Mo
                        int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, float invdx, float invdy,
                        float invdz, int ldimx, int ldimy, int order, void* stream)
 {
+    auto tiled = [&](auto kern, Chunk c, int by) {
+        const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, c, by);
+        kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz, by), dim3(BX, by), 0, (hipStream_t)stream>>>(
+            field1, field2, Model11, dfield1dx, dfield1dy, dfield1dz, dfield2dx, dfield2dy, dfield2dz, ixbeg, ixend,
+            iybeg, iyend, izbeg, izend, invdx, invdy, invdz, (long)ldimx, (long)ldimy, bz);
+        return launch_status();
+    };
+    const bool q = quads_fit(ixbeg, ldimx, ldimy, { field1, field2 });
+    if (order == 16 && field1 && field2 && Model11 && dfield1dx && dfield1dy && dfield1dz && dfield2dx && dfield2dy &&
+        dfield2dz && q && ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy, 8))
+        return tiled(k_fwd_drv_q<BYL, 8>, FWD_DRV16_CHUNK, BYL);
     if (order == 16 && field1 && field2 && Model11 && dfield1dx && dfield1dy && dfield1dz && dfield2dx && dfield2dy &&
         dfield2dz)
         return order_fwd_drv(order, field1, field2, Model11, dfield1dx, dfield1dy, dfield1dz, dfield2dx, dfield2dy,
@@ -1756,12 +1734,7 @@ launch_fwd_kernel2_drv(const float* field1, const float* field2, const float* Mo
     if (!field1 || !field2 || !Model11 || !dfield1dx || !dfield1dy || !dfield1dz || !dfield2dx || !dfield2dy ||
         !dfield2dz || !ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, FWD_DRV_CHUNK, BYL);
-    auto kern = quads_fit(ixbeg, ldimx, { field1, field2 }) ? k_fwd_drv_q<BYL> : k_fwd_drv<BYL>;
-    kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz, BYL), dim3(BX, BYL), 0, (hipStream_t)stream>>>(
-        field1, field2, Model11, dfield1dx, dfield1dy, dfield1dz, dfield2dx, dfield2dy, dfield2dz, ixbeg, ixend, iybeg,
-        iyend, izbeg, izend, invdx, invdy, invdz, (long)ldimx, (long)ldimy, bz);
-    return launch_status();
+    return tiled(q ? k_fwd_drv_q<BYL, R> : k_fwd_drv<BYL>, FWD_DRV_CHUNK, BYL);
 }
 
 int
@@ -1790,24 +1763,29 @@ launch_update_rho_fwd_main_loop_2_1(float* field3, float* field4, const float* f
     if (!field3 || !field4 || !field1_dx || !field2_dx || !field1_dy || !field2_dy || !field1_dz || !field2_dz ||
         !field1 || !field2 || !irho || !model1 || !model2 || !model3 || !model4 || !rx || !ry || !rz)
         return TTI_EINVAL;
-    if (order == 16)
-        return order_fwd_update(order, field3, field4, field1_dx, field2_dx, field1_dy, field2_dy, field1_dz,
-                                field2_dz, field1, field2, irho, model1, model2, model3, model4, rx, ry, rz, ixbeg,
-                                ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy, dt, dx, dy, dz, stream);
-    if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
-        return TTI_EINVAL;
     const float invdx = (float)(1.0 / dx), invdy = (float)(1.0 / dy), invdz = (float)(1.0 / dz);
     const float invdxdy = (float)(1.0 / (4 * dx * dy)), invdydz = (float)(1.0 / (4 * dy * dz)),
                 invdzdx = (float)(1.0 / (4 * dx * dz));
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, FWD_UPDATE_CHUNK);
-    auto kern = quads_fit(ixbeg, ldimx, { field1, field2, field1_dx, field2_dx, field1_dy, field2_dy })
-                    ? k_fwd_update_q<BYS>
-                    : k_fwd_update<BYS>;
-    kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz), dim3(BX, BYS), 0, (hipStream_t)stream>>>(
-        field3, field4, field1_dx, field2_dx, field1_dy, field2_dy, field1_dz, field2_dz, field1, field2, irho, model1,
-        model2, model3, model4, rx, ry, rz, ixbeg, ixend, iybeg, iyend, izbeg, izend, (long)ldimx, (long)ldimy, dt,
-        invdx, invdy, invdz, invdxdy, invdydz, invdzdx, bz);
-    return launch_status();
+    auto tiled = [&](auto kern, Chunk c, int fields) {
+        const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, c);
+        kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz), dim3(BX, BYS, fields), 0,
+               (hipStream_t)stream>>>(
+            field3, field4, field1_dx, field2_dx, field1_dy, field2_dy, field1_dz, field2_dz, field1, field2, irho,
+            model1, model2, model3, model4, rx, ry, rz, ixbeg, ixend, iybeg, iyend, izbeg, izend, (long)ldimx,
+            (long)ldimy, dt, invdx, invdy, invdz, invdxdy, invdydz, invdzdx, bz);
+        return launch_status();
+    };
+    const bool q = quads_fit(ixbeg, ldimx, ldimy, { field1, field2, field1_dx, field2_dx, field1_dy, field2_dy });
+    if (order == 16) {
+        if (q && ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy, 8))
+            return tiled(k_fwd_update_q<BYS, 8>, FWD_UPDATE16_CHUNK, 2);
+        return order_fwd_update(order, field3, field4, field1_dx, field2_dx, field1_dy, field2_dy, field1_dz,
+                                field2_dz, field1, field2, irho, model1, model2, model3, model4, rx, ry, rz, ixbeg,
+                                ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy, dt, dx, dy, dz, stream);
+    }
+    if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
+        return TTI_EINVAL;
+    return q ? tiled(k_fwd_update_q<BYS, R>, FWD_UPDATE_CHUNK, 2) : tiled(k_fwd_update<BYS>, FWD_UPDATE_CHUNK, 1);
 }
 
 int
@@ -1826,22 +1804,27 @@ launch_adj_kernel2_drv(float* dfield1dx, float* dfield2dx, float* dfield1dy, flo
         !field4_rhs || !field1 || !field2 || !Model11 || !model1 || !model2 || !model3 || !model4 || !model5 ||
         !model6 || !model7)
         return TTI_EINVAL;
-    if (order == 16)
+    auto tiled = [&](auto kern, Chunk c) {
+        const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, c);
+        kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz), dim3(BX, BYS), 0, (hipStream_t)stream>>>(
+            dfield1dx, dfield2dx, dfield1dy, dfield2dy, dfield1dz, dfield2dz, field3_rhs, field4_rhs, field1, field2,
+            Model11, model1, model2, model3, model4, model5, model6, model7, ixbeg, ixend, iybeg, iyend, izbeg, izend,
+            (long)ldimx, (long)ldimy, invdx, invdy, invdz, invdxy, invdyz, invdzx, bz);
+        return launch_status();
+    };
+    const bool q = quads_fit(ixbeg, ldimx, ldimy,
+                             { field1, field2, Model11, model1, model2, model3, model4, model5, model6, model7 });
+    if (order == 16) {
+        if (q && ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy, 8))
+            return tiled(k_adj_drv_q<BYS, 8>, ADJ_DRV16_CHUNK);
         return order_adj_drv(order, dfield1dx, dfield2dx, dfield1dy, dfield2dy, dfield1dz, dfield2dz, field3_rhs,
                              field4_rhs, field1, field2, Model11, model1, model2, model3, model4, model5, model6,
                              model7, ixbeg, ixend, iybeg, iyend, izbeg, izend, invdxy, invdyz, invdzx, ldimx, ldimy,
                              invdx, invdy, invdz, stream);
+    }
     if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, ADJ_DRV_CHUNK);
-    const bool q = quads_fit(ixbeg, ldimx,
-                             { field1, field2, Model11, model1, model2, model3, model4, model5, model6, model7 });
-    auto kern = q ? k_adj_drv_q<BYS> : k_adj_drv<BYS>;
-    kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz), dim3(BX, BYS), 0, (hipStream_t)stream>>>(dfield1dx, dfield2dx, dfield1dy, dfield2dy, dfield1dz, dfield2dz,
-                       field3_rhs, field4_rhs, field1, field2, Model11, model1, model2, model3, model4, model5,
-                       model6, model7, ixbeg, ixend, iybeg, iyend, izbeg, izend, (long)ldimx, (long)ldimy, invdx,
-                       invdy, invdz, invdxy, invdyz, invdzx, bz);
-    return launch_status();
+    return tiled(q ? k_adj_drv_q<BYS, R> : k_adj_drv<BYS>, ADJ_DRV_CHUNK);
 }
 
 int
@@ -1862,29 +1845,29 @@ launch_update_adj_kernel_main_3(float* field3, float* field4, const float* field
         return TTI_EINVAL;
     if (sponge_active && (!ab_xx || !ab_yy || !ab_zz))
         return TTI_EINVAL;
-    if (order == 16)
+    const float invdx = (float)(1.0 / dx), invdy = (float)(1.0 / dy), invdz = (float)(1.0 / dz);
+    const bool sp = sponge_active != 0;
+    auto tiled = [&](auto kern, Chunk c, int by) { // in dispatch order
+        const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, c, by);
+        kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz, by), dim3(BX, by), 0, (hipStream_t)stream>>>(
+            field3, field4, field1_dx, field2_dx, field1_dy, field2_dy, field1_dz, field2_dz, field3_rhs, field4_rhs,
+            sp ? (const ab2*)ab_xx : nullptr, sp ? (const ab2*)ab_yy : nullptr, sp ? (const ab2*)ab_zz : nullptr,
+            ixbeg, ixend, iybeg, iyend, izbeg, izend, (long)ldimx, (long)ldimy, dt, invdx, invdy, invdz, bz);
+        return launch_status();
+    };
+    const bool q = quads_fit(ixbeg, ldimx, ldimy, { field1_dx, field2_dx, field1_dy, field2_dy });
+    if (order == 16) {
+        if (q && ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy, 8))
+            return tiled(sp ? k_adj_update_q<BYS, true, 8> : k_adj_update_q<BYS, false, 8>, ADJ_UPDATE16_CHUNK, BYS);
         return order_adj_update(order, field3, field4, field1_dx, field2_dx, field1_dy, field2_dy, field1_dz,
                                 field2_dz, field3_rhs, field4_rhs, ab_xx, ab_yy, ab_zz, ixbeg, ixend, iybeg, iyend,
                                 izbeg, izend, ldimx, ldimy, dt, dx, dy, dz, sponge_active, stream);
+    }
     if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
-    const float invdx = (float)(1.0 / dx), invdy = (float)(1.0 / dy), invdz = (float)(1.0 / dz);
-    const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, ADJ_UPDATE_CHUNK, BYL); // plain dispatch order
-    const dim3 grid = stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz, BYL);
-    const bool q = quads_fit(ixbeg, ldimx, { field1_dx, field2_dx, field1_dy, field2_dy });
-    auto kern = sponge_active ? (q ? k_adj_update_q<BYL, true> : k_adj_update<BYL, true>)
-                              : (q ? k_adj_update_q<BYL, false> : k_adj_update<BYL, false>);
-    const ab2* ab[3] = { nullptr, nullptr, nullptr };
-    if (sponge_active) {
-        ab[0] = (const ab2*)ab_xx;
-        ab[1] = (const ab2*)ab_yy;
-        ab[2] = (const ab2*)ab_zz;
-    }
-    kern<<<grid, dim3(BX, BYL), 0, (hipStream_t)stream>>>(field3, field4, field1_dx, field2_dx, field1_dy, field2_dy,
-                                                          field1_dz, field2_dz, field3_rhs, field4_rhs, ab[0], ab[1],
-                                                          ab[2], ixbeg, ixend, iybeg, iyend, izbeg, izend, (long)ldimx,
-                                                          (long)ldimy, dt, invdx, invdy, invdz, bz);
-    return launch_status();
+    if (q)
+        return tiled(sp ? k_adj_update_q<BYL, true, R> : k_adj_update_q<BYL, false, R>, ADJ_UPDATE_CHUNK, BYL);
+    return tiled(sp ? k_adj_update<BYL, true> : k_adj_update<BYL, false>, ADJ_UPDATE_CHUNK, BYL);
 }
 
 int
@@ -1915,7 +1898,7 @@ launch_update_rho_gradient_rho(float* grad, const float* fwd_field1_dx, const fl
         return TTI_EINVAL;
     const float hx = (float)(1.0 / dx), hy = (float)(1.0 / dy), hz = (float)(1.0 / dz);
     const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, RHO_GRAD_CHUNK);
-    const bool q = quads_fit(ixbeg, ldimx, { fwd_field1_dx, fwd_field2_dx, fwd_field1_dy, fwd_field2_dy, field1, field2,
+    const bool q = quads_fit(ixbeg, ldimx, ldimy, { fwd_field1_dx, fwd_field2_dx, fwd_field1_dy, fwd_field2_dy, field1, field2,
                                             irho, model1, model2, model3, model4, rx, ry });
     auto kern = q ? k_rho_grad_q<BYS> : k_rho_grad<BYS>;
     kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz), dim3(BX, BYS), 0, (hipStream_t)stream>>>(
@@ -1944,7 +1927,7 @@ rho_gradient_f64(double* grad, const float* fwd_field1_dx, const float* fwd_fiel
         return TTI_EINVAL;
     const float hx = (float)(1.0 / dx), hy = (float)(1.0 / dy), hz = (float)(1.0 / dz);
     const int bz = stencil_bz(ixbeg, ixend, iybeg, iyend, izbeg, izend, RHO_GRAD_CHUNK);
-    const bool q = quads_fit(ixbeg, ldimx, { fwd_field1_dx, fwd_field2_dx, fwd_field1_dy, fwd_field2_dy, field1, field2,
+    const bool q = quads_fit(ixbeg, ldimx, ldimy, { fwd_field1_dx, fwd_field2_dx, fwd_field1_dy, fwd_field2_dy, field1, field2,
                                             irho, model1, model2, model3, model4, rx, ry });
     auto kern = q ? k_rho_grad_q<BYS, double> : k_rho_grad<BYS, double>;
     kern<<<stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, bz), dim3(BX, BYS), 0, (hipStream_t)stream>>>(
