@@ -80,7 +80,7 @@ slot_snap(const ShotDev& S, int slot)
 }
 
 template <int SNAP, bool SPONGE>
-__global__ __launch_bounds__(BX* FWD_BY, FWD_BY <= 4 ? 2 : 1) void k_fused_fwd_batch(const ShotDev* __restrict__ shots,
+__global__ __launch_bounds__(2 * BX* FWD_BY, 4) void k_fused_fwd_batch(const ShotDev* __restrict__ shots,
                                                                     const int* __restrict__ tile_shot, int ntiles,
                                                                     int par, int it, int slot, float dt, float invdx,
                                                                     float invdy, float invdz, float i4xy, float i4yz,
@@ -183,7 +183,7 @@ fwd_step(tti_batch* b, int par, int it, int slot, hipStream_t st)
     if (par < 0 || par > 1 || it < 0 || it >= b->nt_max || slot >= b->slots ||
         (slot >= 0 && b->mode == TTI_SNAP_NONE))
         return TTI_EINVAL;
-    const dim3 grid(((b->ntiles[0] + 7) / 8) * 8), block(BX, FWD_BY);
+    const dim3 grid(((b->ntiles[0] + 7) / 8) * 8), block(BX, FWD_BY, 2);
     auto go = [&](auto kernel) {
         kernel<<<grid, block, 0, st>>>(b->shots, b->tile_shot, b->ntiles[0], par, it, slot, b->dt, b->invdx, b->invdy,
                                        b->invdz, b->i4xy, b->i4yz, b->i4zx);

@@ -16,14 +16,15 @@
 // (the reference writes them on the interior only and never fills their outer ghosts) and sigma ghosts hold what
 // the caller stored there.
 //
-// Block = 64 x BY threads, one output column per thread, marching over a chunk of z planes. Per plane p the block
-// stages sigma (halo 8) and b (halo 4) tiles in LDS, builds the staggered derivatives d = b D- sigma of plane p on
-// the tile plus a 4-point rim, and absorbs plane p into register queues; output plane o = p - 4 is finalised with
-// the z part coming from a per-thread column stream 7 planes ahead.
+// A block marches over a chunk of z planes with one output column per thread (adjoint, 64 x 8 threads) or per pair of
+// threads, one for each field (forward, 64 x 8 x 2). Per plane p it stages tiles with an 8-point halo in LDS, builds the
+// staggered derivatives d = b D- sigma (of the adjoint's S) of plane p on the tile plus a 4-point rim, and absorbs plane
+// p into register queues; output plane o = p - 4 is finalised with the z part coming from a per-thread column stream 7
+// planes ahead.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
-#include "common.h"
+#include "stencil_common.h"
 #include "tti_fused.h"
 
 #include <initializer_list>
@@ -33,10 +34,8 @@ namespace tti {
 
 namespace fused {
 
-constexpr int BX = 64;
-constexpr int BY = 8;
-constexpr int TW = BX + 16, TH = BY + 16; // sigma tile with halo 8
-constexpr int BW = BX + 8, BH = BY + 8;   // halo-4 tile
+constexpr int TW = BX + 16;               // width of a tile with halo 8
+constexpr int BW = BX + 8;                // and with halo 4
 constexpr int SNAP_SEG = 64;              // points per x-row segment of an FP16 snapshot (one scale each)
 
 struct Snap
@@ -242,26 +241,30 @@ load_quad(const float* __restrict__ base, long idx, int gx, const Box& g, bool r
     return v;
 }
 
-// Quad mappings of the two tile shapes onto the 512 threads of a block.
-constexpr int TQ_PER_ROW = TW / 4, TQ = TQ_PER_ROW * TH; // 20 x 24 = 480 quads
-constexpr int BQ_PER_ROW = BW / 4, BQ = BQ_PER_ROW * BH; // 18 x 16 = 288 quads
-static_assert(TQ <= BX * BY && BQ <= BX * BY, "one quad per thread");
+constexpr int TQ_PER_ROW = TW / 4, BQ_PER_ROW = BW / 4; // quads per row of the two tile shapes
 
 // ------------------------------------------------------------------------------------------------------------------
 // Forward step: u += dt L(sigma) (+ source), sigma_out = A sigma + B dt u_new; optional snapshot of u_new.
 // Same arithmetic as kernels/kernel_type2_fwd_drv.cu:148-362 + kernels/kernel_type2_fwd.cu:264-540 +
 // kernels/kernel_base.cu:82-104, evaluated in one sweep.
 //
-// Pipeline per output plane o (tile plane p = o + 4): the tile of plane p is already in LDS buffer `cur`;
-//   A  load the column words of plane o+1, store the prefetched tile of plane p+1 into buffer 1-cur, fetch the tile
-//      of plane p+2 (loads are issued before this plane's stores: one counter tracks both)
-//   B  staggered derivatives d_x, d_y of plane p on the tile rim -> LDS, barrier
-//   C  D+ of d_x, d_y, the x-y mixed term and the z-mixed partial sums of plane p (registers)
-//   D  d_z(o+4) from the column queue, finalise plane o from the pointwise values prefetched one plane earlier,
-//      load the pointwise values of plane o+1, store plane o
-// Two barriers per plane (between B and C, and at the end): tiles and derivative planes alternate between two LDS
-// buffers by the parity of o.
-// The loop body is instantiated for both parities of o (queue windows and derivative buffers are static).
+// Pipeline per output plane o (tile plane p = o + 4): the tile of plane p is already in LDS buffer `par`;
+//   A  load the column word of plane o + 8, store the prefetched tile of plane p + 1 into the other buffer, fetch the
+//      tile of plane p + 2 (loads are issued before this plane's stores: one counter tracks both)
+//   B  z-mixed partial sums, the x-y mixed term, and the staggered derivatives d_x, d_y of plane p -> LDS
+//   C  d_z(o+4) from the column queue, V and H of plane o; H1 and V2 -> LDS for the other field's thread
+//   -  the one barrier: every read of the tile comes before it, every read of d_x, d_y and H1, V2 after it, and those
+//      alternate between two buffers as the tiles do
+//   D  D+ of d_x, d_y; update and store plane o, load the pointwise words of plane o + 1
+// Planes p outside the chunk feed only z stencils, so their bodies leave d_x, d_y and the x-y term out.
+//
+// What bounds it (512^3, 2.2 GHz under load): VALU issue 58% and LDS 50% of the time in lock-step phases, 11.0 GB moved
+// (4.1 of the 4.97 TB/s of a copy; with six model volumes aliased, 3.2 GB less, it runs 8% faster). One thread per column
+// needed 253 VGPRs (8 waves a CU) where one per column and field takes 120 (16 waves); the tile of 8 rows instead of 4
+// reads 40% fewer halo quads and computes 2 instead of 3 d_y per column, the second barrier went, and the partial sums
+// shift as they are summed. Together 2.82 -> 2.67 ms per step, 2.98 -> 2.90 ms with the FP16 snapshot, and with the
+// shortened rim planes 27 -> 17 us at 64^3. Blocks of 4 rows, two a CU: 2.83 ms.
+//
 // Global addresses are 32-bit byte offsets from the (scalar) base pointers: the launcher checks that every volume is
 // smaller than 4 GiB.
 // ------------------------------------------------------------------------------------------------------------------
@@ -319,25 +322,17 @@ stg8(F&& v)
 }
 
 #ifndef TTI_FWD_BY
-#define TTI_FWD_BY 4
+#define TTI_FWD_BY 8
 #endif
-constexpr int FWD_BY = TTI_FWD_BY;         // rows per forward block (4: two 256-thread blocks per CU)
-#ifndef TTI_FWD_UNROLL
-#define TTI_FWD_UNROLL 2
-#endif
+constexpr int FWD_BY = TTI_FWD_BY; // rows per forward block
 #ifndef TTI_FWD_SETPRIO
 #define TTI_FWD_SETPRIO 1
 #endif
-constexpr int FU = TTI_FWD_UNROLL;         // forward planes per loop iteration (2 or 6)
+constexpr int FU = 2; // forward planes per loop iteration
 constexpr bool FWD_SETPRIO = TTI_FWD_SETPRIO != 0;
-static_assert(FU == 2 || FU == 4 || FU == 6, "forward unroll of 2, 4 or 6 planes");
-constexpr int XITEMS = BY * BW;            // d_x values per plane (576)
-constexpr int XEXTRA = XITEMS - BX * BY;   // handled by a second item on the first threads (64)
-static_assert(XEXTRA > 0 && XEXTRA <= BX * BY, "two d_x items per thread at most");
-static_assert(BH * BX == 2 * BX * BY, "two d_y items per thread");
 
-// One block's tile (bxi, byi, bzi) of a forward step; called by the single-volume kernel and the batched one.
-// FBY = rows per block (8: one 512-thread block per CU; 4: two independent 256-thread blocks per CU).
+// One block's tile (bxi, byi, bzi) of a forward step; called by the single-volume kernel and the batched one. One thread
+// per column and field (threadIdx.z: 0 sigma_H and u, 1 sigma_V and w).
 template <int FBY, int SNAP, bool SPONGE, bool SIG = false>
 __device__ __forceinline__ void
 fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __restrict__ s1o, float* __restrict__ s2o,
@@ -348,28 +343,31 @@ fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __re
          float invdx, float invdy, float invdz, float i4xy, float i4yz, float i4zx, unsigned src_off, float src_val,
          const Snap& snap, int bz, int bxi, int byi, int bzi)
 {
-    // Tiles and derivative planes are double-buffered by the parity of o: a tile buffer is refilled by the next
-    // plane's stage A, after the barrier that ends this plane.
-    constexpr int NT = BX * FBY;                  // threads
+    constexpr int NT = BX * FBY;                  // threads per field
     constexpr int FTH = FBY + 16, FBH = FBY + 8;  // tile heights (halo 8, halo 4)
     constexpr int FTQ = TQ_PER_ROW * FTH, FBQ = BQ_PER_ROW * FBH;
-    constexpr int QT = (FTQ + NT - 1) / NT, QB = (FBQ + NT - 1) / NT; // quads per thread
-    constexpr int FXI = FBY * BW, XI = (FXI + NT - 1) / NT;           // d_x items per thread
-    constexpr int YI = FBH / FBY;                                     // d_y items per thread
+    constexpr int QT = (FTQ + NT - 1) / NT;                 // sigma quads per thread (of its field)
+    constexpr int YI = FBH / FBY;                           // d_y items per thread
     static_assert(FBH % FBY == 0, "d_y rows split evenly over the thread rows");
-    __shared__ __align__(16) float T1[2][FTH][TW];
-    __shared__ __align__(16) float T2[2][FTH][TW]; // sigma, halo 8: (x0-8+lx, y0-8+ly)
-    __shared__ __align__(16) float Bt[2][FBH][BW]; // b, halo 4: (x0-4+lx, y0-4+ly)
-    __shared__ float X1[2][FBY][BW], X2[2][FBY][BW]; // d_x at (x0-4+j, y0+r)
-    __shared__ float Y1[2][FBH][BX], Y2[2][FBH][BX]; // d_y at (x0+c, y0-4+j)
+    static_assert(FBQ <= 2 * NT, "one b quad per thread");
+    __shared__ __align__(16) float T[2][2][FTH][TW]; // [parity][field] sigma, halo 8: (x0-8+lx, y0-8+ly)
+    __shared__ __align__(16) float Bt[2][FBH][BW];   // b, halo 4: (x0-4+lx, y0-4+ly)
+    __shared__ float X[2][2][FBY][BW];               // d_x at (x0-4+j, y0+r)
+    __shared__ float Y[2][2][FBH][BX];               // d_y at (x0+c, y0-4+j)
+    __shared__ float EX[2][2][FBY][BX];              // H1 and V2, which the other field's update needs
 
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
+    const int F = __builtin_amdgcn_readfirstlane(threadIdx.z);
     const int x0 = g.ixbeg + bxi * BX, y0 = g.iybeg + byi * FBY, z0 = g.izbeg + bzi * bz;
     const int z1 = min(z0 + bz, g.izend + 1);
     const int ix = x0 + tx, iy = y0 + ty;
     const bool active = ix <= g.ixend && iy <= g.iyend;
     const unsigned PB = (unsigned)g.ldx * (unsigned)g.ldy * 4u; // bytes per plane
     const unsigned colb = active ? ((unsigned)iy * (unsigned)g.ldx + (unsigned)ix) * 4u : 0u;
+    const float* const s = F ? s2 : s1;
+    float *const so = F ? s2o : s1o, *const uw = F ? w : u;
+    // u += dt (m1 H1 + m4 V1 + m2 V2), w += dt (m2 H1 + m3 V2 + m4 H2), summed in this order
+    const float *const ma = F ? m2 : m1, *const mb = F ? m3 : m4, *const mc = F ? m4 : m2;
     // snapshot element offsets (32-bit: the launchers check that a snapshot field has < 2^32 elements): plane
     // stride, this thread's column within a plane, and its 64-point segment's scale within a plane
     const unsigned s_plane = (unsigned)(snap.ldy * snap.ldx);
@@ -380,10 +378,10 @@ fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __re
         axy = fminf(abx[ix].a, aby[iy].a);
         bxy = fminf(abx[ix].b, aby[iy].b);
     }
-    // tile quads (clamped into the allocation, see quad_off); slots beyond the count map to the last quad (their
-    // loads and stores are skipped)
-    int tq_row[QT], tq_lx[QT], bq_row[QB], bq_lx[QB];
-    unsigned tqb[QT], bqb[QB];
+    // tile quads (clamped into the allocation, see quad_off): sigma of this thread's field, b over all threads. Slots
+    // past a tile's quad count load and store nothing, so whole waves skip them
+    int tq_row[QT], tq_lx[QT];
+    unsigned tqb[QT];
 #pragma unroll
     for (int k = 0; k < QT; ++k) {
         const int q = min(tid + k * NT, FTQ - 1);
@@ -391,337 +389,257 @@ fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __re
         tq_lx[k] = 4 * (q - tq_row[k] * TQ_PER_ROW);
         tqb[k] = quad_off(g, x0 - 8 + tq_lx[k], y0 - 8 + tq_row[k]);
     }
-#pragma unroll
-    for (int k = 0; k < QB; ++k) {
-        const int q = min(tid + k * NT, FBQ - 1);
-        bq_row[k] = q / BQ_PER_ROW;
-        bq_lx[k] = 4 * (q - bq_row[k] * BQ_PER_ROW);
-        bqb[k] = quad_off(g, x0 - 4 + bq_lx[k], y0 - 4 + bq_row[k]);
-    }
-    // Prefetch registers come in two sets selected by the parity of the plane: a body fills the set the next body
-    // drains, so no loaded register is ever copied (a copy would wait for the load, and for every load before it).
-    float4 pt1[2][QT], pt2[2][QT], pb[2][QB];
-    // quad slots past a tile's quad count load and store nothing, so whole waves skip them (at 64 x 4 the second
-    // sigma slot holds 144 quads for 256 threads: 2.98 instead of 3.04 ms per step at 512^3)
+    const int bq_id = tid + F * NT, bq_row = min(bq_id, FBQ - 1) / BQ_PER_ROW,
+              bq_lx = 4 * (min(bq_id, FBQ - 1) - bq_row * BQ_PER_ROW);
+    const unsigned bqb = quad_off(g, x0 - 4 + bq_lx, y0 - 4 + bq_row);
     auto tq_ok = [&](int k) { return k * NT + NT <= FTQ || tid + k * NT < FTQ; };
-    auto bq_ok = [&](int k) { return k * NT + NT <= FBQ || tid + k * NT < FBQ; };
-    auto fetch = [&](int pp, int set) {
+    float4 pt[QT], pb;
+    auto fetch = [&](int pp) {
         const unsigned o = (unsigned)pp * PB;
 #pragma unroll
-        for (int k = 0; k < QT; ++k) {
-            if (tq_ok(k)) {
-                pt1[set][k] = ldf4(s1, o + tqb[k]);
-                pt2[set][k] = ldf4(s2, o + tqb[k]);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < QB; ++k)
-            if (bq_ok(k))
-                pb[set][k] = ldf4(b, o + bqb[k]);
+        for (int k = 0; k < QT; ++k)
+            if (tq_ok(k))
+                pt[k] = ldf4(s, o + tqb[k]);
+        if (bq_id < FBQ)
+            pb = ldf4(b, o + bqb);
     };
-    auto commit = [&](int buf, int set) {
+    auto commit = [&](int buf) {
 #pragma unroll
-        for (int k = 0; k < QT; ++k) {
-            if (tq_ok(k)) {
-                *reinterpret_cast<float4*>(&T1[buf][tq_row[k]][tq_lx[k]]) = pt1[set][k];
-                *reinterpret_cast<float4*>(&T2[buf][tq_row[k]][tq_lx[k]]) = pt2[set][k];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < QB; ++k)
-            if (bq_ok(k))
-                *reinterpret_cast<float4*>(&Bt[buf][bq_row[k]][bq_lx[k]]) = pb[set][k];
+        for (int k = 0; k < QT; ++k)
+            if (tq_ok(k))
+                *reinterpret_cast<float4*>(&T[buf][F][tq_row[k]][tq_lx[k]]) = pt[k];
+        if (bq_id < FBQ)
+            *reinterpret_cast<float4*>(&Bt[buf][bq_row][bq_lx]) = pb;
     };
-    // d_x items (r, j): item k is tid + k * NT; d_y items: rows ty + h * FBY of the halo-4 band, column tx.
-    // The scale is 1/d for interior points and zero elsewhere (floats: no lane masks live across the loop).
-    int xr[XI], xj[XI];
-    float xs[XI], ys[YI];
-#pragma unroll
-    for (int k = 0; k < XI; ++k) {
-        const int it = min(tid + k * NT, FXI - 1);
-        xr[k] = it / BW;
-        xj[k] = it - xr[k] * BW;
-        xs[k] = in_xy(g, x0 - 4 + xj[k], y0 + xr[k]) ? invdx : 0.0f; // repeated items compute the same value
-    }
+    // d_x items: the thread's own column, whose taps the z-x term needs as well, and the 4 rim columns on either side of
+    // each row on the first threads; d_y items: rows ty + h * FBY of the halo-4 band, column tx (between them the taps
+    // of the y-z term). The scale is 1/d for interior points and zero elsewhere (floats: no lane masks live across the
+    // loop).
+    constexpr int XE = 8 * FBY; // rim items
+    static_assert(XE <= NT, "one rim item per thread");
+    const int xe_r = min(tid, XE - 1) / 8, xe_k = min(tid, XE - 1) % 8, xe_j = xe_k < 4 ? xe_k : BX + xe_k;
+    const float xs = in_xy(g, ix, iy) ? invdx : 0.0f;
+    const float xes = in_xy(g, x0 - 4 + xe_j, y0 + xe_r) ? invdx : 0.0f;
+    float ys[YI];
 #pragma unroll
     for (int h = 0; h < YI; ++h)
         ys[h] = in_xy(g, x0 + tx, y0 - 4 + ty + h * FBY) ? invdy : 0.0f;
 
     // Register queues along z. The loop body is instantiated for FU consecutive planes; the body of plane o with
-    // c = o - (z0 - 8) mod FU sees each queue through a window starting at slot c (FU - 1 spare slots per queue), and
-    // after the FU-th plane the queues shift by FU: one register move per live value every FU planes.
-    float sq1[8 + FU], sq2[8 + FU]; // sigma(o + k)   at [c + k], k = 0..7 (slot c + 8 receives sigma(o + 8))
-    float dz1[7 + FU], dz2[7 + FU]; // d_z(o - 3 + k) at [c + k], k = 0..7
-    float xx1[4 + FU], xx2[4 + FU]; // D+_x d_x (o + k), unscaled by rho, at [c + k], k = 0..4
-    float yy1[4 + FU], yy2[4 + FU]; // D+_y d_y
-    float xy1[4 + FU], xy2[4 + FU]; // X_xy sigma
-    float qx1[8 + FU], qx2[8 + FU]; // z-x mixed partial sums of output o + j at [c + j], j = 0..8
-    float qy1[8 + FU], qy2[8 + FU]; // y-z mixed partial sums
+    // c = o - (z0 - 8) mod FU sees each delay queue through a window starting at slot c (FU - 1 spare slots per queue),
+    // and after the FU-th plane the queues shift by FU. The partial sums shift as they are summed (absorb).
+    float sq[8 + FU]; // sigma(o + k)   at [c + k], k = 0..7 (slot c + 8 receives sigma(o + 8))
+    float dz[7 + FU]; // d_z(o - 3 + k) at [c + k], k = 0..7
+    float xx[4 + FU]; // D+_x d_x (o + k), unscaled by rho, at [c + k], k = 0..4
+    float yy[4 + FU]; // D+_y d_y
+    float xy[4 + FU]; // X_xy sigma
+    float bq[4 + FU]; // b(o + k), from the tile's centre: for d_z(o + 4) and the output plane
+    float qx[9], qy[9]; // z-x and y-z mixed partial sums of output o + j
 #pragma unroll
     for (int k = 0; k < 7 + FU; ++k)
-        dz1[k] = dz2[k] = 0.0f;
+        dz[k] = 0.0f;
 #pragma unroll
     for (int k = 0; k < 4 + FU; ++k)
-        xx1[k] = xx2[k] = yy1[k] = yy2[k] = xy1[k] = xy2[k] = 0.0f;
+        xx[k] = yy[k] = xy[k] = bq[k] = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 8 + FU; ++k)
-        qx1[k] = qx2[k] = qy1[k] = qy2[k] = 0.0f;
-    // column words: sigma and b at a plane clamped into the allocation (a clamped sigma only meets a zero b; b is
-    // zeroed outside the interior planes where it is used, not where it is loaded)
-    auto col = [&](const float* __restrict__ v, int q) {
-        return ldf(v, (unsigned)min(max(q, g.izbeg - R), g.izend + R) * PB + colb);
-    };
+    for (int k = 0; k < 9; ++k)
+        qx[k] = qy[k] = 0.0f;
+    // column words: sigma at a plane clamped into the allocation (a clamped sigma only meets a zero b; b is zeroed
+    // outside the interior planes where it is used)
+    auto col = [&](int q) { return ldf(s, (unsigned)min(max(q, g.izbeg - R), g.izend + R) * PB + colb); };
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        sq1[k] = col(s1, z0 - 8 + k);
-        sq2[k] = col(s2, z0 - 8 + k);
-    }
-    // b(o + k) at [c + k], k = 0..5: b(o + 4) for d_z(o + 4), and b(o) for the output plane, which is not loaded
-    // again 5 planes later when L2 no longer holds it (2.95 -> 2.87 ms per step at 512^3, 3.11 -> 3.03 ms with the
-    // FP16 snapshot)
-    float bq[5 + FU];
-#pragma unroll
-    for (int k = 0; k < 5; ++k)
-        bq[k] = col(b, z0 - 8 + k);
-    // pointwise words of an output plane, one set per parity: m1 m2 m3 m4 rx ry rz, slot 7 unused (b comes from the
-    // b queue), u w
-    float pw[2][10];
-    auto fetch_point = [&](int o, int set) {
+    for (int k = 0; k < 8; ++k)
+        sq[k] = col(z0 - 8 + k);
+    // pointwise words of an output plane: rx ry rz are loaded again once their plane's V and H are formed, the model
+    // words and u or w once its update is, so each has a whole plane to arrive
+    float pr[3], pm[4];
+    auto fetch_r = [&](int o) {
         if (o >= z0 && o < z1) {
             const unsigned io = (unsigned)o * PB + colb;
-            pw[set][0] = ldf(m1, io);
-            pw[set][1] = ldf(m2, io);
-            pw[set][2] = ldf(m3, io);
-            pw[set][3] = ldf(m4, io);
-            pw[set][4] = ldf(vrx, io);
-            pw[set][5] = ldf(vry, io);
-            pw[set][6] = ldf(vrz, io);
-            pw[set][8] = ldf(u, io);
-            pw[set][9] = ldf(w, io);
+            pr[0] = ldf(vrx, io);
+            pr[1] = ldf(vry, io);
+            pr[2] = ldf(vrz, io);
+        }
+    };
+    auto fetch_m = [&](int o) {
+        if (o >= z0 && o < z1) {
+            const unsigned io = (unsigned)o * PB + colb;
+            pm[0] = ldf(ma, io);
+            pm[1] = ldf(mb, io);
+            pm[2] = ldf(mc, io);
+            pm[3] = ldf(uw, io);
         }
     };
 
-    fetch(z0 - R, 0);
-    commit(0, 0);
-    fetch(z0 - R + 1, 0);
+    fetch(z0 - R);
+    commit(0);
+    fetch(z0 - R + 1);
     __syncthreads();
 
-    auto body = [&](auto curc, int o) {
+    auto body = [&](auto curc, auto ownc, int o) {
         constexpr int cur = decltype(curc)::value; // o - (z0 - 8) mod FU: queue window
-        constexpr int par = cur & 1;               // parity of o: prefetch set and derivative buffer
-        // tile buffer of plane p and of plane p + 1, by parity: compile-time, so each LDS address is a thread base
-        // plus constants (with three buffers rotating at run time under a two-plane unroll, every tap address took
-        // a scalar buffer base: 45 more VALU instructions per two planes; the second barrier per plane that two
-        // buffers need costs less: 2.90 -> 2.88 ms per step at 512^3, 3.06 -> 3.02 ms with the FP16 snapshot)
-        constexpr int tb = par, tn = par ^ 1;
+        constexpr bool own = decltype(ownc)::value; // plane p = o + 4 is one of the block's output planes
+        constexpr int par = cur & 1;               // parity of o: tile buffer of plane p (the other: p + 1)
         const int p = o + R;
-        const float pin = (p >= g.izbeg && p <= g.izend) ? 1.0f : 0.0f;
-        const int qd = o + R;
-        const float bd = (qd >= g.izbeg && qd <= g.izend) ? bq[cur + 4] : 0.0f;
-        // ---- A: issue this plane's loads first, so that waiting for them never waits for the stores below (one
-        // counter covers loads and stores): column words of plane o + 1, then the tile of plane p + 1 goes to buffer
-        // tn (last read by the previous plane, before the barrier that ended it) and the tile of plane p + 2 is fetched. The
-        // wave runs this stage at raised priority, so its loads go out ahead of the other block's arithmetic
-        // (measured at 512^3: -1% per step, -2% with the FP16 snapshot; the adjoint gains nothing from it).
+        const bool pint = p >= g.izbeg && p <= g.izend;
+        const float pin = pint ? 1.0f : 0.0f;
+        // ---- A: this plane's loads first, so that waiting for them never waits for the stores below (one counter covers
+        // loads and stores): the column word of plane o + 8; the tile of plane p + 1 goes to the other buffer (last read
+        // before the previous plane's barrier) and the tile of plane p + 2 is fetched
         if (FWD_SETPRIO)
             __builtin_amdgcn_s_setprio(3);
-        sq1[cur + 8] = col(s1, o + 8);
-        sq2[cur + 8] = col(s2, o + 8);
-        bq[cur + 5] = col(b, o + 5);
+        sq[cur + 8] = col(o + 8);
         if (p + 1 <= z1 + R - 1)
-            commit(tn, par);
+            commit(par ^ 1);
         if (p + 2 <= z1 + R - 1)
-            fetch(p + 2, par ^ 1);
-        // pointwise words of plane o + 1 into the set that plane o - 1 drained in its stage D: issued here they have
-        // the whole plane to arrive (at the end of stage D they had part of the next one: 3.34 -> 3.14 ms for the
-        // FP16-snapshot step at 512^3, 3.06 -> 3.04 ms without; the adjoint's pointwise words gain nothing from it)
-        fetch_point(o + 1, par ^ 1);
+            fetch(p + 2);
         if (FWD_SETPRIO)
             __builtin_amdgcn_s_setprio(0);
-        // ---- B: d_x on rows of the tile (x' in [x0-4, x0+68)), d_y on columns (y' in [y0-4, y0+BY+4))
-        // (the scale is zero for non-interior points: every tile value is finite)
-#pragma unroll
-        for (int i = 0; i < XI; ++i) {
-            // items past the count (first wave only for the last slot) repeat the last item: same value, same word
-            if (i == 0 || tid + i * NT < FXI || tid < BX) {
-                const float bb = Bt[tb][xr[i] + 4][xj[i]] * (xs[i] * pin);
-                X1[par][xr[i]][xj[i]] = bb * stg8([&](int k) { return T1[tb][xr[i] + 8][xj[i] + k]; });
-                X2[par][xr[i]][xj[i]] = bb * stg8([&](int k) { return T2[tb][xr[i] + 8][xj[i] + k]; });
-            }
-        }
-#pragma unroll
-        for (int h = 0; h < YI; ++h) {
-            const int j = ty + h * FBY;
-            const float bb = Bt[tb][j][tx + 4] * (ys[h] * pin);
-            Y1[par][j][tx] = bb * stg8([&](int k) { return T1[tb][j + k][tx + 8]; });
-            Y2[par][j][tx] = bb * stg8([&](int k) { return T2[tb][j + k][tx + 8]; });
-        }
-        __syncthreads();
-        // ---- C: plane-p contributions
-        if (active) {
-            float fx1 = 0, fx2 = 0, fy1 = 0, fy2 = 0, fxy1 = 0, fxy2 = 0;
+        const float(*t)[TW] = T[par][F];
+        // ---- B: the z-mixed partial sums; from the planes whose own outputs this block computes also the x-y mixed term,
+        // d_x on rows of the tile (x' in [x0-4, x0+68)) and d_y on columns (y' in [y0-4, y0+BY+4)) (the scale is zero for
+        // non-interior points: every tile value is finite)
+        {
+            float ddx[5], ddy[5];
 #pragma unroll
             for (int n = 1; n <= R; ++n) {
-                const float c = cstg(n);
-                fx1 += c * (X1[par][ty][tx + 4 + n] - X1[par][ty][tx + 5 - n]);
-                fx2 += c * (X2[par][ty][tx + 4 + n] - X2[par][ty][tx + 5 - n]);
-                fy1 += c * (Y1[par][ty + 4 + n][tx] - Y1[par][ty + 5 - n][tx]);
-                fy2 += c * (Y2[par][ty + 4 + n][tx] - Y2[par][ty + 5 - n][tx]);
-                const float e = ecen(n);
-                fxy1 += e * ((T1[tb][ty + 8 + n][tx + 8 + n] - T1[tb][ty + 8 - n][tx + 8 + n]) +
-                             (T1[tb][ty + 8 - n][tx + 8 - n] - T1[tb][ty + 8 + n][tx + 8 - n]));
-                fxy2 += e * ((T2[tb][ty + 8 + n][tx + 8 + n] - T2[tb][ty + 8 - n][tx + 8 + n]) +
-                             (T2[tb][ty + 8 - n][tx + 8 - n] - T2[tb][ty + 8 + n][tx + 8 - n]));
-                // plane p at x-offset +n feeds output p - n (q[4 - n]); at -n output p + n (q[4 + n]), sign flipped
-                const float dx1 = T1[tb][ty + 8][tx + 8 + n] - T1[tb][ty + 8][tx + 8 - n];
-                const float dx2 = T2[tb][ty + 8][tx + 8 + n] - T2[tb][ty + 8][tx + 8 - n];
-                const float dy1 = T1[tb][ty + 8 + n][tx + 8] - T1[tb][ty + 8 - n][tx + 8];
-                const float dy2 = T2[tb][ty + 8 + n][tx + 8] - T2[tb][ty + 8 - n][tx + 8];
-                qx1[cur + 4 - n] += e * dx1;
-                qx1[cur + 4 + n] -= e * dx1;
-                qx2[cur + 4 - n] += e * dx2;
-                qx2[cur + 4 + n] -= e * dx2;
-                qy1[cur + 4 - n] += e * dy1;
-                qy1[cur + 4 + n] -= e * dy1;
-                qy2[cur + 4 - n] += e * dy2;
-                qy2[cur + 4 + n] -= e * dy2;
+                ddx[n] = t[ty + 8][tx + 8 + n] - t[ty + 8][tx + 8 - n];
+                ddy[n] = t[ty + 8 + n][tx + 8] - t[ty + 8 - n][tx + 8];
+                hold(ddx[n]), hold(ddy[n]);
             }
-            xx1[cur + 4] = fx1 * invdx;
-            xx2[cur + 4] = fx2 * invdx;
-            yy1[cur + 4] = fy1 * invdy;
-            yy2[cur + 4] = fy2 * invdy;
-            xy1[cur + 4] = fxy1 * i4xy;
-            xy2[cur + 4] = fxy2 * i4xy;
+            absorb<R>(qx, ddx);
+            absorb<R>(qy, ddy);
         }
-        // ---- D: d_z(o+4) and the finalisation of plane o
-        {
-            const float dzs = bd * invdz;
-            dz1[cur + 7] = dzs * stg8([&](int k) { return sq1[cur + k]; });
-            dz2[cur + 7] = dzs * stg8([&](int k) { return sq2[cur + k]; });
-            if (g.fs && o == g.izbeg) {
-                mirror_dz<cur>(dz1);
-                mirror_dz<cur>(dz2);
+        if constexpr (own) {
+            float fxy = 0;
+#pragma unroll
+            for (int n = 1; n <= R; ++n) {
+                fxy += ecen(n) * ((t[ty + 8 + n][tx + 8 + n] - t[ty + 8 - n][tx + 8 + n]) +
+                                  (t[ty + 8 - n][tx + 8 - n] - t[ty + 8 + n][tx + 8 - n]));
+                hold(fxy);
+            }
+            xy[cur + 4] = fxy * i4xy;
+            hold(xy[cur + 4]);
+            float xv = Bt[par][ty + 4][tx + 4] * (xs * pin) * stg8([&](int k) { return t[ty + 8][tx + 4 + k]; });
+            hold(xv);
+            X[par][F][ty][tx + 4] = xv;
+            if (tid < XE) {
+                xv = Bt[par][xe_r + 4][xe_j] * (xes * pin) * stg8([&](int k) { return t[xe_r + 8][xe_j + k]; });
+                hold(xv);
+                X[par][F][xe_r][xe_j] = xv;
+            }
+#pragma unroll
+            for (int h = 0; h < YI; ++h) {
+                const int j = ty + h * FBY;
+                float yv = Bt[par][j][tx + 4] * (ys[h] * pin) * stg8([&](int k) { return t[j + k][tx + 8]; });
+                hold(yv);
+                Y[par][F][j][tx] = yv;
             }
         }
-        const bool fin = o >= z0 && active;
-        float unew = 0.0f, wnew = 0.0f, s1n = 0.0f, s2n = 0.0f;
-        const unsigned io = (unsigned)o * PB + colb;
-        if (fin) {
-            const float fz1 = stg8([&](int k) { return dz1[cur + k]; });
-            const float fz2 = stg8([&](int k) { return dz2[cur + k]; });
-            const float* P = pw[par];
-            const float mm1 = P[0], mm2 = P[1], mm3 = P[2], mm4 = P[3], vx = P[4], vy = P[5], vz = P[6];
-            const float uo = P[8], wo = P[9];
+        // ---- C: d_z(o+4), then V and H of plane o
+        bq[cur + 4] = Bt[par][ty + 4][tx + 4];
+        dz[cur + 7] = (pint ? bq[cur + 4] : 0.0f) * invdz * stg8([&](int k) { return sq[cur + k]; });
+        if (g.fs && o == g.izbeg)
+            mirror_dz<cur>(dz);
+        float V = 0.0f, Hf = 0.0f;
+        if (o >= z0) {
+            const float fz = stg8([&](int k) { return dz[cur + k]; });
+            const float vx = pr[0], vy = pr[1], vz = pr[2];
             const float rho = recip(bq[cur]);
-            const float f1xx = xx1[cur] * rho, f2xx = xx2[cur] * rho;
-            const float f1yy = yy1[cur] * rho, f2yy = yy2[cur] * rho;
-            const float f1zz = fz1 * invdz * rho, f2zz = fz2 * invdz * rho;
-            const float f1xy = xy1[cur], f2xy = xy2[cur];
-            const float f1zx = qx1[cur] * i4zx, f2zx = qx2[cur] * i4zx;
-            const float f1yz = qy1[cur] * i4yz, f2yz = qy2[cur] * i4yz;
+            const float fxx = xx[cur] * rho, fyy = yy[cur] * rho, fzz = fz * invdz * rho;
+            const float fzx = qx[0] * i4zx, fyz = qy[0] * i4yz;
             const float rx2 = vx * vx, ry2 = vy * vy, rz2 = vz * vz;
             const float rxy = 2.0f * vx * vy, ryz = 2.0f * vy * vz, rzx = 2.0f * vz * vx;
             // sums of products are written as explicit fmaf chains (left to right): with contraction left to the
             // compiler, copies of this body (the loop's warm-up planes vs the rest) may fuse different products and
             // round differently, which would make a point's value depend on where its z chunk starts
-            const float V1 = fmaf(ryz, f1yz, fmaf(rzx, f1zx, fmaf(rxy, f1xy, fmaf(rz2, f1zz, fmaf(ry2, f1yy, rx2 * f1xx)))));
-            const float H1 = __fsub_rn(__fadd_rn(__fadd_rn(f1xx, f1yy), f1zz), V1); // plain adds: no product fused
-            const float V2 = fmaf(ryz, f2yz, fmaf(rzx, f2zx, fmaf(rxy, f2xy, fmaf(rz2, f2zz, fmaf(ry2, f2yy, rx2 * f2xx)))));
-            const float H2 = __fsub_rn(__fadd_rn(__fadd_rn(f2xx, f2yy), f2zz), V2);
-            const float r3 = fmaf(mm2, V2, fmaf(mm4, V1, mm1 * H1));
-            const float r4 = fmaf(mm4, H2, fmaf(mm3, V2, mm2 * H1));
-            unew = uo + r3 * dt;
-            wnew = wo + r4 * dt;
-            if (io == src_off) {
-                unew += src_val;
-                wnew += src_val;
+            V = fmaf(ryz, fyz, fmaf(rzx, fzx, fmaf(rxy, xy[cur], fmaf(rz2, fzz, fmaf(ry2, fyy, rx2 * fxx)))));
+            Hf = __fsub_rn(__fadd_rn(__fadd_rn(fxx, fyy), fzz), V); // plain adds: no product fused
+            EX[par][F][ty][tx] = F ? V : Hf;
+        }
+        fetch_r(o + 1);
+        // the one barrier of the plane: X, Y and EX of this plane are complete, and every read of tile buffer `par` and
+        // of the previous plane's X, Y, EX buffers is done
+        __syncthreads();
+        // ---- D: D+ of d_x, d_y of plane p, and the update of plane o
+        if constexpr (own) {
+            float fx = 0, fy = 0;
+#pragma unroll
+            for (int n = 1; n <= R; ++n) {
+                const float c = cstg(n);
+                fx += c * (X[par][F][ty][tx + 4 + n] - X[par][F][ty][tx + 5 - n]);
+                fy += c * (Y[par][F][ty + 4 + n][tx] - Y[par][F][ty + 5 - n][tx]);
+                hold(fx), hold(fy);
             }
+            xx[cur + 4] = fx * invdx;
+            yy[cur + 4] = fy * invdy;
+            hold(xx[cur + 4]), hold(yy[cur + 4]);
+        }
+        const bool fin = o >= z0 && active;
+        float unew = 0.0f, snew = 0.0f;
+        const unsigned io = (unsigned)o * PB + colb;
+        if (o >= z0) {
+            const float e = EX[par][F ^ 1][ty][tx];
+            const float r = F ? fmaf(pm[2], Hf, fmaf(pm[1], V, pm[0] * e)) : fmaf(pm[2], e, fmaf(pm[1], V, pm[0] * Hf));
+            unew = pm[3] + r * dt;
+            if (io == src_off)
+                unew += src_val;
             float a = 1.0f, bb = 1.0f;
             if constexpr (SPONGE) {
                 a = fminf(axy, abz[o].a);
                 bb = fminf(bxy, abz[o].b);
             }
-            s1n = fmaf(bb * unew, dt, a * sq1[cur]);
-            s2n = fmaf(bb * wnew, dt, a * sq2[cur]);
+            snew = fmaf(bb * unew, dt, a * sq[cur]);
         }
+        fetch_m(o + 1);
         // the stores of plane o
         if (fin) {
-            stf(u, io, unew);
-            stf(w, io, wnew);
-            stf(s1o, io, s1n);
-            stf(s2o, io, s2n);
+            stf(uw, io, unew);
+            stf(so, io, snew);
         }
         if (SNAP != TTI_SNAP_NONE && o >= z0 && iy <= g.iyend) {
             const unsigned pz = (unsigned)(o - g.izbeg);
             const unsigned idx = pz * s_plane + s_col;
             const unsigned sidx = pz * (s_plane / SNAP_SEG) + s_scol;
-            snap_store(SNAP, snap.a, snap.sa, idx, sidx, active, unew);
-            snap_store(SNAP, snap.b, snap.sb, idx, sidx, active, wnew);
-            if constexpr (SIG) { // the sigma this step read (its u, w update used it)
-                snap_store(SNAP, snap.c, snap.sc, idx, sidx, active, sq1[cur]);
-                snap_store(SNAP, snap.d, snap.sd, idx, sidx, active, sq2[cur]);
-            }
+            snap_store(SNAP, F ? snap.b : snap.a, F ? snap.sb : snap.sa, idx, sidx, active, unew);
+            if constexpr (SIG) // the sigma this step read (its u, w update used it)
+                snap_store(SNAP, F ? snap.d : snap.c, F ? snap.sd : snap.sc, idx, sidx, active, sq[cur]);
         }
-        __syncthreads(); // tile buffer tb is refilled by the next plane
         if (cur == FU - 1) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                sq1[k] = sq1[k + FU];
-                sq2[k] = sq2[k + FU];
-            }
+            for (int k = 0; k < 8; ++k)
+                sq[k] = sq[k + FU];
 #pragma unroll
-            for (int k = 0; k < 7; ++k) {
-                dz1[k] = dz1[k + FU];
-                dz2[k] = dz2[k + FU];
-            }
-#pragma unroll
-            for (int k = 0; k < 5; ++k)
-                bq[k] = bq[k + FU];
+            for (int k = 0; k < 7; ++k)
+                dz[k] = dz[k + FU];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                xx1[k] = xx1[k + FU];
-                xx2[k] = xx2[k + FU];
-                yy1[k] = yy1[k + FU];
-                yy2[k] = yy2[k + FU];
-                xy1[k] = xy1[k + FU];
-                xy2[k] = xy2[k + FU];
+                xx[k] = xx[k + FU];
+                yy[k] = yy[k + FU];
+                xy[k] = xy[k + FU];
+                bq[k] = bq[k + FU];
             }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                qx1[k] = qx1[k + FU];
-                qx2[k] = qx2[k + FU];
-                qy1[k] = qy1[k + FU];
-                qy2[k] = qy2[k + FU];
-            }
-#pragma unroll
-            for (int k = 8; k < 8 + FU; ++k)
-                qx1[k] = qx2[k] = qy1[k] = qy2[k] = 0.0f;
         }
     };
 
-    // FU bodies per iteration; the chunk may end after any of them
-    for (int o = z0 - 8; o < z1; o += FU) {
-        body(std::integral_constant<int, 0>{}, o);
-        if (o + 1 >= z1)
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, 1>;
+    // planes that only feed the z stencils of the block's outputs: 4 before them and 4 after
+    auto rim = [&](int o, int end) {
+        for (; o < end; ++o)
+            if (((o - z0) & 1) == 0)
+                body(C0{}, std::false_type{}, o);
+            else
+                body(C1{}, std::false_type{}, o);
+    };
+    rim(z0 - 8, z0 - 4);
+    for (int o = z0 - 4; o < z1 - 4; o += 2) {
+        body(C0{}, std::true_type{}, o);
+        if (o + 1 >= z1 - 4)
             break;
-        body(std::integral_constant<int, 1>{}, o + 1);
-        if constexpr (FU >= 4) {
-            if (o + 2 >= z1)
-                break;
-            body(std::integral_constant<int, 2>{}, o + 2);
-            if (o + 3 >= z1)
-                break;
-            body(std::integral_constant<int, 3>{}, o + 3);
-        }
-        if constexpr (FU == 6) {
-            if (o + 4 >= z1)
-                break;
-            body(std::integral_constant<int, 4>{}, o + 4);
-            if (o + 5 >= z1)
-                break;
-            body(std::integral_constant<int, 5>{}, o + 5);
-        }
+        body(C1{}, std::true_type{}, o + 1);
     }
+    rim(z1 - 4, z1);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -1263,12 +1181,12 @@ inject_point(float* __restrict__ u, float* __restrict__ w, float* __restrict__ a
 // Host-side argument checks shared by the launchers
 // ------------------------------------------------------------------------------------------------------------------
 
-// Resident blocks on the whole GPU (two 256-thread forward blocks or one 512-thread adjoint block per CU, by their
-// registers) and the cost of a chunk's 8 recomputed planes and prologue, for chunk_depth; [0] forward, [1] adjoint.
+// Resident blocks on the whole GPU (one 1024-thread forward or 512-thread adjoint block per CU, by their registers) and
+// the cost of a chunk's 8 recomputed planes and prologue, for chunk_depth; [0] forward, [1] adjoint.
 // Measured over z depths of 2 to 256 planes on volumes of 40^3 to 400^3, a step takes 2.43 us (forward, two blocks per
 // CU; 2.05 us one) and 3.2 us (adjoint) per plane and round within 8%. Against 128-plane chunks throughout: 64^3 149 ->
 // 27 us forward and 193 -> 38 us adjoint, 128^3 281 -> 58 and 359 -> 75 us.
-constexpr int STEP_SLOTS[2] = { 2 * CUS, CUS };
+constexpr int STEP_SLOTS[2] = { CUS, CUS };
 constexpr float STEP_WARM = 9.5f;
 
 // The fused kernels stage tiles with 16-byte loads: the interior must start on a 4-float boundary, rows must be a

@@ -41,9 +41,36 @@ here(unsigned off)
 // Keeps v where it is computed: without it the compiler sinks a plane's sums to the end of the loop body, past the
 // next plane's work, with every LDS word they need held in registers until then.
 __device__ __forceinline__ void
-pin(float& v)
+hold(float& v)
 {
     asm volatile("" : "+v"(v));
+}
+
+// a b + c as a three-address v_fma_f32. The compiler prefers v_fmac (result in c's register) and, where the result
+// belongs elsewhere, a move: 18 of 236 VALU instructions a plane in the forward step.
+__device__ __forceinline__ float
+fma3(float a, float b, float c)
+{
+    float r;
+    asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r) : "s"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// Moves the queue of mixed partial sums one plane on and absorbs the differences d[1..RO] of that plane, in one FMA per
+// slot: afterwards q[j] belongs to output plane p - RO + j (plane p at offset +n feeds output p - n, at -n output p + n
+// with the sign flipped). Slots go upwards, so each is read by its left neighbour before it is written.
+template <int RO>
+__device__ __forceinline__ void
+absorb(float (&q)[2 * RO + 1], const float (&d)[RO + 1])
+{
+#pragma unroll
+    for (int j = 0; j < 2 * RO; ++j) {
+        const int n = j < RO ? RO - j : j - RO;
+        q[j] = n ? fma3(j < RO ? FD<RO>::e[n] : -FD<RO>::e[n], d[n], q[j + 1]) : q[j + 1];
+        hold(q[j]);
+    }
+    q[2 * RO] = -FD<RO>::e[RO] * d[RO];
+    hold(q[2 * RO]);
 }
 
 // Words of a plane: `plane` is a scalar (the volume plus a uniform plane or tile-origin offset), `off` a 32-bit byte

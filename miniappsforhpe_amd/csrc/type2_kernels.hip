@@ -28,22 +28,6 @@ constexpr Chunk FWD_DRV16_CHUNK{ 1, 6.0f }, FWD_UPDATE16_CHUNK{ 1, 17.5f }, ADJ_
     ADJ_UPDATE16_CHUNK{ 1, 6.0f, 64 };
 
 
-// Moves the queue of mixed partial sums one plane on and absorbs the differences d[1..RO] of that plane, in one FMA per
-// slot: afterwards q[j] belongs to output plane p - RO + j (plane p at offset +n feeds output p - n, at -n output p + n
-// with the sign flipped). Slots go upwards, so each is read by its left neighbour before it is written.
-template <int RO>
-__device__ __forceinline__ void
-absorb(float (&q)[2 * RO + 1], const float (&d)[RO + 1])
-{
-#pragma unroll
-    for (int j = 0; j <= 2 * RO; ++j) {
-        const int n = j < RO ? RO - j : j - RO;
-        const float e = j < RO ? FD<RO>::e[n] : -FD<RO>::e[n], next = j < 2 * RO ? q[j + 1] : 0.0f;
-        q[j] = n ? fmaf(e, d[n], next) : next;
-        pin(q[j]);
-    }
-}
-
 // ------------------------------------------------------------------------------------------------------------------
 // a2: d_a f = b * D-_a f  (kernels/kernel_type2_fwd_drv.cu:148-362; launcher :368-409)
 // ------------------------------------------------------------------------------------------------------------------
@@ -496,7 +480,7 @@ __global__ __launch_bounds__(2 * BX* BY) void k_fwd_update_q(
                                  (S[ty + RO - n][tx + HX - n] - S[ty + RO + n][tx + HX - n]));
             ddx[n] = S[ty + RO][tx + HX + n] - S[ty + RO][tx + HX - n];
             ddy[n] = S[ty + RO + n][tx + HX] - S[ty + RO - n][tx + HX];
-            pin(a), pin(ddx[n]), pin(ddy[n]);
+            hold(a), hold(ddx[n]), hold(ddy[n]);
         }
         absorb<RO>(qzx, ddx);
         absorb<RO>(qyz, ddy);
