@@ -99,7 +99,7 @@ __global__ __launch_bounds__(2 * BX* FWD_BY, 4) void k_fused_fwd_batch(const Sho
 }
 
 template <int SNAP, bool SPONGE>
-__global__ __launch_bounds__(ADJ_AX* ADJ_AY, ADJ_AX* ADJ_AY <= 256 ? 2 : 1) void k_fused_adj_batch(const ShotDev* __restrict__ shots,
+__global__ __launch_bounds__(2 * ADJ_AX* ADJ_AY, 4) void k_fused_adj_batch(const ShotDev* __restrict__ shots,
                                                             const int* __restrict__ tile_shot, int ntiles, int par,
                                                             int slot, float dt, float invdx, float invdy, float invdz,
                                                             float i4xy, float i4yz, float i4zx)
@@ -211,7 +211,7 @@ adj_step(tti_batch* b, int par, int n, int slot, hipStream_t st)
         return TTI_EINVAL;
     if (b->maxrec > 0 && !b->have_residual)
         return TTI_EINVAL;
-    const dim3 grid(((b->ntiles[1] + 7) / 8) * 8), block(ADJ_AX, ADJ_AY);
+    const dim3 grid(((b->ntiles[1] + 7) / 8) * 8), block(ADJ_AX, ADJ_AY, 2);
     auto go = [&](auto kernel) {
         kernel<<<grid, block, 0, st>>>(b->shots, b->tile_shot + b->ntiles[0], b->ntiles[1], par, slot, b->dt, b->invdx, b->invdy,
                                        b->invdz, b->i4xy, b->i4yz, b->i4zx);

@@ -28,7 +28,7 @@ __global__ __launch_bounds__(2 * BX* FBY, 4) void k_fused_fwd( // 4 waves per SI
 }
 
 template <int SNAP, bool SPONGE>
-__global__ __launch_bounds__(ADJ_AX* ADJ_AY, ADJ_AX* ADJ_AY <= 256 ? 2 : 1) void k_fused_adj(
+__global__ __launch_bounds__(2 * ADJ_AX* ADJ_AY, 4) void k_fused_adj(
     const float* __restrict__ a1, const float* __restrict__ a2, float* __restrict__ a1o, float* __restrict__ a2o,
     float* __restrict__ u, float* __restrict__ w, const float* __restrict__ m1, const float* __restrict__ m2,
     const float* __restrict__ m3, const float* __restrict__ m4, const float* __restrict__ vrx,
@@ -226,7 +226,7 @@ tti_fused_adj_step(const float* field1, const float* field2, float* field1_out, 
     const Launch L = plan(ixbeg, ixend, iybeg, iyend, izbeg, izend, zblock, ADJ_AX, ADJ_AY, 1);
     const Snap sn = to_snap(snap);
     auto go = [&](auto kernel) {
-        kernel<<<L.grid, dim3(ADJ_AX, ADJ_AY), 0, (hipStream_t)stream>>>(
+        kernel<<<L.grid, dim3(ADJ_AX, ADJ_AY, 2), 0, (hipStream_t)stream>>>(
             field1, field2, field1_out, field2_out, field3, field4, model1, model2, model3, model4, rx, ry, rz,
             Model11, (const ab2*)ABx, (const ab2*)ABy, (const ab2*)ABz, g, dt, (float)(1.0 / dx), (float)(1.0 / dy),
             (float)(1.0 / dz), (float)(1.0 / (4 * dx * dy)), (float)(1.0 / (4 * dy * dz)),

@@ -16,11 +16,11 @@
 // (the reference writes them on the interior only and never fills their outer ghosts) and sigma ghosts hold what
 // the caller stored there.
 //
-// A block marches over a chunk of z planes with one output column per thread (adjoint, 64 x 8 threads) or per pair of
-// threads, one for each field (forward, 64 x 8 x 2). Per plane p it stages tiles with an 8-point halo in LDS, builds the
-// staggered derivatives d = b D- sigma (of the adjoint's S) of plane p on the tile plus a 4-point rim, and absorbs plane
-// p into register queues; output plane o = p - 4 is finalised with the z part coming from a per-thread column stream 7
-// planes ahead.
+// A block marches over a chunk of z planes with one output column per pair of threads, one for each field (64 x 8 x 2
+// threads). Per plane p it stages tiles with an 8-point halo in LDS, builds the staggered derivatives d = b D- sigma (of
+// the adjoint's S) of plane p on the tile plus a 4-point rim, and absorbs plane p into register queues. Forward, output
+// plane o = p - 4 is finalised with the z part coming from a per-thread column stream 7 planes ahead; the adjoint's S_z
+// comes from the tile centres and its output plane is p - 7.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
@@ -369,10 +369,10 @@ fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __re
     // u += dt (m1 H1 + m4 V1 + m2 V2), w += dt (m2 H1 + m3 V2 + m4 H2), summed in this order
     const float *const ma = F ? m2 : m1, *const mb = F ? m3 : m4, *const mc = F ? m4 : m2;
     // snapshot element offsets (32-bit: the launchers check that a snapshot field has < 2^32 elements): plane
-    // stride, this thread's column within a plane, and its 64-point segment's scale within a plane
+    // stride and this thread's column within a plane; rows are whole 64-point segments, so an element's scale is its
+    // offset / 64
     const unsigned s_plane = (unsigned)(snap.ldy * snap.ldx);
     const unsigned s_col = (unsigned)(iy - g.iybeg) * (unsigned)snap.ldx + (unsigned)(ix - g.ixbeg);
-    const unsigned s_scol = (unsigned)(iy - g.iybeg) * (unsigned)(snap.ldx / SNAP_SEG) + (unsigned)((x0 - g.ixbeg) / SNAP_SEG);
     float axy = 1.0f, bxy = 1.0f;
     if (SPONGE && active) {
         axy = fminf(abx[ix].a, aby[iy].a);
@@ -599,8 +599,7 @@ fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __re
         }
         if (SNAP != TTI_SNAP_NONE && o >= z0 && iy <= g.iyend) {
             const unsigned pz = (unsigned)(o - g.izbeg);
-            const unsigned idx = pz * s_plane + s_col;
-            const unsigned sidx = pz * (s_plane / SNAP_SEG) + s_scol;
+            const unsigned idx = pz * s_plane + s_col, sidx = idx / SNAP_SEG;
             snap_store(SNAP, F ? snap.b : snap.a, F ? snap.sb : snap.sa, idx, sidx, active, unew);
             if constexpr (SIG) // the sigma this step read (its u, w update used it)
                 snap_store(SNAP, F ? snap.d : snap.c, F ? snap.sd : snap.sc, idx, sidx, active, sq[cur]);
@@ -652,9 +651,9 @@ fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __re
 // Same pipeline as the forward kernel; the tile stage holds the pointwise temporaries S_x, S_y, M_xy, M_zx, M_yz
 // and b of plane p on a plus-shaped footprint, computed from the 10 prefetched input quads when they are stored.
 // ------------------------------------------------------------------------------------------------------------------
-struct Temps
+struct Temps // lap2 = m4 f2 (see s2_of)
 {
-    float lap1, hz1, lap2, hz2;
+    float lap1, hz1, hz2;
 };
 
 __device__ __forceinline__ Temps
@@ -664,68 +663,54 @@ temps(float f1, float f2, float mm1, float mm2, float mm3, float mm4)
     // explicit fmaf: one fixed rounding for every copy of the code (see the forward finalisation)
     t.lap1 = fmaf(mm2, f2, mm1 * f1);
     t.hz1 = fmaf(-mm2, f2, (-mm1 + mm4) * f1);
-    t.lap2 = mm4 * f2;
     t.hz2 = fmaf(-mm4 + mm3, f2, mm2 * f1);
     return t;
 }
 
-// Adjoint tile shape: AX x AY output columns per block, one per thread (AX = 64: a wave is one 64-point row;
-// AX = 32: a wave is two 32-point rows, each half-wave one contiguous LDS row). AY rows.
-#ifndef TTI_ADJ_AX
-#define TTI_ADJ_AX 64
-#endif
-#ifndef TTI_ADJ_AY
-#define TTI_ADJ_AY 8
-#endif
-constexpr int ADJ_AX = TTI_ADJ_AX, ADJ_AY = TTI_ADJ_AY;
+// S_a = rho (lap + r_a^2 hz) of either field, each with one fixed rounding (lap2 = m4 f2 is a product itself)
+__device__ __forceinline__ float
+s_of(float rho, float lap1, float r, float hz1)
+{
+    return rho * fmaf(r * r, hz1, lap1);
+}
+__device__ __forceinline__ float
+s2_of(float rho, float m4, float f2, float r, float hz2)
+{
+    return rho * fmaf(m4, f2, __fmul_rn(r * r, hz2));
+}
 
-template <int AX, int AY>
+constexpr int ADJ_AX = BX, ADJ_AY = 8; // output columns per block, a pair of threads each
+
+// Half-quads (2 consecutive x points) of the plus-shaped footprint of the adjoint tile, one per thread
+template <int AY>
 struct AdjShape
 {
-    static constexpr int NT = AX * AY;                 // threads
-    static constexpr int TW = AX + 16, TH = AY + 16;   // footprint with halo 8: (x0-8+lx, y0-8+ly)
-    static constexpr int BW = AX + 8, BH = AY + 8;     // halo-4 region
-    static constexpr int QR = TW / 4;                  // quads per footprint row
-    // quads of the plus-shaped footprint: rows [8, 8+AY) whole; rows [4, 8) and [8+AY, 12+AY) from x' = 4 (the halo-4
-    // square); the 4 outermost rows on each side from x' = 8 (the y halo of the block's own columns)
-    static constexpr int NQ = AY * QR + 8 * (QR - 2) + 8 * (QR - 4);
-    static constexpr int FXI = AY * BW, XI = (FXI + NT - 1) / NT; // d_x items and items per thread
-    static constexpr int YI = (BH + AY - 1) / AY;                  // d_y items per thread
-    static_assert(AX % 32 == 0 && AX <= 64 && NT % 64 == 0 && SNAP_SEG % AX == 0, "adjoint tile shape");
-    static_assert(NQ <= NT, "one footprint quad per thread");
+    static constexpr int NT = 2 * BX * AY;           // threads
+    static constexpr int TH = AY + 16, BH = AY + 8;  // footprint with halo 8: (x0-8+lx, y0-8+ly); halo-4 region
+    static constexpr int HR = TW / 2;                // half-quads per footprint row
+    // rows [8, 8+AY) whole; rows [4, 8) and [8+AY, 12+AY) from x' = 4 (the halo-4 square); the 4 outermost rows on each
+    // side from x' = 8 (the y halo of the block's own columns; these need S_y only)
+    static constexpr int OUTER = 8 * (HR - 8), NH = OUTER + AY * HR + 8 * (HR - 4);
+    static constexpr int YI = BH / AY; // d_y items per thread
+    static_assert(NH <= NT && BH % AY == 0, "one footprint half-quad per thread");
 };
 
-template <int AX, int AY>
-struct __align__(16) AdjTiles
-{
-    using Sh = AdjShape<AX, AY>;
-    // the two fields of each temporary interleaved: every stencil tap is one 8-byte LDS read for both (measured at
-    // 512^3: 3.87 -> 3.75 ms per step, 4.42 -> 4.31 ms with imaging; the forward's sigma tiles lost 2.5% the same way)
-    float2 SX[AY][Sh::TW];      // S_x at (x0-8+lx, y0+r)
-    float2 SY[Sh::TH][AX];      // S_y at (x0+c, y0-8+ly)
-    float2 MXY[Sh::BH][Sh::BW]; // M_xy at (x0-4+lx, y0-4+ly)
-    float2 MZX[AY][Sh::BW];     // M_zx at (x0-4+lx, y0+r)
-    float2 MYZ[Sh::BH][AX];     // M_yz at (x0+c, y0-4+ly)
-    float Bt[Sh::BH][Sh::BW];                   // b at (x0-4+lx, y0-4+ly)
-};
-
-// Footprint quad t (t < NQ) of the plus-shaped adjoint footprint: its row and x' offset, bands of rows in order
-template <int AX, int AY>
+// Footprint half-quad t (t < NH): its row and x' offset, bands of rows in order
+template <int AY>
 __device__ __forceinline__ void
-adj_quad(int t, int& row, int& lx)
+adj_half(int t, int& row, int& lx)
 {
-    using Sh = AdjShape<AX, AY>;
-    constexpr int QR = Sh::QR;
-    // (first row, rows, quads per row, first quad) of the five bands, the two outer ones (S_y only) first, so that
-    // the threads of those bands fill whole waves
+    constexpr int HR = AdjShape<AY>::HR;
+    // (first row, rows, half-quads per row, first one) of the five bands, the two outer ones first, so that the threads
+    // of those bands fill whole waves
     constexpr int rs[5] = { 0, 12 + AY, 4, 8, 8 + AY }, br[5] = { 4, 4, 4, AY, 4 };
-    constexpr int bq[5] = { QR - 4, QR - 4, QR - 2, QR, QR - 2 }, b0[5] = { 2, 2, 1, 0, 1 };
+    constexpr int bq[5] = { HR - 8, HR - 8, HR - 4, HR, HR - 4 }, b0[5] = { 4, 4, 2, 0, 2 };
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
         const int n = br[k] * bq[k];
         if (t < n) {
             row = rs[k] + t / bq[k];
-            lx = 4 * (b0[k] + t % bq[k]);
+            lx = 2 * (b0[k] + t % bq[k]);
             return;
         }
         t -= n;
@@ -734,8 +719,15 @@ adj_quad(int t, int& row, int& lx)
     lx = 0;
 }
 
-// One block's tile of an adjoint step; SNAP = snapshot mode of the imaging condition (TTI_SNAP_NONE: no imaging)
-template <int SNAP, bool SPONGE, int AX = ADJ_AX, int AY = ADJ_AY>
+// One block's tile of an adjoint step; SNAP = snapshot mode of the imaging condition (TTI_SNAP_NONE: no imaging). One
+// thread per column and field (threadIdx.z: 0 sigma_H and u, 1 sigma_V and w): VALU, LDS and the latency between them
+// bound it together (57 B/pt at the copy rate are 1.5 of 3.4 ms at 512^3), so what counts is waves to fill the gaps: one
+// thread per column held both fields' queues in 256 registers, 8 waves per CU; this holds 16. Each temporary is formed
+// once, by the thread that loaded its half-quad, for both fields. S_z comes with the tile, so no second stream of 6
+// volumes runs 7 planes ahead, at the price of 3 more recomputed planes per chunk, which form S_z alone. One barrier per
+// plane: X and Y are written before it and read after it, the tiles of the next plane go into the other buffer.
+// 512^3 3.57 -> 3.37 ms, with FP16 imaging 4.08 -> 3.78 (64-column, 8-row blocks of either kind; 64^3 38 -> 30 us).
+template <int SNAP, bool SPONGE>
 __device__ __forceinline__ void
 adj_tile(const float* __restrict__ a1, const float* __restrict__ a2, float* __restrict__ a1o, float* __restrict__ a2o,
          float* __restrict__ u, float* __restrict__ w, const float* __restrict__ m1, const float* __restrict__ m2,
@@ -745,392 +737,345 @@ adj_tile(const float* __restrict__ a1, const float* __restrict__ a2, float* __re
          float invdx, float invdy, float invdz, float i4xy, float i4yz, float i4zx, const Snap& snap,
          double* __restrict__ grad, int bz, int bxi, int byi, int bzi)
 {
-    using Sh = AdjShape<AX, AY>;
-    constexpr int NT = Sh::NT, BW = Sh::BW, BH = Sh::BH, XI = Sh::XI, YI = Sh::YI, FXI = Sh::FXI;
-    // planes per loop iteration: the z queues shift once per iteration, and the shift is a register move per live
-    // value (70 of the 520 VALU instructions per plane at 2 planes, 49 of 498 at 4). Four planes where the registers
-    // allow it (512^3: 3.575 -> 3.558 ms per step, same bits); with imaging they spill 4 VGPRs (4.06 -> 4.27 ms)
-    constexpr int AU = SNAP == TTI_SNAP_NONE ? 4 : 2;
-    __shared__ AdjTiles<AX, AY> S[2];
-    __shared__ float2 X[AY][BW]; // d_x of both fields
-    __shared__ float2 Y[BH][AX]; // d_y
+    constexpr int AY = ADJ_AY;
+    using Sh = AdjShape<AY>;
+    constexpr int NT = BX * AY, TH = Sh::TH, BH = Sh::BH; // NT: threads per field
+    constexpr int DEP = 7;  // output plane o = p - DEP
+    constexpr bool imaging = SNAP != TTI_SNAP_NONE;
+    // [parity][field] temporaries of plane p
+    __shared__ __align__(16) float SX[2][2][AY][TW];  // S_x at (x0-8+lx, y0+r)
+    __shared__ __align__(16) float SY[2][2][TH][BX];  // S_y at (x0+c, y0-8+ly)
+    __shared__ __align__(16) float MXY[2][2][BH][BW]; // M_xy at (x0-4+lx, y0-4+ly)
+    __shared__ __align__(16) float MZX[2][2][AY][BW]; // M_zx at (x0-4+lx, y0+r)
+    __shared__ __align__(16) float MYZ[2][2][BH][BX]; // M_yz at (x0+c, y0-4+ly)
+    __shared__ __align__(16) float SZ[2][2][AY][BX];  // S_z and sigma of the block's own columns
+    __shared__ __align__(16) float SA[2][2][AY][BX];
+    __shared__ __align__(16) float Bt[2][BH][BW];     // b at (x0-4+lx, y0-4+ly)
+    __shared__ float X[2][2][AY][BW];                 // d_x, d_y
+    __shared__ float Y[2][2][BH][BX];
+    __shared__ double EX[imaging ? 2 : 1][imaging ? AY : 1][imaging ? BX : 1]; // w' w_snap
 
-    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * AX + tx;
-    const int x0 = g.ixbeg + bxi * AX, y0 = g.iybeg + byi * AY, z0 = g.izbeg + bzi * bz;
+    const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y), tid = ty * BX + tx;
+    const int F = __builtin_amdgcn_readfirstlane(threadIdx.z);
+    const int x0 = g.ixbeg + bxi * BX, y0 = g.iybeg + byi * AY, z0 = g.izbeg + bzi * bz;
     const int z1 = min(z0 + bz, g.izend + 1);
     const int ix = x0 + tx, iy = y0 + ty;
     const bool active = ix <= g.ixend && iy <= g.iyend;
     const unsigned PB = (unsigned)g.ldx * (unsigned)g.ldy * 4u;
     const unsigned colb = active ? ((unsigned)iy * (unsigned)g.ldx + (unsigned)ix) * 4u : 0u;
+    float *const ao = F ? a2o : a1o, *const uw = F ? w : u;
     float axy = 1.0f, bxy = 1.0f;
     if (SPONGE && active) {
         axy = fminf(abx[ix].a, aby[iy].a);
         bxy = fminf(abx[ix].b, aby[iy].b);
     }
     // snapshot and image element offsets (32-bit: the launchers check both fit): plane strides and this thread's
-    // column within a plane; the block lies inside one 64-point segment of a snapshot row
+    // column within a plane; snapshot rows are whole 64-point segments, so an element's scale is its offset / 64
     const unsigned s_plane = (unsigned)(snap.ldy * snap.ldx);
-    const unsigned s_col = (unsigned)(iy - g.iybeg) * (unsigned)snap.ldx + (unsigned)(ix - g.ixbeg);
-    const unsigned s_scol =
-        (unsigned)(iy - g.iybeg) * (unsigned)(snap.ldx / SNAP_SEG) + (unsigned)((x0 - g.ixbeg) / SNAP_SEG);
+    const unsigned s_col = active ? (unsigned)(iy - g.iybeg) * (unsigned)snap.ldx + (unsigned)(ix - g.ixbeg) : 0u;
     const unsigned g_row = (unsigned)(g.ixend - g.ixbeg + 1);
     const unsigned g_plane = g_row * (unsigned)(g.iyend - g.iybeg + 1);
-    const unsigned g_col = (unsigned)(iy - g.iybeg) * g_row + (unsigned)(ix - g.ixbeg);
+    const unsigned g_col = active && !F ? (unsigned)(iy - g.iybeg) * g_row + (unsigned)(ix - g.ixbeg) : 0u;
 
-    // this thread's quad of the plus-shaped footprint (quads are 4-aligned in lx, as are the footprint regions);
-    // threads beyond the quad count load nothing
-    int tq_row = 0, tq_lx = 0;
-    const bool tq_need = tid < Sh::NQ;
-    // The 4 outer y rows on each side of the footprint (the first two bands, whole waves at AX = 64 and 32) need S_y
-    // only: their threads load 8 words (no rx, rz) and form nothing else (3.76 -> 3.66 ms per step at 512^3)
-    const bool sy_only = tid < 8 * (Sh::QR - 4);
-    adj_quad<AX, AY>(tq_need ? tid : 0, tq_row, tq_lx);
-    const bool row8 = tq_row >= 8 && tq_row < 8 + AY;
-    const bool col8 = tq_lx >= 8 && tq_lx < 8 + AX;
-    const bool sq4 = tq_lx >= 4 && tq_lx < 4 + BW && tq_row >= 4 && tq_row < 4 + BH;
-    const unsigned tqb = quad_off(g, x0 - 8 + tq_lx, y0 - 8 + tq_row); // clamped, see quad_off
-    float4 qa1, qa2, qm1, qm2, qm3, qm4, qrx, qry, qrz, qb;
-    auto fetch = [&](int pp) {
-        if (!tq_need)
+    // this thread's half-quad of the footprint: threads beyond the count load nothing
+    const int ht = tid + F * NT;
+    int hrow = 0, hlx = 0;
+    const bool need = ht < Sh::NH;
+    const bool sy_only = ht < Sh::OUTER;
+    adj_half<AY>(need ? ht : 0, hrow, hlx);
+    // What this thread's half-quad gives, as bits tested where they are used (kept as lane masks they filled the scalar
+    // registers): 1 S_x and M_zx rows, 2 S_y and M_yz columns, 4 M_xy and b, 8 S_y alone, 16, 32, 64 a part in planes of
+    // level 1, 2, 3
+    int role = 0;
+    if (need) {
+        const bool r8 = hrow >= 8 && hrow < 8 + AY, c8 = hlx >= 8 && hlx < 8 + BX;
+        const bool s4 = hlx >= 4 && hlx < 4 + BW && hrow >= 4 && hrow < 4 + BH;
+        role = (r8 ? 1 : 0) | (c8 ? 2 : 0) | (s4 ? 4 : 0) | (sy_only ? 8 : 0) | (r8 && c8 ? 16 : 0) |
+               (s4 && (r8 || c8) ? 32 : 0) | 64;
+    }
+    // byte offset within a plane, clamped into the allocation as quad_off does
+    const unsigned hb = ((unsigned)min(max(y0 - 8 + hrow, g.iybeg - R), g.iyend + R) * (unsigned)g.ldx +
+                         (unsigned)min(max(x0 - 8 + hlx, g.ixbeg - R), (int)g.ldx - 2)) *
+                        4u;
+    // What the planes outside [z0, z1) give: 2 M_zx, M_yz and S_z (p within 4 planes of the chunk), 1 S_z alone (the 3
+    // planes after those); 3 everything; 4 past the last one, no thread's part
+    auto level = [&](int p) { return p >= z1 + DEP ? 4 : p >= z1 + R ? 1 : p >= z0 && p < z1 ? 3 : 2; };
+    float2 qa1, qa2, qm1, qm2, qm3, qm4, qrx, qry, qrz, qb;
+    auto fetch = [&](int p) {
+        const unsigned ro = here((unsigned)role);
+        if (!(ro & (8u << level(p))))
             return;
-        const unsigned i = (unsigned)pp * PB + tqb;
-        qa1 = ldf4(a1, i);
-        qa2 = ldf4(a2, i);
-        qm1 = ldf4(m1, i);
-        qm2 = ldf4(m2, i);
-        qm3 = ldf4(m3, i);
-        qm4 = ldf4(m4, i);
-        qry = ldf4(vry, i);
-        qb = ldf4(b, i);
-        if (!sy_only) {
-            qrx = ldf4(vrx, i);
-            qrz = ldf4(vrz, i);
+        const unsigned i = (unsigned)min(p, g.izend + R) * PB + here(hb); // a clamped plane's S_z only meets a zero b
+        auto ld = [&](const float* v) {
+            return *reinterpret_cast<const float2*>(
+                __builtin_assume_aligned(reinterpret_cast<const char*>(v) + i, 8));
+        };
+        qa1 = ld(a1);
+        qa2 = ld(a2);
+        qm1 = ld(m1);
+        qm2 = ld(m2);
+        qm3 = ld(m3);
+        qm4 = ld(m4);
+        qry = ld(vry);
+        qb = ld(b);
+        if (!(ro & 8u)) {
+            qrx = ld(vrx);
+            qrz = ld(vrz);
         }
     };
-    auto commit = [&](int buf) {
-        if (!tq_need)
+    auto commit = [&](int p, int buf) {
+        const int lv = level(p);
+        const unsigned ro = here((unsigned)role);
+        if (!(ro & (8u << lv)))
             return;
-        AdjTiles<AX, AY>& t = S[buf];
-        const float* A1 = &qa1.x;
-        const float* A2 = &qa2.x;
-        const float* M1 = &qm1.x;
-        const float* M2 = &qm2.x;
-        const float* M3 = &qm3.x;
-        const float* M4 = &qm4.x;
-        const float* RX = &qrx.x;
-        const float* RY = &qry.x;
-        const float* RZ = &qrz.x;
-        const float* BB = &qb.x;
-        auto st2 = [](float2* dst, const float* a, const float* b) { // 4 points of two fields, interleaved
-            *reinterpret_cast<float4*>(dst) = make_float4(a[0], b[0], a[1], b[1]);
-            *reinterpret_cast<float4*>(dst + 2) = make_float4(a[2], b[2], a[3], b[3]);
+        const bool row8 = ro & 1u, col8 = ro & 2u, sq4 = ro & 4u;
+        const int hr = (int)here((unsigned)hrow), hl = (int)here((unsigned)hlx); // LDS places formed here, not kept
+        const Temps t0 = temps(qa1.x, qa2.x, qm1.x, qm2.x, qm3.x, qm4.x);
+        const Temps t1 = temps(qa1.y, qa2.y, qm1.y, qm2.y, qm3.y, qm4.y);
+        const float r0 = recip(qb.x), r1 = recip(qb.y);
+        auto st = [](float* dst, float e0, float e1) { *reinterpret_cast<float2*>(dst) = make_float2(e0, e1); };
+        // S of both fields for the direction cosines v, M for the pairs va, vb
+        auto S = [&](float* d1, float* d2, float2 v) {
+            st(d1, s_of(r0, t0.lap1, v.x, t0.hz1), s_of(r1, t1.lap1, v.y, t1.hz1));
+            st(d2, s2_of(r0, qm4.x, qa2.x, v.x, t0.hz2), s2_of(r1, qm4.y, qa2.y, v.y, t1.hz2));
         };
-        if (sy_only) {
-            float y1[4], y2[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const Temps tt = temps(A1[e], A2[e], M1[e], M2[e], M3[e], M4[e]);
-                const float rho = recip(BB[e]);
-                const float vy = RY[e];
-                y1[e] = rho * (tt.lap1 + vy * vy * tt.hz1);
-                y2[e] = rho * (tt.lap2 + vy * vy * tt.hz2);
-            }
-            st2(&t.SY[tq_row][tq_lx - 8], y1, y2);
+        auto M = [&](float* d1, float* d2, float2 va, float2 vb) {
+            st(d1, 2.0f * va.x * vb.x * t0.hz1, 2.0f * va.y * vb.y * t1.hz1);
+            st(d2, 2.0f * va.x * vb.x * t0.hz2, 2.0f * va.y * vb.y * t1.hz2);
+        };
+        if (lv == 3 && col8)
+            S(&SY[buf][0][hr][hl - 8], &SY[buf][1][hr][hl - 8], qry);
+        if (ro & 8u)
             return;
-        }
-        float sx1[4], sx2[4], sy1[4], sy2[4], mxy1[4], mxy2[4], mzx1[4], mzx2[4], myz1[4], myz2[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const Temps tt = temps(A1[e], A2[e], M1[e], M2[e], M3[e], M4[e]);
-            const float rho = recip(BB[e]);
-            const float vx = RX[e], vy = RY[e], vz = RZ[e];
-            sx1[e] = rho * (tt.lap1 + vx * vx * tt.hz1);
-            sx2[e] = rho * (tt.lap2 + vx * vx * tt.hz2);
-            sy1[e] = rho * (tt.lap1 + vy * vy * tt.hz1);
-            sy2[e] = rho * (tt.lap2 + vy * vy * tt.hz2);
-            mxy1[e] = 2.0f * vx * vy * tt.hz1;
-            mxy2[e] = 2.0f * vx * vy * tt.hz2;
-            mzx1[e] = 2.0f * vz * vx * tt.hz1;
-            mzx2[e] = 2.0f * vz * vx * tt.hz2;
-            myz1[e] = 2.0f * vy * vz * tt.hz1;
-            myz2[e] = 2.0f * vy * vz * tt.hz2;
-        }
-        auto st = [](float* dst, const float* v) {
-            *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-        };
-        if (row8) {
-            st2(&t.SX[tq_row - 8][tq_lx], sx1, sx2);
-        }
-        if (col8) {
-            st2(&t.SY[tq_row][tq_lx - 8], sy1, sy2);
-        }
+        if (lv == 3 && row8)
+            S(&SX[buf][0][hr - 8][hl], &SX[buf][1][hr - 8][hl], qrx);
         if (sq4) {
-            st2(&t.MXY[tq_row - 4][tq_lx - 4], mxy1, mxy2);
-            st(&t.Bt[tq_row - 4][tq_lx - 4], BB);
-            if (row8) {
-                st2(&t.MZX[tq_row - 8][tq_lx - 4], mzx1, mzx2);
+            if (lv == 3)
+                M(&MXY[buf][0][hr - 4][hl - 4], &MXY[buf][1][hr - 4][hl - 4], qrx, qry);
+            if (lv >= 2) {
+                st(&Bt[buf][hr - 4][hl - 4], qb.x, qb.y);
+                if (row8)
+                    M(&MZX[buf][0][hr - 8][hl - 4], &MZX[buf][1][hr - 8][hl - 4], qrz, qrx);
+                if (col8)
+                    M(&MYZ[buf][0][hr - 4][hl - 8], &MYZ[buf][1][hr - 4][hl - 8], qry, qrz);
             }
-            if (col8) {
-                st2(&t.MYZ[tq_row - 4][tq_lx - 8], myz1, myz2);
-            }
-        }
-    };
-    // d_x items (r, j) = item tid + i NT of the AY x BW rim rows; d_y items: rows ty + h AY of the BH band, column tx.
-    // The scale is 1/d for interior points and zero elsewhere (floats: no lane masks live across the loop).
-    int xr[XI], xj[XI];
-    float xs[XI], ys[YI];
-#pragma unroll
-    for (int i = 0; i < XI; ++i) {
-        const int it = min(tid + i * NT, FXI - 1); // items past the count repeat the last one (same value, same word)
-        xr[i] = it / BW;
-        xj[i] = it - xr[i] * BW;
-        xs[i] = in_xy(g, x0 - 4 + xj[i], y0 + xr[i]) ? invdx : 0.0f;
-    }
-#pragma unroll
-    for (int h = 0; h < YI; ++h)
-        ys[h] = ty + h * AY < BH && in_xy(g, x0 + tx, y0 - 4 + ty + h * AY) ? invdy : 0.0f;
-
-    // z queues seen through a window at slot c = o - z0 mod AU, shifted by AU every AU-th plane (as in the
-    // forward kernel)
-    float sz1[7 + AU], sz2[7 + AU];       // S_z(o + k)                       at [c + k], k = 0..7
-    float dz1[7 + AU], dz2[7 + AU];       // d_z(o - 3 + k)                   at [c + k], k = 0..7
-    // right-hand side partial sums of output o + j at [c + j], j = 0..8: the X_zx + X_yz terms of the planes
-    // o + j - 4 .. o + j + 4 and, when plane o + j itself is on the tile, its in-plane terms D+_x d_x + D+_y d_y +
-    // X_xy M_xy (no separate queue: they are summed into the same slot)
-    float q1[8 + AU], q2[8 + AU];
-#pragma unroll
-    for (int k = 0; k < 7 + AU; ++k)
-        dz1[k] = dz2[k] = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8 + AU; ++k)
-        q1[k] = q2[k] = 0.0f;
-
-    // S_z of the column at plane q, clamped into the allocation (a clamped value only meets a zero b below); the 8
-    // column words are loaded one plane before they are combined, so the loads overlap a whole plane
-    struct Col
-    {
-        float a1, a2, m1, m2, m3, m4, b, vz;
-    };
-    auto col_load = [&](int q) {
-        const unsigned i = (unsigned)min(max(q, g.izbeg - R), g.izend + R) * PB + colb;
-        return Col{ ldf(a1, i), ldf(a2, i), ldf(m1, i), ldf(m2, i), ldf(m3, i), ldf(m4, i), ldf(b, i), ldf(vrz, i) };
-    };
-    auto col_sz = [&](const Col& c, float& v1, float& v2) {
-        const Temps t = temps(c.a1, c.a2, c.m1, c.m2, c.m3, c.m4);
-        const float rho = recip(c.b);
-        v1 = rho * (t.lap1 + c.vz * c.vz * t.hz1);
-        v2 = rho * (t.lap2 + c.vz * c.vz * t.hz2);
-    };
-    // the column's sigma and b words ride along in queues of their own instead of being loaded again planes later
-    // (when L2 no longer holds them): sigma of plane o + k at [c + k] (k = 0..7, the output plane's sigma for its
-    // time update), b of plane o + 4 + k at [c + k] (k = 0..3, for d_z(o + 4)); 3.64 -> 3.57 ms per step at 512^3,
-    // 4.18 -> 4.06 ms with imaging. b is zeroed outside the interior planes where it is used, not where it is
-    // loaded: a select right after a load waits for that load and every load issued before it
-    float sa1[7 + AU], sa2[7 + AU], sb[3 + AU];
-#pragma unroll
-    for (int k = 0; k < 7; ++k) {
-        const Col c = col_load(z0 - 8 + k);
-        col_sz(c, sz1[k], sz2[k]);
-        sa1[k] = c.a1;
-        sa2[k] = c.a2;
-        if (k >= 4)
-            sb[k - 4] = c.b;
-    }
-    // prefetch registers in two sets selected by the parity of the plane (a body fills the set the next drains)
-    Col ncol[2];
-    ncol[0] = col_load(z0 - 1);
-    // pointwise words of an output plane: u w (+ snapshot u, w and the image value)
-    float pw[2][2];
-    SnapWord sw_u[2], sw_w[2];
-    double g0[2] = { 0.0, 0.0 };
-    unsigned gi[2] = { 0, 0 };
-    constexpr bool imaging = SNAP != TTI_SNAP_NONE;
-    auto fetch_point = [&](int o, int set) {
-        if (o >= z0 && o < z1) {
-            const unsigned io = (unsigned)o * PB + colb;
-            pw[set][0] = ldf(u, io);
-            pw[set][1] = ldf(w, io);
-            if (imaging && active) {
-                const unsigned pz = (unsigned)(o - g.izbeg);
-                const unsigned idx = pz * s_plane + s_col;
-                const unsigned sidx = pz * (s_plane / SNAP_SEG) + s_scol;
-                sw_u[set] = snap_fetch(SNAP, snap.a, snap.sa, idx, sidx);
-                sw_w[set] = snap_fetch(SNAP, snap.b, snap.sb, idx, sidx);
-                gi[set] = pz * g_plane + g_col;
-                g0[set] = grad[gi[set]];
+            if (row8 && col8) {
+                S(&SZ[buf][0][hr - 8][hl - 8], &SZ[buf][1][hr - 8][hl - 8], qrz);
+                if (lv == 3) {
+                    st(&SA[buf][0][hr - 8][hl - 8], qa1.x, qa1.y);
+                    st(&SA[buf][1][hr - 8][hl - 8], qa2.x, qa2.y);
+                }
             }
         }
     };
+    // d_x items: the thread's own column and the 4 rim columns on either side of each row on the first threads; d_y items:
+    // rows ty + h AY of the BH band, column tx. The scale is 1/d for interior points and zero elsewhere (floats: no lane
+    // masks live across the loop).
+    constexpr int XE = 8 * AY;
+    static_assert(XE <= NT, "one rim item per thread");
+    const int xe_r = min(tid, XE - 1) / 8, xe_k = min(tid, XE - 1) % 8, xe_j = xe_k < 4 ? xe_k : BX + xe_k;
+    const float xs = in_xy(g, ix, iy) ? invdx : 0.0f;
+    const float xes = in_xy(g, x0 - 4 + xe_j, y0 + xe_r) ? invdx : 0.0f;
+    float ys[Sh::YI];
+#pragma unroll
+    for (int h = 0; h < Sh::YI; ++h)
+        ys[h] = in_xy(g, x0 + tx, y0 - 4 + ty + h * AY) ? invdy : 0.0f;
 
+    // z queues; the delay queues are seen through a window at slot c = p - (z0 - 4) mod 2 and shift by 2 every second plane,
+    // the right-hand side sums shift as they are summed
+    float sz[9], sa[9]; // S_z and sigma of plane p - 7 + k  at [c + k], k = 0..7
+    float dz[9];        // d_z(p - 10 + k) = d_z(o - 3 + k)  at [c + k], k = 0..7
+    float sb[5];        // b(p - 3 + k)                      at [c + k], k = 0..3
+    // right-hand side sums of output p - 7 + j, j = 0..11: the X_zx + X_yz terms of the planes around it and, when plane
+    // p is the output itself, its in-plane terms D+_x d_x + D+_y d_y + X_xy M_xy
+    float q[12];
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+        sz[k] = sa[k] = dz[k] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+        sb[k] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 12; ++k)
+        q[k] = 0.0f;
+    // S_z of the 3 planes before the first tile plane, clamped into the allocation (a clamped value only meets a zero b)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const unsigned i = (unsigned)max(z0 - 7 + k, g.izbeg - R) * PB + colb;
+        const float c2 = ldf(a2, i), c4 = ldf(m4, i);
+        const Temps t = temps(ldf(a1, i), c2, ldf(m1, i), ldf(m2, i), ldf(m3, i), c4);
+        const float rho = recip(ldf(b, i)), vz = ldf(vrz, i);
+        sz[4 + k] = F ? s2_of(rho, c4, c2, vz, t.hz2) : s_of(rho, t.lap1, vz, t.hz1);
+    }
+    // pointwise words of an output plane: u or w (+ the snapshot word and, in the first field's thread, the image value)
+    float pu = 0.0f;
+    SnapWord sw{ 0u, 1.0f };
+    double g0 = 0.0;
+    // An imaging step issues these loads on every path (planes outside the block's read its nearest one): past loads that
+    // may not have been issued, the wait for a tile quad drains everything in flight, and with the extra words in registers
+    // too the loop spilled (512^3 FP16 4.17 -> 3.78 ms). Without imaging it is the branch that is faster (3.47 -> 3.37 ms).
+    auto own_plane = [&](int o) { return min(max(o, z0), z1 - 1); };
+    auto fetch_point = [&](int o) {
+        if (!imaging && (o < z0 || o >= z1))
+            return;
+        o = own_plane(o);
+        pu = ldf(uw, (unsigned)o * PB + here(colb));
+        if (imaging) {
+            const unsigned idx = (unsigned)(o - g.izbeg) * s_plane + here(s_col);
+            sw = snap_fetch(SNAP, F ? snap.b : snap.a, F ? snap.sb : snap.sa, idx, idx / SNAP_SEG);
+        }
+    };
+    auto fetch_image = [&](int o) {
+        if (imaging)
+            g0 = grad[(unsigned)(own_plane(o) - g.izbeg) * g_plane + here(g_col)];
+    };
+
+    fetch_point(z0);
+    fetch_image(z0);
     fetch(z0 - R);
-    commit(0);
+    commit(z0 - R, 0);
     fetch(z0 - R + 1);
     __syncthreads();
 
-    auto body = [&](auto curc, int o) {
-        constexpr int cur = decltype(curc)::value; // queue window
-        constexpr int par = cur & 1;               // prefetch set and tile buffer
-        const int p = o + R;
+    auto body = [&](auto curc, auto ownc, int p) {
+        constexpr int cur = decltype(curc)::value;   // queue window, tile buffer
+        constexpr bool own = decltype(ownc)::value;  // plane p is one of the block's output planes
+        const int o = p - DEP, c = p - 3;
         const float pin = (p >= g.izbeg && p <= g.izend) ? 1.0f : 0.0f;
-        col_sz(ncol[par], sz1[cur + 7], sz2[cur + 7]);
-        sa1[cur + 7] = ncol[par].a1;
-        sa2[cur + 7] = ncol[par].a2;
-        sb[cur + 3] = ncol[par].b;
-        const float bd = (o + R >= g.izbeg && o + R <= g.izend) ? sb[cur] : 0.0f;
-        const AdjTiles<AX, AY>& t = S[par];
-        // ---- A: this plane's loads before its stores (one counter tracks both): column words of plane o + 1, the
-        // temporaries of plane p + 1 into the other buffer (last read before the previous barrier), tile of p + 2
-        ncol[par ^ 1] = col_load(o + 8);
-        if (p + 1 <= z1 + R - 1)
-            commit(par ^ 1);
-        if (p + 2 <= z1 + R - 1)
-            fetch(p + 2);
-        // ---- B: d_x, d_y of plane p
-        // (the scale is zero for non-interior points: every tile value is finite)
-#pragma unroll
-        for (int i = 0; i < XI; ++i) {
-            // items past the count (last slot only) repeat the last item: same value, same word
-            if (i == 0 || tid + i * NT < FXI) {
-                const float bb = t.Bt[xr[i] + 4][xj[i]] * (xs[i] * pin);
-                float2 v[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    v[k] = t.SX[xr[i]][xj[i] + k];
-                X[xr[i]][xj[i]] = make_float2(bb * stg8([&](int k) { return v[k].x; }),
-                                              bb * stg8([&](int k) { return v[k].y; }));
-            }
-        }
-#pragma unroll
-        for (int h = 0; h < YI; ++h) {
-            const int j = ty + h * AY;
-            if (h == 0 || j < BH) {
-                const float bb = t.Bt[j][tx + 4] * (ys[h] * pin);
-                float2 v[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    v[k] = t.SY[j + k][tx];
-                Y[j][tx] = make_float2(bb * stg8([&](int k) { return v[k].x; }), bb * stg8([&](int k) { return v[k].y; }));
-            }
-        }
-        __syncthreads();
-        // ---- C: plane-p contributions
-        if (active) {
-            float gx1 = 0, gx2 = 0, gy1 = 0, gy2 = 0, hxy1 = 0, hxy2 = 0;
+        // ---- A: this plane's loads before its stores (one counter tracks both): the temporaries of plane p + 1 into the
+        // other buffer (last read before the previous plane's barrier), tile of plane p + 2
+        if (p + 1 < z1 + DEP)
+            commit(p + 1, cur ^ 1);
+        fetch(p + 2);
+        // ---- B: X_yz + X_zx of plane p into the sums; from the block's output planes also X_xy, d_x and d_y
+        sz[cur + 7] = SZ[cur][F][ty][tx];
+        sb[cur + 3] = Bt[cur][ty + 4][tx + 4];
+        {
+            float d[R + 1];
 #pragma unroll
             for (int n = 1; n <= R; ++n) {
-                const float c = cstg(n);
-                const float2 xp = X[ty][tx + 4 + n], xm = X[ty][tx + 5 - n];
-                const float2 yp = Y[ty + 4 + n][tx], ym = Y[ty + 5 - n][tx];
-                gx1 += c * (xp.x - xm.x);
-                gx2 += c * (xp.y - xm.y);
-                gy1 += c * (yp.x - ym.x);
-                gy2 += c * (yp.y - ym.y);
-                const float e = ecen(n);
-                const float2 pp = t.MXY[ty + 4 + n][tx + 4 + n], pm = t.MXY[ty + 4 + n][tx + 4 - n];
-                const float2 mm = t.MXY[ty + 4 - n][tx + 4 - n], mp = t.MXY[ty + 4 - n][tx + 4 + n];
-                hxy1 += e * (pp.x - pm.x + mm.x - mp.x);
-                hxy2 += e * (pp.y - pm.y + mm.y - mp.y);
-                const float2 yzp = t.MYZ[ty + 4 + n][tx], yzm = t.MYZ[ty + 4 - n][tx];
-                const float2 zxp = t.MZX[ty][tx + 4 + n], zxm = t.MZX[ty][tx + 4 - n];
-                const float d1 = fmaf(i4yz, yzp.x - yzm.x, i4zx * (zxp.x - zxm.x));
-                const float d2 = fmaf(i4yz, yzp.y - yzm.y, i4zx * (zxp.y - zxm.y));
-                q1[cur + 4 - n] += e * d1;
-                q1[cur + 4 + n] -= e * d1;
-                q2[cur + 4 - n] += e * d2;
-                q2[cur + 4 + n] -= e * d2;
+                d[n] = fmaf(i4yz, MYZ[cur][F][ty + 4 + n][tx] - MYZ[cur][F][ty + 4 - n][tx],
+                            i4zx * (MZX[cur][F][ty][tx + 4 + n] - MZX[cur][F][ty][tx + 4 - n]));
+                hold(d[n]);
             }
-            // in-plane terms of output p (slot c + 4); explicit roundings: no product is fused into these sums
-            q1[cur + 4] = __fadd_rn(q1[cur + 4], __fadd_rn(__fadd_rn(__fmul_rn(gx1, invdx), __fmul_rn(gy1, invdy)),
-                                                           __fmul_rn(hxy1, i4xy)));
-            q2[cur + 4] = __fadd_rn(q2[cur + 4], __fadd_rn(__fadd_rn(__fmul_rn(gx2, invdx), __fmul_rn(gy2, invdy)),
-                                                           __fmul_rn(hxy2, i4xy)));
+            // plane p at offset +n feeds output p - n (slot 7 - n), at -n output p + n (slot 7 + n), sign flipped
+#pragma unroll
+            for (int j = 0; j < 11; ++j) {
+                const int n = j < 7 ? 7 - j : j - 7;
+                q[j] = n >= 1 && n <= R ? fma3(j < 7 ? ecen(n) : -ecen(n), d[n], q[j + 1]) : q[j + 1];
+                hold(q[j]);
+            }
+            q[11] = -ecen(R) * d[R];
+            hold(q[11]);
         }
-        // ---- D: d_z(o+4), finalise plane o
-        {
-            const float dzs = bd * invdz;
-            dz1[cur + 7] = dzs * stg8([&](int k) { return sz1[cur + k]; });
-            dz2[cur + 7] = dzs * stg8([&](int k) { return sz2[cur + k]; });
-            if (g.fs && o == g.izbeg) {
-                mirror_dz<cur>(dz1);
-                mirror_dz<cur>(dz2);
+        float hxy = 0.0f;
+        if constexpr (own) {
+            sa[cur + 7] = SA[cur][F][ty][tx];
+#pragma unroll
+            for (int n = 1; n <= R; ++n) {
+                hxy += ecen(n) * (MXY[cur][F][ty + 4 + n][tx + 4 + n] - MXY[cur][F][ty + 4 + n][tx + 4 - n] +
+                                  MXY[cur][F][ty + 4 - n][tx + 4 - n] - MXY[cur][F][ty + 4 - n][tx + 4 + n]);
+                hold(hxy);
+            }
+            // (the scale is zero for non-interior points: every tile value is finite)
+            float v = Bt[cur][ty + 4][tx + 4] * (xs * pin) * stg8([&](int k) { return SX[cur][F][ty][tx + 4 + k]; });
+            hold(v);
+            X[cur][F][ty][tx + 4] = v;
+            if (tid < XE) {
+                v = Bt[cur][xe_r + 4][xe_j] * (xes * pin) * stg8([&](int k) { return SX[cur][F][xe_r][xe_j + k]; });
+                hold(v);
+                X[cur][F][xe_r][xe_j] = v;
+            }
+#pragma unroll
+            for (int h = 0; h < Sh::YI; ++h) {
+                const int j = ty + h * AY;
+                v = Bt[cur][j][tx + 4] * (ys[h] * pin) * stg8([&](int k) { return SY[cur][F][j + k][tx]; });
+                hold(v);
+                Y[cur][F][j][tx] = v;
             }
         }
+        // ---- C: d_z(p - 3), then plane o = p - 7
+        dz[cur + 7] = ((c >= g.izbeg && c <= g.izend) ? sb[cur] : 0.0f) * invdz * stg8([&](int k) { return sz[cur + k]; });
+        if (g.fs && o == g.izbeg)
+            mirror_dz<cur>(dz);
         const bool fin = o >= z0 && active;
-        float un = 0.0f, wn = 0.0f, a1n = 0.0f, a2n = 0.0f;
-        double gn = 0.0;
-        const unsigned gis = gi[par];
-        const float uo = pw[par][0], wo = pw[par][1], ao1 = sa1[cur], ao2 = sa2[cur];
-        if (fin) {
-            const float gz1 = stg8([&](int k) { return dz1[cur + k]; });
-            const float gz2 = stg8([&](int k) { return dz2[cur + k]; });
-            // fixed rounding whichever products the compiler can see (see the forward finalisation)
-            const float r3 = fmaf(gz1, invdz, q1[cur]);
-            const float r4 = fmaf(gz2, invdz, q2[cur]);
-            float a = 1.0f, bb = 1.0f;
-            if constexpr (SPONGE) {
-                a = fminf(axy, abz[o].a);
-                bb = fminf(bxy, abz[o].b);
-            }
-            un = SPONGE ? fmaf(bb * dt, r3, a * uo) : fmaf(r3, dt, uo);
-            wn = SPONGE ? fmaf(bb * dt, r4, a * wo) : fmaf(r4, dt, wo);
-            a1n = fmaf(bb * un, dt, a * ao1);
-            a2n = fmaf(bb * wn, dt, a * ao2);
-            if (imaging) {
-                const float su = snap_decode(SNAP, sw_u[par]), sw = snap_decode(SNAP, sw_w[par]);
-                gn = g0[par] + fma((double)wn, (double)sw, (double)un * (double)su);
-            }
+        const float gz = stg8([&](int k) { return dz[cur + k]; });
+        // fixed rounding whichever products the compiler can see (see the forward finalisation)
+        const float r = fmaf(gz, invdz, q[0]);
+        float a = 1.0f, bb = 1.0f;
+        if constexpr (SPONGE) {
+            const ab2 z = abz[own_plane(o)];
+            a = fminf(axy, z.a);
+            bb = fminf(bxy, z.b);
         }
-        // pointwise words of plane o + 1 (their registers are free now), then the stores of plane o
-        fetch_point(o + 1, par ^ 1);
-        if (fin) {
-            const unsigned io = (unsigned)o * PB + colb;
-            stf(u, io, un);
-            stf(w, io, wn);
-            stf(a1o, io, a1n);
-            stf(a2o, io, a2n);
-            if (imaging)
-                grad[gis] = gn;
+        const float un = SPONGE ? fmaf(bb * dt, r, a * pu) : fmaf(r, dt, pu);
+        const float an = fmaf(bb * un, dt, a * sa[cur]);
+        double prod = 0.0;
+        if (imaging) {
+            prod = (double)un * (double)snap_decode(SNAP, sw); // exact
+            if (F)
+                EX[cur][ty][tx] = prod;
         }
-        // ---- E: barrier (the tile buffer and X/Y are rewritten by the next plane)
+        // the pointwise words of plane o + 1 (their registers are free now), then the stores of plane o
+        fetch_point(o + 1);
+        if (fin) {
+            const unsigned io = (unsigned)o * PB + here(colb);
+            stf(uw, io, un);
+            stf(ao, io, an);
+        }
+        // the one barrier of the plane: d_x, d_y (and w' w_snap) are complete, every read of tile buffer `cur` is done
         __syncthreads();
-        if (cur == AU - 1) {
+        // ---- D: in-plane terms of output p; the image of plane o
+        if constexpr (own) {
+            float gx = 0, gy = 0;
+#pragma unroll
+            for (int n = 1; n <= R; ++n) {
+                const float cc = cstg(n);
+                gx += cc * (X[cur][F][ty][tx + 4 + n] - X[cur][F][ty][tx + 5 - n]);
+                gy += cc * (Y[cur][F][ty + 4 + n][tx] - Y[cur][F][ty + 5 - n][tx]);
+                hold(gx), hold(gy);
+            }
+            // explicit roundings: no product is fused into these sums
+            q[7] = __fadd_rn(q[7], __fadd_rn(__fadd_rn(__fmul_rn(gx, invdx), __fmul_rn(gy, invdy)), __fmul_rn(hxy, i4xy)));
+            hold(q[7]);
+        }
+        if (imaging) {
+            const double gn = g0 + (prod + EX[cur][ty][tx]);
+            fetch_image(o + 1);
+            if (fin && !F)
+                grad[(unsigned)(o - g.izbeg) * g_plane + here(g_col)] = gn;
+        }
+        if (cur == 1) {
 #pragma unroll
             for (int k = 0; k < 7; ++k) {
-                sz1[k] = sz1[k + AU];
-                sz2[k] = sz2[k + AU];
-                dz1[k] = dz1[k + AU];
-                dz2[k] = dz2[k + AU];
-                sa1[k] = sa1[k + AU];
-                sa2[k] = sa2[k + AU];
+                sz[k] = sz[k + 2];
+                sa[k] = sa[k + 2];
+                dz[k] = dz[k + 2];
             }
 #pragma unroll
             for (int k = 0; k < 3; ++k)
-                sb[k] = sb[k + AU];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                q1[k] = q1[k + AU];
-                q2[k] = q2[k + AU];
-            }
-#pragma unroll
-            for (int k = 8; k < 8 + AU; ++k)
-                q1[k] = q2[k] = 0.0f;
+                sb[k] = sb[k + 2];
         }
     };
 
-    for (int o = z0 - 8; o < z1; o += AU) {
-        body(std::integral_constant<int, 0>{}, o);
-        if (o + 1 >= z1)
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, 1>;
+    // planes that only feed the z stencils of the block's outputs: 4 before them and 7 after
+    auto rim = [&](int p, int end) {
+        for (; p < end; ++p)
+            if (((p - z0) & 1) == 0)
+                body(C0{}, std::false_type{}, p);
+            else
+                body(C1{}, std::false_type{}, p);
+    };
+    rim(z0 - R, z0);
+    for (int p = z0; p < z1; p += 2) {
+        body(C0{}, std::true_type{}, p);
+        if (p + 1 >= z1)
             break;
-        body(std::integral_constant<int, 1>{}, o + 1);
-        if constexpr (AU == 4) {
-            if (o + 2 >= z1)
-                break;
-            body(std::integral_constant<int, 2>{}, o + 2);
-            if (o + 3 >= z1)
-                break;
-            body(std::integral_constant<int, 3>{}, o + 3);
-        }
+        body(C1{}, std::true_type{}, p + 1);
     }
+    rim(z1, z1 + DEP);
 }
 
 
@@ -1181,7 +1126,7 @@ inject_point(float* __restrict__ u, float* __restrict__ w, float* __restrict__ a
 // Host-side argument checks shared by the launchers
 // ------------------------------------------------------------------------------------------------------------------
 
-// Resident blocks on the whole GPU (one 1024-thread forward or 512-thread adjoint block per CU, by their registers) and
+// Resident blocks on the whole GPU (one 1024-thread block per CU, by their registers) and
 // the cost of a chunk's 8 recomputed planes and prologue, for chunk_depth; [0] forward, [1] adjoint.
 // Measured over z depths of 2 to 256 planes on volumes of 40^3 to 400^3, a step takes 2.43 us (forward, two blocks per
 // CU; 2.05 us one) and 3.2 us (adjoint) per plane and round within 8%. Against 128-plane chunks throughout: 64^3 149 ->
