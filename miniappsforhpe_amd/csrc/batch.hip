@@ -66,16 +66,28 @@ batch_tile(const ShotDev* __restrict__ shots, const int* __restrict__ tile_shot,
     return S;
 }
 
+// A pointer read from a shot descriptor as one to global memory: the compiler only knows that of kernel arguments, and a
+// flat access counts as an LDS access too, so every wait for a tile value waited for the volumes' loads in flight. Six
+// shots of 96 to 189 points a side, per step: 0.69 -> 0.44 ms forward and 0.87 -> 0.64 ms
+// adjoint, with the FP16 snapshot 0.79 -> 0.51 and 1.15 -> 0.72 (the box is copied for the same kind of reason: read
+// through the descriptor it is read again after every store).
+template <class T>
+__device__ __forceinline__ T*
+glob(T* const& field)
+{
+    using G = __attribute__((address_space(1))) T*;
+    return (T*)*reinterpret_cast<const G*>(&field);
+}
+
 __device__ __forceinline__ Snap
 slot_snap(const ShotDev& S, int slot)
 {
     Snap s = S.snap;
-    s.a = static_cast<char*>(s.a) + (long)slot * S.slot_bytes;
-    s.b = static_cast<char*>(s.b) + (long)slot * S.slot_bytes;
-    if (s.sa != nullptr) {
-        s.sa += (long)slot * S.scale_slot;
-        s.sb += (long)slot * S.scale_slot;
-    }
+    s.a = glob((char* const&)S.snap.a) + (long)slot * S.slot_bytes;
+    s.b = glob((char* const&)S.snap.b) + (long)slot * S.slot_bytes;
+    const long scales = s.sa != nullptr ? (long)slot * S.scale_slot : 0;
+    s.sa = glob(S.snap.sa) + scales;
+    s.sb = glob(S.snap.sb) + scales;
     return s;
 }
 
@@ -91,11 +103,13 @@ __global__ __launch_bounds__(2 * BX* FWD_BY, 4) void k_fused_fwd_batch(const Sho
     if (S == nullptr)
         return;
     const Snap sn = SNAP != TTI_SNAP_NONE ? slot_snap(*S, slot) : S->snap;
-    const float sv = S->src_amp != nullptr ? S->src_amp[it] : 0.0f;
-    fwd_tile<FWD_BY, SNAP, SPONGE>(S->s1[par], S->s2[par], S->s1[par ^ 1], S->s2[par ^ 1], S->u, S->w, S->m[0], S->m[1],
-                                   S->m[2], S->m[3], S->m[4], S->m[5], S->m[6], S->m[7], S->ab[0], S->ab[1], S->ab[2],
-                                   S->g, dt, invdx, invdy, invdz, i4xy, i4yz, i4zx, S->src_off, sv, sn, S->bz[0], bxi,
-                                   byi, bzi);
+    const float sv = S->src_amp != nullptr ? glob(S->src_amp)[it] : 0.0f;
+    const Box g = S->g;
+    fwd_tile<FWD_BY, SNAP, SPONGE>(glob(S->s1[par]), glob(S->s2[par]), glob(S->s1[par ^ 1]), glob(S->s2[par ^ 1]),
+                                   glob(S->u), glob(S->w), glob(S->m[0]), glob(S->m[1]), glob(S->m[2]), glob(S->m[3]),
+                                   glob(S->m[4]), glob(S->m[5]), glob(S->m[6]), glob(S->m[7]), glob(S->ab[0]),
+                                   glob(S->ab[1]), glob(S->ab[2]), g, dt, invdx, invdy, invdz, i4xy, i4yz, i4zx,
+                                   S->src_off, sv, sn, S->bz[0], bxi, byi, bzi);
 }
 
 template <int SNAP, bool SPONGE>
@@ -109,10 +123,11 @@ __global__ __launch_bounds__(2 * ADJ_AX* ADJ_AY, 4) void k_fused_adj_batch(const
     if (S == nullptr)
         return;
     const Snap sn = SNAP != TTI_SNAP_NONE ? slot_snap(*S, slot) : S->snap;
-    adj_tile<SNAP, SPONGE>(S->s1[par], S->s2[par], S->s1[par ^ 1], S->s2[par ^ 1], S->u, S->w, S->m[0], S->m[1],
-                           S->m[2], S->m[3], S->m[4], S->m[5], S->m[6], S->m[7], S->ab[0], S->ab[1], S->ab[2], S->g, dt,
-                           invdx, invdy, invdz, i4xy, i4yz, i4zx, sn, S->grad, S->bz[1], bxi, byi,
-                           bzi);
+    const Box g = S->g;
+    adj_tile<SNAP, SPONGE>(glob(S->s1[par]), glob(S->s2[par]), glob(S->s1[par ^ 1]), glob(S->s2[par ^ 1]), glob(S->u),
+                           glob(S->w), glob(S->m[0]), glob(S->m[1]), glob(S->m[2]), glob(S->m[3]), glob(S->m[4]),
+                           glob(S->m[5]), glob(S->m[6]), glob(S->m[7]), glob(S->ab[0]), glob(S->ab[1]), glob(S->ab[2]),
+                           g, dt, invdx, invdy, invdz, i4xy, i4yz, i4zx, sn, glob(S->grad), S->bz[1], bxi, byi, bzi);
 }
 
 // receivers of every shot (blockIdx.y = shot) after forward step `it`: sigma is the buffer the step wrote
@@ -324,13 +339,14 @@ shot_chunk(const tti_shot& q, const Box& g, int depth)
 
 // The chunk depth of a pass over all shots: chunk_depth's weighing of idle CUs against recomputed planes, for blocks of
 // uneven length. The launch is replayed block by block: each XCD takes its eighth of the tile list in order, a block
-// starts when one of the XCD's resident blocks ends, the last one gives the time. Six shots of 96 to 189 points a side
-// take 0.69 ms forward and 0.79 ms adjoint per step at 24 planes, 1.04 and 1.19 ms at 128. Long lists (over 16 rounds)
-// are priced without the replay: their ends weigh little (24 shots: 9.06 ms at 48 planes, 9.16 ms at 128).
+// starts when one of the XCD's resident blocks ends, the last one gives the time. Six shots of 96 to 189 points a side,
+// 24 steps and their adjoint: 27.1 ms at the 48 planes it chooses, 27.9 at 24, 30.2 at 32, 32.6 at 128. Long lists (over
+// 16 rounds) are priced without the replay: their ends weigh little.
 int
 batch_depth(const tti_shot* shots, const std::vector<ShotDev>& h, int pss)
 {
     const int slots = STEP_SLOTS[pss], per_xcd = slots / 8;
+    const float warm = STEP_WARM[pss];
     int best = 0;
     double cost = 0.0;
     for (int depth : { 256, 192, 128, 96, 80, 64, 56, 48, 40, 32, 28, 24, 20, 16, 12, 10, 8, 6, 4, 3, 2 }) {
@@ -340,9 +356,11 @@ batch_depth(const tti_shot* shots, const std::vector<ShotDev>& h, int pss)
             const int bz = shot_chunk(shots[s], h[s].g, depth);
             const long k = (long)h[s].ntx[pss] * h[s].nty[pss] * ((planes(h[s].g) + bz - 1) / bz);
             n += k;
-            work += (double)k * (bz + STEP_WARM);
-            longest = std::max(longest, (double)bz + STEP_WARM);
+            work += (double)k * (bz + warm);
+            longest = std::max(longest, (double)bz + warm);
         }
+        if (best != 0 && work / slots >= 0.97 * cost)
+            continue; // its recomputed planes alone cost more
         double t = work / slots + 0.5 * longest;
         if (n <= 16L * slots) {
             const long per = (n + 7) / 8;
@@ -360,8 +378,8 @@ batch_depth(const tti_shot* shots, const std::vector<ShotDev>& h, int pss)
                         start = busy.top();
                         busy.pop();
                     }
-                    busy.push(start + (float)bz + STEP_WARM);
-                    end = std::max(end, start + (float)bz + STEP_WARM);
+                    busy.push(start + (float)bz + warm);
+                    end = std::max(end, start + (float)bz + warm);
                 }
             }
             t = end;

@@ -57,7 +57,7 @@ constexpr int CUS = 256; // compute units of one MI355X
 // marching 72 planes at 2 us) and a round that is barely begun costs a whole one; many shallow ones recompute halos.
 // Returns the depth of the cheapest number of chunks, none deeper than `cap`; a shallower one has to gain 3% over the
 // best so far, because deeper chunks also read less. A last round of at most one block per CU runs its planes faster
-// (2.05 us against 2.43 us with two blocks per CU in the fused forward kernel).
+// (2.05 us against 2.43 us with two 512-thread blocks per CU of a fused forward kernel).
 inline int
 chunk_depth(int nz, long tiles, int slots, float warm, int cap)
 {

@@ -127,7 +127,7 @@ plan(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, int zbloc
     const int nx = ixend - ixbeg + 1, ny = iyend - iybeg + 1, nz = izend - izbeg + 1;
     L.ntx = (nx + bx - 1) / bx;
     L.nty = (ny + by - 1) / by;
-    L.bz = chunk_depth(nz, (long)L.ntx * L.nty, STEP_SLOTS[pass], STEP_WARM, zblock > 0 ? zblock : 128);
+    L.bz = chunk_depth(nz, (long)L.ntx * L.nty, STEP_SLOTS[pass], STEP_WARM[pass], zblock > 0 ? zblock : 128);
     L.ntz = (nz + L.bz - 1) / L.bz;
     const int nt = L.ntx * L.nty * L.ntz;
     L.grid = dim3(((nt + 7) / 8) * 8); // multiple of 8 so the XCD round-robin decode covers every tile

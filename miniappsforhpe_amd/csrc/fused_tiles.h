@@ -1126,12 +1126,13 @@ inject_point(float* __restrict__ u, float* __restrict__ w, float* __restrict__ a
 // ------------------------------------------------------------------------------------------------------------------
 
 // Resident blocks on the whole GPU (one 1024-thread block per CU, by their registers) and
-// the cost of a chunk's 8 recomputed planes and prologue, for chunk_depth; [0] forward, [1] adjoint.
-// Measured over z depths of 2 to 256 planes on volumes of 40^3 to 400^3, a step takes 2.43 us (forward, two blocks per
-// CU; 2.05 us one) and 3.2 us (adjoint) per plane and round within 8%. Against 128-plane chunks throughout: 64^3 149 ->
-// 27 us forward and 193 -> 38 us adjoint, 128^3 281 -> 58 and 359 -> 75 us.
+// the cost, in planes, of a chunk's recomputed rim planes (8 and 11) and prologue, for chunk_depth; [0] forward, [1]
+// adjoint. Fitted over z depths of 1 to 256 planes on volumes of 40^3 to 400^3: a plane takes 1.82 and 2.06 us where few
+// blocks run (64^3: 17.0 us forward at 2 planes, 129.7 at 64; 29.5 and 157.5 adjoint) and 2.3 and 3.1 us on a full GPU,
+// and no fixed depth of the sweep beats the chosen one by more than 2% from 96 points a side up. 128-plane chunks
+// throughout: 64^3 130 and 158 us against 17 and 30, 128^3 253 and 304 against 46 and 63.
 constexpr int STEP_SLOTS[2] = { CUS, CUS };
-constexpr float STEP_WARM = 9.5f;
+constexpr float STEP_WARM[2] = { 7.5f, 12.5f };
 
 // The fused kernels stage tiles with 16-byte loads: the interior must start on a 4-float boundary, rows must be a
 // multiple of 4 floats and every volume 16-byte aligned.
