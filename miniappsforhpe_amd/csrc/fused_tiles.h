@@ -741,6 +741,9 @@ adj_tile(const float* __restrict__ a1, const float* __restrict__ a2, float* __re
     constexpr int NT = BX * AY, TH = Sh::TH, BH = Sh::BH; // NT: threads per field
     constexpr int DEP = 7;  // output plane o = p - DEP
     constexpr bool imaging = SNAP != TTI_SNAP_NONE;
+    // The FP16 image (word and scale) with a sponge is the one form that does not fit 128 VGPRs: it spilled 7 and took 4.34
+    // ms at 512^3, with the columns' x-y sponge values read back from LDS 3.78 ms. The other forms keep them in registers.
+    constexpr bool tapers = SPONGE && SNAP == TTI_SNAP_FP16;
     // [parity][field] temporaries of plane p
     __shared__ __align__(16) float SX[2][2][AY][TW];  // S_x at (x0-8+lx, y0+r)
     __shared__ __align__(16) float SY[2][2][TH][BX];  // S_y at (x0+c, y0-8+ly)
@@ -753,6 +756,7 @@ adj_tile(const float* __restrict__ a1, const float* __restrict__ a2, float* __re
     __shared__ float X[2][2][AY][BW];                 // d_x, d_y
     __shared__ float Y[2][2][BH][BX];
     __shared__ double EX[imaging ? 2 : 1][imaging ? AY : 1][imaging ? BX : 1]; // w' w_snap
+    __shared__ float2 AB[tapers ? AY : 1][tapers ? BX : 1];                    // x-y sponge values of the columns
 
     const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y), tid = ty * BX + tx;
     const int F = __builtin_amdgcn_readfirstlane(threadIdx.z);
@@ -768,6 +772,8 @@ adj_tile(const float* __restrict__ a1, const float* __restrict__ a2, float* __re
         axy = fminf(abx[ix].a, aby[iy].a);
         bxy = fminf(abx[ix].b, aby[iy].b);
     }
+    if (tapers && !F)
+        AB[ty][tx] = make_float2(axy, bxy); // read past the prologue's barrier
     // snapshot and image element offsets (32-bit: the launchers check both fit): plane strides and this thread's
     // column within a plane; snapshot rows are whole 64-point segments, so an element's scale is its offset / 64
     const unsigned s_plane = (unsigned)(snap.ldy * snap.ldx);
@@ -1004,8 +1010,9 @@ adj_tile(const float* __restrict__ a1, const float* __restrict__ a2, float* __re
         float a = 1.0f, bb = 1.0f;
         if constexpr (SPONGE) {
             const ab2 z = abz[own_plane(o)];
-            a = fminf(axy, z.a);
-            bb = fminf(bxy, z.b);
+            const float2 xy = tapers ? AB[ty][tx] : make_float2(axy, bxy);
+            a = fminf(xy.x, z.a);
+            bb = fminf(xy.y, z.b);
         }
         const float un = SPONGE ? fmaf(bb * dt, r, a * pu) : fmaf(r, dt, pu);
         const float an = fmaf(bb * un, dt, a * sa[cur]);

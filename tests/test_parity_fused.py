@@ -229,6 +229,32 @@ def test_fused_imaging_condition(mode, rng, cuda):
     assert rel_l2(grad.cpu().numpy(), ref) < 1e-6
 
 
+@pytest.mark.parametrize("mode", [1, 2, 3])
+def test_fused_imaging_with_sponge_vs_oracle(mode, rng, cuda):
+    """An imaging adjoint step with absorbing sides (the FP16 form keeps the sponge values in LDS): state against the
+    oracle's step, image against the decoded snapshot."""
+    from miniappsforhpe_amd.propagator import SnapshotStore
+
+    G, OG, m, sp, P = setup((70, 19, 67), rng, cuda, sponge=True)
+    store = SnapshotStore(G, mode, 1, cuda)
+    a = [interior_random(G, rng) for _ in range(4)]
+    for dst, src in zip((*P.sigma, P.u, P.w), a):
+        dst.copy_(to_gpu(src, cuda))
+    P.prime()
+    P.step_fwd_fused(snap=store.desc(0))
+    du, dw = from_gpu(store.decode(0, 3)), from_gpu(store.decode(0, 4))
+    P.reset()
+    for dst, src in zip((*P.sigma, P.u, P.w), a):
+        dst.copy_(to_gpu(src, cuda))
+    grad = torch.zeros((G.nz, G.ny, G.nx), dtype=torch.float64, device=cuda)
+    P.step_adj_fused(snap=store.desc(0), grad=grad)
+    O.step_adj(OG, *a, m, [OG.zeros() for _ in range(8)], sp, O.f32(4e-4), DX, DY, DZ, sponge_active=True)
+    for got, ref in zip((*P.sigma, P.u, P.w), a):
+        assert rel_l2(from_gpu(got), ref) < 2e-5
+    ua, wa = from_gpu(G.interior(P.u)), from_gpu(G.interior(P.w))
+    assert rel_l2(grad.cpu().numpy(), ua * du + wa * dw) < 1e-6
+
+
 @pytest.mark.parametrize("mode", [2, 3])
 def test_snapshot_encoding_is_exact(mode, rng, cuda):
     """The snapshot written by the fused forward equals, bit for bit, the host encoding of the step's u and w: FP16
