@@ -55,12 +55,14 @@ constexpr int CUS = 256; // compute units of one MI355X
 // its planes plus `warm` (its prologue and the halo planes it recomputes, in planes), and the grid runs in rounds of
 // `slots` resident blocks, so few deep blocks leave CUs idle (a 64^3 volume in chunks of 128 planes is 16 blocks, each
 // marching 72 planes at 2 us) and a round that is barely begun costs a whole one; many shallow ones recompute halos.
-// Returns the depth of the cheapest number of chunks, none deeper than `cap`; a shallower one has to gain 3% over the
-// best so far, because deeper chunks also read less. A last round of at most one block per CU runs its planes faster
+// Returns the depth of the cheapest number of chunks, none deeper than `cap` (any value: the fused steps pass a caller's
+// zblock, which may be the largest int for "no limit"); a shallower one has to gain 3% over the best so far, because
+// deeper chunks also read less. A last round of at most one block per CU runs its planes faster
 // (2.05 us against 2.43 us with two 512-thread blocks per CU of a fused forward kernel).
 inline int
 chunk_depth(int nz, long tiles, int slots, float warm, int cap)
 {
+    cap = cap < 1 ? 1 : cap > nz ? nz : cap;
     int best = 0;
     float cost = 0.0f;
     for (int c = (nz + cap - 1) / cap;;) {

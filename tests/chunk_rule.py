@@ -1,0 +1,67 @@
+"""The z chunks that the launchers choose, from the rule itself: csrc/common.h chunk_depth and the constants of the fused
+steps compiled for the host, and the Chunk constants as the kernel sources state them. Tests use it to take shapes whose
+chunks are known and to say so."""
+import functools
+import re
+import subprocess
+import tempfile
+from pathlib import Path
+
+import pytest
+
+from miniappsforhpe_amd import build as B
+
+SRC = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "fused_tiles.h"
+using namespace tti;
+using namespace tti::fused;
+int main(int, char** v)
+{
+    const int nz = atoi(v[2]), cap = atoi(v[6]), pass = atoi(v[1]);
+    const long tiles = atol(v[3]);
+    printf("%d\n", pass < 0 ? chunk_depth(nz, tiles, atoi(v[4]), (float)atof(v[5]), cap)
+                            : chunk_depth(nz, tiles, STEP_SLOTS[pass], STEP_WARM[pass], cap));
+}
+"""
+
+
+@functools.lru_cache(maxsize=None)
+def _program():
+    if not Path(B.HIPCC).exists():
+        pytest.skip("no hipcc")
+    d = Path(tempfile.mkdtemp(prefix="chunk_rule"))
+    (d / "c.hip").write_text(SRC)
+    subprocess.run([B.HIPCC, *B.HIP_FLAGS, "--offload-host-only", str(d / "c.hip"), "-o", str(d / "c")], check=True,
+                   capture_output=True)
+    return str(d / "c")
+
+
+@functools.lru_cache(maxsize=None)
+def depth(nz, tiles, slots, warm, cap, fused_pass=-1):
+    args = [str(a) for a in (fused_pass, nz, tiles, slots, warm, cap)]
+    return int(subprocess.run([_program(), *args], check=True, capture_output=True, text=True).stdout)
+
+
+def tiles(shape, rows):
+    return -(-shape[0] // 64) * -(-shape[1] // rows)
+
+
+def fused_depth(shape, fused_pass, zblock):
+    """Planes per block of the fused forward (0) or adjoint (1) step; tiles of 64 x 8 columns."""
+    return depth(shape[2], tiles(shape, 8), 0, 0, zblock, fused_pass)
+
+
+@functools.lru_cache(maxsize=None)
+def chunks():
+    """{name: (blocks per CU, warm, cap)} of every Chunk constant in the kernel sources."""
+    text = "".join((B.CSRC / f"{n}_kernels.hip").read_text() for n in ("type2", "type1", "etti"))
+    found = re.findall(r"(\w+_CHUNK)\{ (\d+), ([\d.]+)f(?:, (\d+))? \}", text)
+    return {n: (int(k), float(w), int(c or 256)) for n, k, w, c in found}
+
+
+def stencil_depth(shape, name, rows):
+    """Planes per block of the kernel with Chunk constant `name` and tiles of 64 x rows columns."""
+    per_cu, warm, cap = chunks()[name]
+    return depth(shape[2], tiles(shape, rows), per_cu * 256, warm, cap)

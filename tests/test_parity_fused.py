@@ -356,6 +356,23 @@ def test_chunk_depth_keeps_results(shape, caps, rng, cuda):
             assert torch.equal(a, b), zb
 
 
+def test_zblock_without_limit(rng, cuda):
+    """zblock is the most planes a block may hold: the largest int is no limit, with the bits of any other value."""
+    G, OG, m, sp, P = setup((70, 19, 67), rng, cuda)
+    init = [to_gpu(interior_random(G, rng), cuda) for _ in range(4)]
+    got = []
+    for zb in (64, 2**31 - 1):
+        P.reset()
+        P.zblock = zb
+        P.s1[0].copy_(init[0]); P.s2[0].copy_(init[1]); P.u.copy_(init[2]); P.w.copy_(init[3])
+        P.prime()
+        P.step_fwd_fused()
+        P.step_adj_fused()
+        got.append([t.clone() for t in (*P.sigma, P.u, P.w)])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("nsteps", [1, 8])
 def test_adjoint_dot_product_fused(rng, cuda, nsteps):
     """<P x, y> = <x, P^T y> for nsteps fused forward steps vs nsteps fused adjoint steps (no sponge, zero ghosts),
