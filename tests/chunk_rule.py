@@ -44,6 +44,18 @@ def depth(nz, tiles, slots, warm, cap, fused_pass=-1):
     return int(subprocess.run([_program(), *args], check=True, capture_output=True, text=True).stdout)
 
 
+# Shapes (nx, ny, nz, row alignment) whose x-y tiles are a whole number of rounds of every kernel named with them, so that
+# the rule keeps z in one chunk, several times as long as the kernels' register queues: the type2 kernels (tiles of 64 x 8
+# and 64 x 16 columns; the second layout runs the element-wise ones), type1, the elastic ones (velocity and strains; the
+# mixed interpolations), order 16 (ghost 8), and the fused steps at a zblock past nz.
+DEEP_TYPE2 = [(8, 4096, 44, 4), (5, 4096, 41, 1)]
+DEEP_TYPE1 = [(8, 2048, 44, 4), (5, 2048, 41, 1)]
+DEEP_ETTI, DEEP_ETTI_MIXED = (8, 4096, 40, 4), (8, 8192, 40, 4)
+DEEP_ORDER16 = (8, 4096, 40, 4)
+DEEP_FUSED = (8, 2048, 60, 4)
+TWO_CHUNKS_FUSED = (72, 1024, 70, 4)  # 2 x 128 tiles: at zblock 64 two chunks of 35 planes
+
+
 def tiles(shape, rows):
     return -(-shape[0] // 64) * -(-shape[1] // rows)
 

@@ -21,3 +21,24 @@ def test_full_rounds_keep_the_deepest_chunk():
     for slots in (256, 512, 1024):
         for nz in (2, 48, 200):
             assert C.depth(nz, 1024, slots, 9.0, 256) == nz
+
+
+def test_depths_of_the_shapes_that_parity_tests_take():
+    """The oracle comparisons cover the long march as well as the shortest chunks: what they say of their shapes' chunks
+    is so."""
+    one = {s: s[2] for s in C.DEEP_TYPE2 + C.DEEP_TYPE1 + [C.DEEP_ETTI, C.DEEP_ETTI_MIXED, C.DEEP_ORDER16]}
+    for s in C.DEEP_TYPE2:
+        for name, rows in (("FWD_DRV", 16), ("FWD_UPDATE", 8), ("ADJ_DRV", 8), ("ADJ_UPDATE", 16), ("RHO_GRAD", 8)):
+            assert C.stencil_depth(s, name + "_CHUNK", rows) == one[s], name
+    for s in C.DEEP_TYPE1:
+        assert C.stencil_depth(s, "T1_CHUNK", 8) == one[s]
+    for name, rows in (("FWD_DRV16", 16), ("FWD_UPDATE16", 8), ("ADJ_DRV16", 8), ("ADJ_UPDATE16", 8)):
+        assert C.stencil_depth(C.DEEP_ORDER16, name + "_CHUNK", rows) == one[C.DEEP_ORDER16], name
+    for name, s in (("VELOCITY", C.DEEP_ETTI), ("STRAIN", C.DEEP_ETTI), ("MIXED", C.DEEP_ETTI_MIXED)):
+        assert C.stencil_depth(s, name + "_CHUNK", 8) == one[s], name
+    small = (70, 19, 67)
+    assert all(C.stencil_depth(small, n, r) <= 4 for n in C.chunks() for r in (8, 16))
+    for p in (0, 1):
+        assert C.fused_depth(C.DEEP_FUSED, p, 64) == 60 and C.fused_depth(C.DEEP_FUSED, p, 16) == 15
+        assert C.fused_depth(C.TWO_CHUNKS_FUSED, p, 64) == 35
+        assert C.fused_depth(small, p, 64) == 2

@@ -1,6 +1,7 @@
 """The gfx950 eTTI kernels (include/tti_etti.h) against the FP64 oracle (oracle/etti_oracle.py) on the same FP32
-inputs: ragged interiors (x not a multiple of 64, y not of 8) and z extents over one and two z blocks, random ghosts,
-the coefficient set the reference's init_constant would upload and the Taylor / midpoint sets.
+inputs: ragged interiors (x not a multiple of 64, y not of 8) in z chunks of a few planes and tall ones that stay a
+single chunk of 40 (DEEP_ETTI, DEEP_ETTI_MIXED), random ghosts, the coefficient set the reference's init_constant would
+upload and the Taylor / midpoint sets.
 
 Bar: relative L2 <= 1e-6 on every written volume, ghosts and padding untouched (exact); copies, mirrors and the
 forwarding entry points bit-exact.
@@ -11,6 +12,7 @@ import numpy as np
 import pytest
 
 import etti_oracle as E
+from chunk_rule import DEEP_ETTI, DEEP_ETTI_MIXED
 
 pytestmark = pytest.mark.gpu
 
@@ -18,6 +20,12 @@ TAYLOR = (1225 / 1024, -245 / 3072, 49 / 5120, -5 / 7168)
 MIDPOINT = (1225 / 2048, -245 / 2048, 49 / 2048, -5 / 2048)
 COEFS = {"reference": (E.REF_CONSTANT, E.REF_CONSTANT), "taylor": (TAYLOR, MIDPOINT)}
 SHAPES = [(37, 21, 19), (70, 13, 70)]
+
+
+def _grid(shape):
+    from miniappsforhpe_amd.grid import Grid
+
+    return Grid(*shape[:3], align=shape[3] if len(shape) > 3 else 32)
 
 
 def _f32(c):
@@ -57,12 +65,11 @@ def _check(G, got, ref, inp, name, tol=1e-6):
 
 
 @pytest.mark.parametrize("coef", ["reference", "taylor"])
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + [DEEP_ETTI])
 def test_gpu_velocity(shape, coef, rng, cuda, setup):
     from miniappsforhpe_amd import ops
-    from miniappsforhpe_amd.grid import Grid
 
-    G = Grid(*shape)
+    G = _grid(shape)
     df, si = COEFS[coef]
     ops.etti_set_coefficients(df, si)
     print(f"etti velocity {shape} {coef}", flush=True)
@@ -83,14 +90,13 @@ def test_gpu_velocity(shape, coef, rng, cuda, setup):
 
 
 @pytest.mark.parametrize("coef", ["reference", "taylor"])
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + [DEEP_ETTI])
 def test_gpu_strain(shape, coef, rng, cuda, setup):
     import torch
 
     from miniappsforhpe_amd import ops
-    from miniappsforhpe_amd.grid import Grid
 
-    G = Grid(*shape)
+    G = _grid(shape)
     df, si = COEFS[coef]
     ops.etti_set_coefficients(df, si)
     print(f"etti strain {shape} {coef}", flush=True)
@@ -106,13 +112,13 @@ def test_gpu_strain(shape, coef, rng, cuda, setup):
         _check(G, g["d%d" % k], o["d%d" % k], v["d%d" % k], "d%d" % k)
 
 
-@pytest.mark.parametrize("xs,ys,zs", [(a, b, c) for a in (0, 1) for b in (0, 1) for c in (0, 1)])
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape,xs,ys,zs",
+                         [(s, a, b, c) for s in SHAPES for a in (0, 1) for b in (0, 1) for c in (0, 1)] +
+                         [(DEEP_ETTI_MIXED, 0, 1, 0), (DEEP_ETTI_MIXED, 1, 0, 1)])
 def test_gpu_mixed(shape, xs, ys, zs, rng, cuda, setup):
     from miniappsforhpe_amd import ops
-    from miniappsforhpe_amd.grid import Grid
 
-    G = Grid(*shape)
+    G = _grid(shape)
     ops.etti_set_coefficients(None, E.REF_CONSTANT)
     print(f"etti mixed {shape} shifts {(xs, ys, zs)}", flush=True)
     v = _vols(G, rng, ["g", "xz", "yz"])

@@ -18,6 +18,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from chunk_rule import DEEP_ORDER16
 
 DX, DY, DZ = 10.0, 12.5, 8.0
 
@@ -303,10 +304,11 @@ def test_gpu_type2_order16(shape, order16, cuda):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape,align", [((37, 11, 13), 1), ((64, 8, 1), 32), ((330, 25, 40), 32)])
+@pytest.mark.parametrize("shape,align", [((37, 11, 13), 1), ((64, 8, 1), 32), ((330, 25, 40), 32), (DEEP_ORDER16[:3], 4)])
 def test_gpu_type2_order16_layouts(shape, align, order16, cuda):
     """The four order-16 operators chained as a forward and an adjoint step: rows of 53 floats (element-wise kernels), one
-    plane and one whole tile, and a grid of 6 x 4 tiles with ragged ends cut into several z chunks (tiled kernels)."""
+    plane and one whole tile, a grid of 6 x 4 tiles with ragged ends cut into z chunks of 2 and 4 planes, and a tall one
+    that stays a single chunk of 40, past the 16-word queues (tiled kernels)."""
     from miniappsforhpe_amd import ops
     from miniappsforhpe_amd.grid import Grid
 

@@ -8,20 +8,21 @@ import numpy as np
 import pytest
 import torch
 
+import chunk_rule
 import oracle as O
-from test_parity_type2 import f32, from_gpu, make_models, rel_l2, to_gpu
+from chunk_rule import DEEP_FUSED, TWO_CHUNKS_FUSED
+from test_parity_type2 import f32, from_gpu, grid_pair, make_models, rel_l2, to_gpu
 
 pytestmark = pytest.mark.gpu
 
 DX, DY, DZ = 10.0, 11.0, 9.0
-SHAPES = [(70, 19, 67), (40, 33, 150)]
+SHAPES = [(70, 19, 67), (40, 33, 150)]  # cut into chunks of 2 planes
 
 
 def setup(shape, rng, cuda, sponge=False, zblock=64):
-    from miniappsforhpe_amd.grid import Grid
     from miniappsforhpe_amd.propagator import TTIPropagator
 
-    G, OG = Grid(*shape), O.Geom(*shape)
+    G, OG = grid_pair(shape)
     m = make_models(G, rng)
     sp = None
     if sponge:
@@ -37,7 +38,7 @@ def interior_random(G, rng):
     return f32(a)
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + [TWO_CHUNKS_FUSED])
 @pytest.mark.parametrize("sponge", [False, True])
 def test_fused_forward_vs_oracle(shape, sponge, rng, cuda):
     G, OG, m, sp, P = setup(shape, rng, cuda, sponge)
@@ -85,7 +86,7 @@ def test_fused_forward_vs_plain_path(shape, rng, cuda):
         assert rel_l2(a, b) < 1e-5
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + [TWO_CHUNKS_FUSED])
 @pytest.mark.parametrize("sponge", [False, True])
 def test_fused_adjoint_vs_oracle(shape, sponge, rng, cuda):
     G, OG, m, sp, P = setup(shape, rng, cuda, sponge)
@@ -121,11 +122,11 @@ def test_fused_adjoint_vs_plain_path(rng, cuda):
         assert rel_l2(a, b) < 1e-5
 
 
-@pytest.mark.parametrize("shape,zblock", [(SHAPES[0], 64), (SHAPES[1], 16)])
+@pytest.mark.parametrize("shape,zblock", [(SHAPES[0], 64), (SHAPES[1], 16), (DEEP_FUSED, 64), (DEEP_FUSED, 16)])
 def test_fused_free_surface_vs_oracle(shape, zblock, rng, cuda):
     """Stress-free surface at the top interior plane (the reference's mirrors of sigma and of the derivatives):
     5 fused forward steps, then 4 fused adjoint steps, each against the oracle's step composition with
-    free_surface=True (z chunks of 16 planes in the second case, so the mirrored plane lies in the first of many)."""
+    free_surface=True, with z chunks of 2 (the mirror reaches into the second), 60 and 15 planes."""
     G, OG, m, sp, P = setup(shape, rng, cuda, zblock=zblock)
     P.free_surface = True
     s1, s2, u, w = (interior_random(G, rng) for _ in range(4))
@@ -297,12 +298,15 @@ def test_snapshot_encoding_is_exact(mode, rng, cuda):
 
 @pytest.mark.parametrize("zblock,strip", [(16, 3), (40, 1), (200, 2)])
 def test_block_schedule_keeps_results(zblock, strip, rng, cuda):
-    """The z depth of the blocks and the strip schedule of the tiles (4 x tiles here: strips of 3 + 1, 1, 2 + 2)
-    change which block computes a point, never its value: forward steps with an FP16 snapshot and adjoint steps with
-    FP64 imaging are bit-identical to the default schedule."""
+    """The z depth of the blocks (50 planes, against 15, 34 and 100) and the strip schedule of the tiles (4 x tiles here:
+    strips of 3 + 1, 1, 2 + 2) change which block computes a point, never its value: forward steps with an FP16 snapshot
+    and adjoint steps with FP64 imaging are bit-identical to the default schedule."""
     from miniappsforhpe_amd.propagator import SnapshotStore
 
-    G, OG, m, sp, P = setup((200, 21, 37), rng, cuda)
+    shape = (200, 512, 100)
+    for p in (0, 1):
+        assert chunk_rule.fused_depth(shape, p, zblock) != chunk_rule.fused_depth(shape, p, 64)
+    G, OG, m, sp, P = setup(shape, rng, cuda)
     init = [to_gpu(interior_random(G, rng), cuda) for _ in range(4)]
 
     def run(zb, st):
@@ -325,12 +329,16 @@ def test_block_schedule_keeps_results(zblock, strip, rng, cuda):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("shape,caps", [((400, 300, 23), (1, 2, 7, 12)), ((64, 8, 300), (1, 3, 64)), ((5, 3, 1), (1,))])
+@pytest.mark.parametrize("shape,caps", [((130, 680, 72), (1, 2, 7, 12, 40)), ((64, 8, 300), (1,)), ((5, 3, 2), (1,))])
 def test_chunk_depth_keeps_results(shape, caps, rng, cuda):
-    """The launchers choose the z chunks (zblock is the most they may hold): the enough-tiles volume keeps deep chunks,
-    the narrow one is cut into many, one plane has one; every cap, down to one plane a block, gives the same bits."""
+    """The launchers choose the z chunks (zblock is the most they may hold): 3 x 85 tiles keep 72 planes in one, the narrow
+    volumes are cut into chunks of 2; every cap that makes them shallower, down to one plane a block, gives the same
+    bits."""
     from miniappsforhpe_amd.propagator import SnapshotStore
 
+    for p in (0, 1):
+        depths = [chunk_rule.fused_depth(shape, p, zb) for zb in (*caps, 256)]
+        assert sorted(set(depths)) == depths and depths[-1] == (72 if shape[2] == 72 else 2)
     G, OG, m, sp, P = setup(shape, rng, cuda, sponge=True)
     P.free_surface = shape[2] > 4
     init = [to_gpu(interior_random(G, rng), cuda) for _ in range(4)]

@@ -1,14 +1,16 @@
-"""GPU parity of the constant-density (type1) operators against the FP64 oracle (relative L2 <= 1e-5)."""
+"""GPU parity of the constant-density (type1) operators against the FP64 oracle (relative L2 <= 1e-5), on grids that are
+cut into z chunks of 2 planes and on tall ones that stay a single chunk of 41 or 44 (DEEP_TYPE1)."""
 import numpy as np
 import pytest
 
 import oracle as O
+from chunk_rule import DEEP_TYPE1
 from test_parity_type2 import f32, from_gpu, grid_pair, make_models, rel_l2, to_gpu
 
 pytestmark = pytest.mark.gpu
 
 DX, DY, DZ = 10.0, 12.0, 9.0
-SHAPES = [(70, 19, 67), (33, 41, 70), (37, 11, 13, 1)]  # the last: element-wise kernels (rows of 45 floats)
+SHAPES = [(70, 19, 67), (33, 41, 70), (37, 11, 13, 1), *DEEP_TYPE1]  # rows of 45 and 13 floats: element-wise kernels
 
 
 @pytest.mark.parametrize("shape", SHAPES)
