@@ -119,9 +119,9 @@ __global__ __launch_bounds__(BX* EBY) void k_etti_velocity(
     const EttiTile T(nx, ny, ldx, bxi, byi);
     const int z0 = R + bzi * bz, z1 = min(z0 + bz, R + nz);
     const long sz = ldx * ldy;
-    const TileQuads<W, EBY, NT> qx(tid, ldx, T.xlim_h, T.ylim_c);
-    const TileQuads<BX, H, NT> qy(tid, ldx, T.xlim_c, T.ylim_h);
-    const TileQuads<W, H, NT> qxy(tid, ldx, T.xlim_h, T.ylim_h);
+    const TileQuads<W, EBY, NT, false> qx(tid, ldx, T.xlim_h, T.ylim_c);
+    const TileQuads<BX, H, NT, false> qy(tid, ldx, T.xlim_c, T.ylim_h);
+    const TileQuads<W, H, NT, false> qxy(tid, ldx, T.xlim_h, T.ylim_h);
     const long ox = (long)T.y0 * ldx + (T.x0 - R), oy = (long)(T.y0 - R) * ldx + T.x0,
                oxy = (long)(T.y0 - R) * ldx + (T.x0 - R);
     float4 r4[qx.QT], r8[qx.QT], r5[qy.QT], r9[qy.QT], r7[qxy.QT];
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(BX* EBY) void k_etti_strain(
     const EttiTile T(nx, ny, ldx, bxi, byi);
     const int z0 = R + bzi * bz, z1 = min(z0 + bz, R + nz);
     const long sz = ldx * ldy;
-    const TileQuads<W, H, NT> qt(tid, ldx, T.xlim_h, T.ylim_h);
+    const TileQuads<W, H, NT, false> qt(tid, ldx, T.xlim_h, T.ylim_h);
     const long org = (long)(T.y0 - R) * ldx + (T.x0 - R);
     float4 r1[qt.QT], r2[qt.QT], r3[qt.QT];
     auto fetch = [&](int z) {
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(BX* EBY) void k_etti_mixed(const float* __restrict_
     const EttiTile T(nx, ny, ldx, bxi, byi);
     const int z0 = R + bzi * bz, z1 = min(z0 + bz, R + nz);
     const long sz = ldx * ldy;
-    const TileQuads<W, H, NT> qt(tid, ldx, T.xlim_h, T.ylim_h);
+    const TileQuads<W, H, NT, false> qt(tid, ldx, T.xlim_h, T.ylim_h);
     const long org = (long)(T.y0 - R) * ldx + (T.x0 - R);
     float4 r[qt.QT];
     float axz[8], ayz[8];
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(BX* EBY) void k_etti_stress(StressArgs A, int nx, i
         for (int k = 0; k < 6; ++k)
             s[k] = A.f[k][i];
     }
-    const TileQuads<W, H, NT> qt(tid, ldx, T.xlim_h, T.ylim_h);
+    const TileQuads<W, H, NT, false> qt(tid, ldx, T.xlim_h, T.ylim_h);
     const long org = (long)z * sz + (long)(T.y0 - R) * ldx + (T.x0 - R);
     float4 r[6][qt.QT];
 #pragma unroll

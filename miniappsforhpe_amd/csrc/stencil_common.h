@@ -3,6 +3,7 @@
 
 #include <cstdint>
 #include <initializer_list>
+#include <type_traits>
 
 #include "fd_tables.h"
 
@@ -115,11 +116,14 @@ load_tile(float (*t)[W], const float* __restrict__ src, long origin, long ldx, i
 // allocation. The launchers check that ldx is a multiple of 4 and the volumes are 16-byte aligned, and every tile
 // origin is a multiple of 4 columns, so each quad is one aligned float4 load and one aligned LDS store. fetch()
 // issues the loads; commit() masks and stores them a plane later (a select right after a load would wait for it).
-template <int W, int H, int NT>
+// LANE32: 32-bit byte offsets from a scalar plane pointer (planes of less than 4 GiB), which leave the type2 and type1
+// kernels their registers; the elastic kernels have registers to spare and are faster with 64-bit element offsets (strains
+// 1.81 -> 1.75 ms at 512^3, 34 -> 31 us at 150 x 203 x 117, velocity 42 -> 40 us there).
+template <int W, int H, int NT, bool LANE32 = true>
 struct TileQuads
 {
     static constexpr int QPR = W / 4, NQ = QPR * H, QT = (NQ + NT - 1) / NT;
-    unsigned off[QT]; // byte offset from the tile origin within a plane
+    std::conditional_t<LANE32, unsigned, long> off[QT]; // from the tile origin within a plane (64 bits: -1 not loaded)
     int lds[QT];      // first element of the quad in the W x H LDS tile, -1: no quad for this slot
     int keep[QT];     // elements of the quad inside xlim (0..4; 0: not loaded)
 
@@ -132,15 +136,22 @@ struct TileQuads
             const bool has = q < NQ;
             lds[k] = has ? row * W + lx : -1;
             keep[k] = has && row < ylim ? min(max(xlim - lx, 0), 4) : 0;
-            off[k] = ((unsigned)row * (unsigned)ldx + (unsigned)lx) * 4u;
+            if constexpr (LANE32)
+                off[k] = ((unsigned)row * (unsigned)ldx + (unsigned)lx) * 4u;
+            else
+                off[k] = keep[k] > 0 ? (long)row * ldx + lx : -1;
         }
     }
     __device__ __forceinline__ void fetch(float4 (&r)[QT], const float* __restrict__ origin) const
     {
 #pragma unroll
         for (int k = 0; k < QT; ++k)
-            if (keep[k] > 0)
-                r[k] = ldp4(origin, here(off[k]));
+            if constexpr (LANE32) {
+                if (keep[k] > 0)
+                    r[k] = ldp4(origin, here(off[k]));
+            } else if (off[k] >= 0) {
+                r[k] = *reinterpret_cast<const float4*>(origin + off[k]);
+            }
     }
     __device__ __forceinline__ void commit(float* tile, const float4 (&r)[QT]) const
     {
