@@ -57,10 +57,13 @@ constexpr int CUS = 256; // compute units of one MI355X
 // marching 72 planes at 2 us) and a round that is barely begun costs a whole one; many shallow ones recompute halos.
 // Returns the depth of the cheapest number of chunks, none deeper than `cap` (any value: the fused steps pass a caller's
 // zblock, which may be the largest int for "no limit"); a shallower one has to gain 3% over the best so far, because
-// deeper chunks also read less. A last round of at most one block per CU runs its planes faster
-// (2.05 us against 2.43 us with two 512-thread blocks per CU of a fused forward kernel).
+// deeper chunks also read less. Where several blocks fit a CU, a last round of at most one block per CU runs its planes
+// faster and counts 0.85 of a round: only the elastic kernels have such rounds, and on the volumes where it changes the
+// choice the mixed interpolations take 5.8 to 6.7 us with it and 6.9 to 7.5 without (40 to 180 points a side; chunks of 3
+// and 4 planes instead of 2), the strains the same either way. The deepest chunk is taken at once where its blocks fill
+// `full` of one round or more (see MIXED_CHUNK).
 inline int
-chunk_depth(int nz, long tiles, int slots, float warm, int cap)
+chunk_depth(int nz, long tiles, int slots, float warm, int cap, float full = 2.0f)
 {
     cap = cap < 1 ? 1 : cap > nz ? nz : cap;
     int best = 0;
@@ -70,6 +73,8 @@ chunk_depth(int nz, long tiles, int slots, float warm, int cap)
         if (best && bz < 2)
             break;
         const long n = tiles * ((nz + bz - 1) / bz), r = n % slots;
+        if (!best && n <= slots && (float)n >= full * (float)slots)
+            return bz;
         const float rounds = (float)(n / slots) + (r == 0 ? 0.0f : r <= CUS && slots > CUS ? 0.85f : 1.0f);
         const float t = ((float)bz + warm) * rounds;
         if (!best || t < 0.97f * cost) {

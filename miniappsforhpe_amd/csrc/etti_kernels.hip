@@ -574,7 +574,12 @@ etti_grid(int nx, int ny, int nz, int bz)
 
 // Chunks of the z-marching kernels (see stencil_bz; against 64-plane chunks at 64^3: velocity 76 -> 15 us, strains 58 ->
 // 14, mixed interpolations 29 -> 9 us)
-constexpr Chunk VELOCITY_CHUNK{ 2, 2.0f }, STRAIN_CHUNK{ 2, 4.0f }, MIXED_CHUNK{ 4, 9.0f };
+constexpr Chunk VELOCITY_CHUNK{ 2, 2.0f }, STRAIN_CHUNK{ 2, 4.0f };
+// The mixed interpolations do little per word, so three blocks per CU already reach the rate of four: blocks of the
+// deepest chunk that are all resident at once and fill two thirds of the round beat cut ones that start the march over
+// (fill 0.75: 384 x 512 x 512 397 -> 340 us, 640 x 640 x 200 296 -> 264; 0.68: 400^3 274 -> 243; 0.63: 317 -> 311 and 188
+// -> 190; 0.5: 182 -> 231, so not there).
+constexpr Chunk MIXED_CHUNK{ 4, 9.0f, 256, 0.667f };
 
 int
 etti_bz(int nx, int ny, int nz, Chunk k)

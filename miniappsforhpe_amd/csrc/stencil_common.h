@@ -221,20 +221,22 @@ stencil_grid(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, i
     return dim3((nx + BX - 1) / BX, (ny + by - 1) / by, (nz + bz - 1) / bz);
 }
 
-// What chunk_depth needs of a z-marching kernel: its resident blocks per CU and the planes' worth of a chunk's prologue
-// and recomputed halo, both from its sweep over chunk depths of 2 to 256 planes at 64^3 to 320 x 288 x 240. The deepest
-// chunk is 256 planes (4% more reads at 128; no faster at 512).
+// What chunk_depth needs of a z-marching kernel: the blocks per CU that make a round and the planes' worth of a chunk's
+// prologue and recomputed halo, both from its sweep over chunk depths of 2 to 256 planes at 64^3 to 320 x 288 x 240. The
+// element-wise kernels of the same operators take the constants of the tiled ones. The deepest chunk is 256 planes (4%
+// more reads at 128; no faster at 512).
 struct Chunk
 {
     int per_cu;
     float warm;
     int cap = 256;
+    float full = 2.0f; // share of one round that the deepest chunk's blocks have to fill to be taken (2: never)
 };
 
 inline int
 stencil_bz(int ixbeg, int ixend, int iybeg, int iyend, int izbeg, int izend, Chunk k, int by = BYS)
 {
     const dim3 g = stencil_grid(ixbeg, ixend, iybeg, iyend, izbeg, izend, 1, by);
-    return chunk_depth((int)g.z, (long)g.x * g.y, k.per_cu * CUS, k.warm, k.cap);
+    return chunk_depth((int)g.z, (long)g.x * g.y, k.per_cu * CUS, k.warm, k.cap, k.full);
 }
 } // namespace tti

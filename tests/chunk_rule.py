@@ -20,8 +20,9 @@ using namespace tti::fused;
 int main(int, char** v)
 {
     const int nz = atoi(v[2]), cap = atoi(v[6]), pass = atoi(v[1]);
+    const float full = (float)atof(v[7]);
     const long tiles = atol(v[3]);
-    printf("%d\n", pass < 0 ? chunk_depth(nz, tiles, atoi(v[4]), (float)atof(v[5]), cap)
+    printf("%d\n", pass < 0 ? chunk_depth(nz, tiles, atoi(v[4]), (float)atof(v[5]), cap, full)
                             : chunk_depth(nz, tiles, STEP_SLOTS[pass], STEP_WARM[pass], cap));
 }
 """
@@ -39,8 +40,8 @@ def _program():
 
 
 @functools.lru_cache(maxsize=None)
-def depth(nz, tiles, slots, warm, cap, fused_pass=-1):
-    args = [str(a) for a in (fused_pass, nz, tiles, slots, warm, cap)]
+def depth(nz, tiles, slots, warm, cap, fused_pass=-1, full=2.0):
+    args = [str(a) for a in (fused_pass, nz, tiles, slots, warm, cap, full)]
     return int(subprocess.run([_program(), *args], check=True, capture_output=True, text=True).stdout)
 
 
@@ -51,6 +52,7 @@ def depth(nz, tiles, slots, warm, cap, fused_pass=-1):
 DEEP_TYPE2 = [(8, 4096, 44, 4), (5, 4096, 41, 1)]
 DEEP_TYPE1 = [(8, 2048, 44, 4), (5, 2048, 41, 1)]
 DEEP_ETTI, DEEP_ETTI_MIXED = (8, 4096, 40, 4), (8, 8192, 40, 4)
+THREE_QUARTERS_ETTI_MIXED = (8, 6144, 100, 4)  # 768 blocks of one chunk, all resident (cut by the rounds alone)
 DEEP_ORDER16 = (8, 4096, 40, 4)
 DEEP_FUSED = (8, 2048, 60, 4)
 TWO_CHUNKS_FUSED = (72, 1024, 70, 4)  # 2 x 128 tiles: at zblock 64 two chunks of 35 planes
@@ -67,13 +69,13 @@ def fused_depth(shape, fused_pass, zblock):
 
 @functools.lru_cache(maxsize=None)
 def chunks():
-    """{name: (blocks per CU, warm, cap)} of every Chunk constant in the kernel sources."""
+    """{name: (blocks per CU, warm, cap, full)} of every Chunk constant in the kernel sources."""
     text = "".join((B.CSRC / f"{n}_kernels.hip").read_text() for n in ("type2", "type1", "etti"))
-    found = re.findall(r"(\w+_CHUNK)\{ (\d+), ([\d.]+)f(?:, (\d+))? \}", text)
-    return {n: (int(k), float(w), int(c or 256)) for n, k, w, c in found}
+    found = re.findall(r"(\w+_CHUNK)\{ (\d+), ([\d.]+)f(?:, (\d+)(?:, ([\d.]+)f)?)? \}", text)
+    return {n: (int(k), float(w), int(c or 256), float(f or 2)) for n, k, w, c, f in found}
 
 
 def stencil_depth(shape, name, rows):
     """Planes per block of the kernel with Chunk constant `name` and tiles of 64 x rows columns."""
-    per_cu, warm, cap = chunks()[name]
-    return depth(shape[2], tiles(shape, rows), per_cu * 256, warm, cap)
+    per_cu, warm, cap, full = chunks()[name]
+    return depth(shape[2], tiles(shape, rows), per_cu * 256, warm, cap, full=full)

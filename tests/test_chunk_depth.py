@@ -36,9 +36,19 @@ def test_depths_of_the_shapes_that_parity_tests_take():
         assert C.stencil_depth(C.DEEP_ORDER16, name + "_CHUNK", rows) == one[C.DEEP_ORDER16], name
     for name, s in (("VELOCITY", C.DEEP_ETTI), ("STRAIN", C.DEEP_ETTI), ("MIXED", C.DEEP_ETTI_MIXED)):
         assert C.stencil_depth(s, name + "_CHUNK", 8) == one[s], name
+    s = C.THREE_QUARTERS_ETTI_MIXED
+    assert C.stencil_depth(s, "MIXED_CHUNK", 8) == 100 > C.depth(100, 768, 1024, 9.0, 256)
     small = (70, 19, 67)
     assert all(C.stencil_depth(small, n, r) <= 4 for n in C.chunks() for r in (8, 16))
     for p in (0, 1):
         assert C.fused_depth(C.DEEP_FUSED, p, 64) == 60 and C.fused_depth(C.DEEP_FUSED, p, 16) == 15
         assert C.fused_depth(C.TWO_CHUNKS_FUSED, p, 64) == 35
         assert C.fused_depth(small, p, 64) == 2
+
+
+def test_deepest_chunk_that_fills_a_round():
+    """`full`: the deepest chunk is taken where its blocks fill that share of one round, no more than one; else the rounds
+    decide."""
+    for tiles, nz, deep in ((768, 200, True), (684, 200, True), (640, 200, False), (1025, 200, False), (384, 400, True)):
+        cut = C.depth(nz, tiles, 1024, 9.0, 256)
+        assert C.depth(nz, tiles, 1024, 9.0, 256, full=0.667) == (200 if deep else cut)
