@@ -21,6 +21,10 @@ namespace tti {
 // 122 -> 21, adjoint derivatives 143 -> 36, adjoint update 70 -> 15, density gradient 149 -> 19 us.
 constexpr Chunk FWD_DRV_CHUNK{ 1, 4.0f }, FWD_UPDATE_CHUNK{ 1, 9.5f }, ADJ_DRV_CHUNK{ 1, 9.0f },
     RHO_GRAD_CHUNK{ 1, 3.0f };
+// Points below which the order-8 forward update takes a thread per column and field. One thread per column against two:
+// 64^3 16.7 and 15.1 us, 128^3 45.6 and 41.0, 150 x 203 x 117 89.9 and 81.3, 200 x 300 x 100 157.0 and 157.0, 192^3 150.8
+// and 153.8, 301 x 217 x 190 277 and 282, 400^3 1321 and 1405, 480^3 2174 and 2397, 512^3 2504 and 2552.
+constexpr long FWD_UPDATE_SPLIT_BELOW = 6000000;
 // the adjoint update runs in dispatch order, where chunks over 64 planes read more (1.37 ms at 64, 1.43 at 256, 512^3)
 constexpr Chunk ADJ_UPDATE_CHUNK{ 1, 4.0f, 64 };
 // order 16: 16 halo planes
@@ -356,15 +360,36 @@ __global__ __launch_bounds__(BX* BY) void k_fwd_update(
     }
 }
 
+// H and V of a field from its sums: second differences scaled by 1/(rho d), the x-y term scaled, the z-mixed ones not yet.
+// Every product and sum has one fixed rounding, so that both kernels below give the same bits.
+struct HV
+{
+    float h, v;
+};
+__device__ __forceinline__ HV
+fwd_hv(float fxx, float fyy, float fzz, float fxy, float qzx, float qyz, float sx, float sy, float sz, float invdzdx,
+       float invdydz, float vx, float vy, float vz)
+{
+    fxx = __fmul_rn(fxx, sx);
+    fyy = __fmul_rn(fyy, sy);
+    fzz = __fmul_rn(fzz, sz);
+    HV t;
+    t.v = fmaf(2.0f * vy * vz, __fmul_rn(qyz, invdydz),
+               fmaf(2.0f * vz * vx, __fmul_rn(qzx, invdzdx),
+                    fmaf(2.0f * vx * vy, fxy, fmaf(vz * vz, fzz, fmaf(vy * vy, fyy, __fmul_rn(vx * vx, fxx))))));
+    t.h = __fsub_rn(__fadd_rn(__fadd_rn(fxx, fyy), fzz), t.v);
+    return t;
+}
+
 // The same operator with the plane pipeline of the gfx950 stencils: the tiles of plane p + 1 (sigma, and the d_x / d_y
 // tiles of output plane p + 1 - RO) are loaded as float4 quads during plane p - 1 and stored into the other LDS buffer
 // during plane p, the d_z column word and the pointwise words of the next output plane are loaded one plane ahead, and
 // one barrier per plane separates a buffer's last read from its refill. Needs quads_fit (launcher falls back).
-// One thread per column and field (threadIdx.z): the z queues of one field fit 88 VGPRs (124 at RO = 8, where both
+// One thread per column and field (threadIdx.z): the z queues of one field fit 89 VGPRs (125 at RO = 8, where both
 // fields in one thread spilled 93 of 256), so 16 waves are resident per CU instead of 8. u needs V2 and w needs H1 of
-// the other field's thread: they pass through LDS and a plane's update is finished after the barrier that ends it.
-// It is bound by HBM at 512^3 (2.48 ms with one thread per column, 2.53 ms; 80 B a point at the copy rate: 2.16 ms) and
-// by latency below (256^3 335 -> 317 us, 301 x 217 x 190 280 -> 272 us); order 16 at 200 x 168 x 144 419 -> 163 us.
+// the other field's thread: they pass through LDS and a plane's update is finished after the barrier that ends it. It is
+// the faster one where latency bounds the update, on volumes of a few million points, and everywhere at order 16 (200 x
+// 168 x 144: 419 -> 163 us); k_fwd_update_qc takes the larger ones at order 8.
 template <int BY, int RO>
 __global__ __launch_bounds__(2 * BX* BY) void k_fwd_update_q(
     float* __restrict__ u, float* __restrict__ w, const float* __restrict__ d1x, const float* __restrict__ d2x,
@@ -476,8 +501,10 @@ __global__ __launch_bounds__(2 * BX* BY) void k_fwd_update_q(
         float a = 0, ddx[RO + 1], ddy[RO + 1];
 #pragma unroll
         for (int n = 1; n <= RO; ++n) {
-            a += FD<RO>::e[n] * ((S[ty + RO + n][tx + HX + n] - S[ty + RO - n][tx + HX + n]) +
-                                 (S[ty + RO - n][tx + HX - n] - S[ty + RO + n][tx + HX - n]));
+            a = fmaf(FD<RO>::e[n],
+                     (S[ty + RO + n][tx + HX + n] - S[ty + RO - n][tx + HX + n]) +
+                         (S[ty + RO - n][tx + HX - n] - S[ty + RO + n][tx + HX - n]),
+                     a);
             ddx[n] = S[ty + RO][tx + HX + n] - S[ty + RO][tx + HX - n];
             ddy[n] = S[ty + RO + n][tx + HX] - S[ty + RO - n][tx + HX];
             hold(a), hold(ddx[n]), hold(ddy[n]);
@@ -494,20 +521,15 @@ __global__ __launch_bounds__(2 * BX* BY) void k_fwd_update_q(
 #pragma unroll
             for (int n = 1; n <= RO; ++n) {
                 const float c = FD<RO>::c[n];
-                fxx += c * (X[ty][tx + HX + n] - X[ty][tx + HX - n + 1]);
-                fyy += c * (Y[ty + RO + n][tx] - Y[ty + RO - n + 1][tx]);
-                fzz += c * (dz[RO - 1 + n] - dz[RO - n]);
+                fxx = fmaf(c, X[ty][tx + HX + n] - X[ty][tx + HX - n + 1], fxx);
+                fyy = fmaf(c, Y[ty + RO + n][tx] - Y[ty + RO - n + 1][tx], fyy);
+                fzz = fmaf(c, dz[RO - 1 + n] - dz[RO - n], fzz);
             }
             const float rho = 1.0f / pw[0];
-            fxx *= invdx * rho;
-            fyy *= invdy * rho;
-            fzz *= invdz * rho;
-            const float vx = pw[1], vy = pw[2], vz = pw[3];
-            const float V = vx * vx * fxx + vy * vy * fyy + vz * vz * fzz + 2.0f * vx * vy * xy[0] +
-                            2.0f * vz * vx * (qzx[0] * invdzdx) + 2.0f * vy * vz * (qyz[0] * invdydz);
-            const float Hf = fxx + fyy + fzz - V;
-            ex[b][F][ty][tx] = F ? V : Hf;
-            part = pw[4] * Hf + pw[5] * V;
+            const HV t = fwd_hv(fxx, fyy, fzz, xy[0], qzx[0], qyz[0], invdx * rho, invdy * rho, invdz * rho, invdzdx,
+                                invdydz, pw[1], pw[2], pw[3]);
+            ex[b][F][ty][tx] = F ? t.v : t.h;
+            part = fmaf(pw[5], t.v, __fmul_rn(pw[4], t.h));
             mc = pw[6];
             old = pw[7];
         }
@@ -521,6 +543,211 @@ __global__ __launch_bounds__(2 * BX* BY) void k_fwd_update_q(
         __syncthreads();
     }
     finish(z1 - 1, (pend - 1 - p0) & 1);
+}
+
+// The same with one thread per column for both fields (222 VGPRs, 8 waves per CU), order 8: every pointwise word is loaded
+// once instead of by both fields' threads, which is what counts once the 18 volumes are past the 256 MB that the caches
+// hold and HBM bounds it. Same bits as k_fwd_update_q.
+template <int BY>
+__global__ __launch_bounds__(BX* BY) void k_fwd_update_qc(
+    float* __restrict__ u, float* __restrict__ w, const float* __restrict__ d1x, const float* __restrict__ d2x,
+    const float* __restrict__ d1y, const float* __restrict__ d2y, const float* __restrict__ d1z,
+    const float* __restrict__ d2z, const float* __restrict__ f1, const float* __restrict__ f2,
+    const float* __restrict__ irho, const float* __restrict__ m1, const float* __restrict__ m2,
+    const float* __restrict__ m3, const float* __restrict__ m4, const float* __restrict__ rx,
+    const float* __restrict__ ry, const float* __restrict__ rz, int ixbeg, int ixend, int iybeg, int iyend,
+    int izbeg, int izend, long ldx, long ldy, float dt, float invdx, float invdy, float invdz, float invdxdy,
+    float invdydz, float invdzdx, int bz)
+{
+    constexpr int W = BX + 2 * R, H = BY + 2 * R, NT = BX * BY;
+    __shared__ __align__(16) float s1[2][H][W]; // sigma at plane p (halo 4 in x and y)
+    __shared__ __align__(16) float s2[2][H][W];
+    __shared__ __align__(16) float x1[2][BY][W]; // d_x at plane o (halo 4 in x)
+    __shared__ __align__(16) float x2[2][BY][W];
+    __shared__ __align__(16) float y1[2][H][BX]; // d_y at plane o (halo 4 in y)
+    __shared__ __align__(16) float y2[2][H][BX];
+    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
+    int bxi, byi, bzi;
+    stencil_tile(bxi, byi, bzi);
+    const int x0 = ixbeg + bxi * BX, y0 = iybeg + byi * BY, z0 = izbeg + bzi * bz;
+    const int z1 = min(z0 + bz, izend + 1);
+    const int ix = x0 + tx, iy = y0 + ty;
+    const bool active = ix <= ixend && iy <= iyend;
+    const long sz = ldx * ldy;
+    const int xlim = min(W, ixend + R + 1 - (x0 - R));
+    const int ylim = min(H, iyend + R + 1 - (y0 - R));
+    const int xlim_c = min(BX, ixend + 1 - x0);
+    const int ylim_c = min(BY, iyend + 1 - y0);
+    const long col = (long)iy * ldx + ix;
+    const int p0 = z0 - R, pend = z1 + R; // tile planes p in [p0, pend), output o = p - R
+
+    const TileQuads<W, H, NT, false> qs(tid, ldx, xlim, ylim);
+    const TileQuads<W, BY, NT, false> qx(tid, ldx, xlim, ylim_c);
+    const TileQuads<BX, H, NT, false> qy(tid, ldx, xlim_c, ylim);
+    const long os = (long)(y0 - R) * ldx + (x0 - R), ox = (long)y0 * ldx + (x0 - R), oy = (long)(y0 - R) * ldx + x0;
+    float4 rs1[qs.QT], rs2[qs.QT], rx1[qx.QT], rx2[qx.QT], ry1[qy.QT], ry2[qy.QT];
+    auto fetch = [&](int p) {
+        const long pz = (long)p * sz;
+        qs.fetch(rs1, f1 + pz + os);
+        qs.fetch(rs2, f2 + pz + os);
+        if (p - R >= z0) {
+            const long oz = (long)(p - R) * sz;
+            qx.fetch(rx1, d1x + oz + ox);
+            qx.fetch(rx2, d2x + oz + ox);
+            qy.fetch(ry1, d1y + oz + oy);
+            qy.fetch(ry2, d2y + oz + oy);
+        }
+    };
+    auto commit = [&](int p, int b) {
+        qs.commit(&s1[b][0][0], rs1);
+        qs.commit(&s2[b][0][0], rs2);
+        if (p - R >= z0) {
+            qx.commit(&x1[b][0][0], rx1);
+            qx.commit(&x2[b][0][0], rx2);
+            qy.commit(&y1[b][0][0], ry1);
+            qy.commit(&y2[b][0][0], ry2);
+        }
+    };
+    // pointwise words of an output plane: 1/rho, m1..m4, rx, ry, rz, u, w
+    float pw[10];
+    auto load_pw = [&](int o) {
+        if (active && o >= z0 && o < z1) {
+            const long i = (long)o * sz + col;
+            pw[0] = irho[i];
+            pw[1] = m1[i];
+            pw[2] = m2[i];
+            pw[3] = m3[i];
+            pw[4] = m4[i];
+            pw[5] = rx[i];
+            pw[6] = ry[i];
+            pw[7] = rz[i];
+            pw[8] = u[i];
+            pw[9] = w[i];
+        }
+    };
+
+    float qzx1[9], qyz1[9], qzx2[9], qyz2[9]; // mixed partial sums: Q[j] <-> output plane p - 4 + j
+    float xy1[5], xy2[5];                     // F_xy delayed: xy[4] = F_xy(p)
+    float dz1[8], dz2[8];                     // dz[k] <-> d_z(p - 7 + k)
+#pragma unroll
+    for (int j = 0; j < 9; ++j)
+        qzx1[j] = qyz1[j] = qzx2[j] = qyz2[j] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 5; ++j)
+        xy1[j] = xy2[j] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        dz1[j] = dz2[j] = 0.0f;
+    float n1z = 0.0f, n2z = 0.0f; // d_z of the next plane
+    if (active) {
+        n1z = d1z[(long)p0 * sz + col];
+        n2z = d2z[(long)p0 * sz + col];
+    }
+    load_pw(p0 - R + 1);
+    fetch(p0);
+    commit(p0, 0);
+    if (p0 + 1 < pend)
+        fetch(p0 + 1);
+    __syncthreads();
+
+    for (int p = p0; p < pend; ++p) {
+        const int o = p - R, b = (p - p0) & 1;
+        const bool emit = o >= z0;
+        dz1[7] = n1z;
+        dz2[7] = n2z;
+        if (active && p + 1 < pend) {
+            n1z = d1z[(long)(p + 1) * sz + col];
+            n2z = d2z[(long)(p + 1) * sz + col];
+        }
+        if (p + 1 < pend)
+            commit(p + 1, b ^ 1);
+        if (p + 2 < pend)
+            fetch(p + 2);
+        float un = 0.0f, wn = 0.0f;
+        if (active) {
+            const float(*S1)[W] = s1[b];
+            const float(*S2)[W] = s2[b];
+#pragma unroll
+            for (int j = 0; j < 9; ++j) {
+                const int k = R - j;
+                if (k != 0) {
+                    const int ak = k < 0 ? -k : k;
+                    const float e = ecen(ak);
+                    qzx1[j] = fmaf(e, S1[ty + R][tx + R + k] - S1[ty + R][tx + R - k], qzx1[j]);
+                    qyz1[j] = fmaf(e, S1[ty + R + k][tx + R] - S1[ty + R - k][tx + R], qyz1[j]);
+                    qzx2[j] = fmaf(e, S2[ty + R][tx + R + k] - S2[ty + R][tx + R - k], qzx2[j]);
+                    qyz2[j] = fmaf(e, S2[ty + R + k][tx + R] - S2[ty + R - k][tx + R], qyz2[j]);
+                }
+            }
+            float a1 = 0, a2 = 0;
+#pragma unroll
+            for (int n = 1; n <= R; ++n) {
+                const float e = ecen(n);
+                a1 = fmaf(e,
+                          (S1[ty + R + n][tx + R + n] - S1[ty + R - n][tx + R + n]) +
+                              (S1[ty + R - n][tx + R - n] - S1[ty + R + n][tx + R - n]),
+                          a1);
+                a2 = fmaf(e,
+                          (S2[ty + R + n][tx + R + n] - S2[ty + R - n][tx + R + n]) +
+                              (S2[ty + R - n][tx + R - n] - S2[ty + R + n][tx + R - n]),
+                          a2);
+            }
+            xy1[4] = a1 * invdxdy;
+            xy2[4] = a2 * invdxdy;
+
+            if (emit) {
+                const float(*X1)[W] = x1[b];
+                const float(*X2)[W] = x2[b];
+                const float(*Y1)[BX] = y1[b];
+                const float(*Y2)[BX] = y2[b];
+                float fxx1 = 0, fxx2 = 0, fyy1 = 0, fyy2 = 0, fzz1 = 0, fzz2 = 0;
+#pragma unroll
+                for (int n = 1; n <= R; ++n) {
+                    const float c = cstg(n);
+                    fxx1 = fmaf(c, X1[ty][tx + R + n] - X1[ty][tx + R - n + 1], fxx1);
+                    fxx2 = fmaf(c, X2[ty][tx + R + n] - X2[ty][tx + R - n + 1], fxx2);
+                    fyy1 = fmaf(c, Y1[ty + R + n][tx] - Y1[ty + R - n + 1][tx], fyy1);
+                    fyy2 = fmaf(c, Y2[ty + R + n][tx] - Y2[ty + R - n + 1][tx], fyy2);
+                    fzz1 = fmaf(c, dz1[3 + n] - dz1[4 - n], fzz1);
+                    fzz2 = fmaf(c, dz2[3 + n] - dz2[4 - n], fzz2);
+                }
+                const float rho = 1.0f / pw[0];
+                const HV t1 = fwd_hv(fxx1, fyy1, fzz1, xy1[0], qzx1[0], qyz1[0], invdx * rho, invdy * rho, invdz * rho,
+                                     invdzdx, invdydz, pw[5], pw[6], pw[7]);
+                const HV t2 = fwd_hv(fxx2, fyy2, fzz2, xy2[0], qzx2[0], qyz2[0], invdx * rho, invdy * rho, invdz * rho,
+                                     invdzdx, invdydz, pw[5], pw[6], pw[7]);
+                const float mm1 = pw[1], mm2 = pw[2], mm3 = pw[3], mm4 = pw[4];
+                un = fmaf(fmaf(mm2, t2.v, fmaf(mm4, t1.v, __fmul_rn(mm1, t1.h))), dt, pw[8]);
+                wn = fmaf(fmaf(mm2, t1.h, fmaf(mm3, t2.v, __fmul_rn(mm4, t2.h))), dt, pw[9]);
+            }
+        }
+        // the pointwise words of the next output plane (their registers are free now), then this plane's stores
+        load_pw(o + 1);
+        if (active && emit) {
+            const long i = (long)o * sz + col;
+            u[i] = un;
+            w[i] = wn;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            qzx1[j] = qzx1[j + 1];
+            qyz1[j] = qyz1[j + 1];
+            qzx2[j] = qzx2[j + 1];
+            qyz2[j] = qyz2[j + 1];
+        }
+        qzx1[8] = qyz1[8] = qzx2[8] = qyz2[8] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            xy1[j] = xy1[j + 1];
+            xy2[j] = xy2[j + 1];
+        }
+#pragma unroll
+        for (int j = 0; j < 7; ++j) {
+            dz1[j] = dz1[j + 1];
+            dz2[j] = dz2[j + 1];
+        }
+        __syncthreads();
+    }
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -1769,7 +1996,11 @@ launch_update_rho_fwd_main_loop_2_1(float* field3, float* field4, const float* f
     }
     if (!ranges_ok(ixbeg, ixend, iybeg, iyend, izbeg, izend, ldimx, ldimy))
         return TTI_EINVAL;
-    return q ? tiled(k_fwd_update_q<BYS, R>, FWD_UPDATE_CHUNK, 2) : tiled(k_fwd_update<BYS>, FWD_UPDATE_CHUNK, 1);
+    if (!q)
+        return tiled(k_fwd_update<BYS>, FWD_UPDATE_CHUNK, 1);
+    const long n = (long)(ixend - ixbeg + 1) * (iyend - iybeg + 1) * (izend - izbeg + 1);
+    return n < FWD_UPDATE_SPLIT_BELOW ? tiled(k_fwd_update_q<BYS, R>, FWD_UPDATE_CHUNK, 2)
+                                      : tiled(k_fwd_update_qc<BYS>, FWD_UPDATE_CHUNK, 1);
 }
 
 int

@@ -94,6 +94,41 @@ def test_fwd_update(shape, rng, cuda):
     assert rel_l2(from_gpu(wg) - w0, wo - w0) < 1e-5
 
 
+@pytest.mark.parametrize("shape", [(130, 207, 235), (8, 4096, 184, 4)])
+def test_fwd_update_of_a_part_keeps_its_bits(shape, rng, cuda):
+    """Volumes of 6 million points and more take one thread per column, smaller ones one per column and field: the whole
+    volume in one call and its two halves in y as calls of their own give the same bits, and the oracle's values."""
+    import torch
+
+    from miniappsforhpe_amd import ops
+    from miniappsforhpe_amd._lib import call
+
+    G, OG = grid_pair(shape)
+    assert G.npoints >= 6_000_000 > G.npoints // 2 + G.nx * G.nz
+    # stiffness in m2/s2: the update is of the size of u, whose rounding (2^-24 |u|) is then under the 1e-5 asked of it
+    # (with stiffness 1 the update is 1e-3 of u and that rounding alone is 1e-4 of it)
+    m = [rng.uniform(0.5, 1.5, G.shape).astype(np.float32) * np.float32(1e7 if k < 4 else 1) for k in range(8)]
+    f, d, uw = ([rng.standard_normal(G.shape, dtype=np.float32) for _ in range(k)] for k in (2, 6, 2))
+    fg, dg, mg = ([to_gpu(x, cuda) for x in v] for v in (f, d, m))
+    whole, parts = ([to_gpu(x, cuda) for x in uw] for _ in range(2))
+    ops.fwd_update(G, *whole, dg, *fg, mg, 4e-4, DX, DY, DZ)
+    p = lambda *t: [x.data_ptr() for x in t]
+    x0, x1, y0, y1, z0, z1 = G.ranges
+    ym = y0 + (G.ny // 2 // 8 * 8 if G.ny > 1000 else G.ny // 2)
+    for ya, yb in ((y0, ym - 1), (ym, y1)):
+        call("launch_update_rho_fwd_main_loop_2_1", *p(*parts, dg[0], dg[3], dg[1], dg[4], dg[2], dg[5], *fg, mg[7],
+             *mg[:4], *mg[4:7]), *[None] * 12, x0, x1, ya, yb, z0, z1, G.ldx, G.ldy, 4e-4, DX, DY, DZ, 0, 8, 0, 0, 0,
+             torch.cuda.current_stream().cuda_stream)
+    c = O.fd_consts(DX, DY, DZ)
+    ref = [x.astype(np.float64) for x in uw]
+    O.fwd_update(OG, *ref, [x.astype(np.float64) for x in d], *[x.astype(np.float64) for x in f],
+                 [x.astype(np.float64) for x in m], O.f32(4e-4), c["invdx"], c["invdy"], c["invdz"], c["invdxy"],
+                 c["invdyz"], c["invdzx"])
+    for a, b, o, x in zip(whole, parts, ref, uw):
+        assert rel_l2(from_gpu(a) - x, o - x) < 1e-5
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_adj_drv(shape, rng, cuda):
     from miniappsforhpe_amd import ops
