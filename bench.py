@@ -42,7 +42,7 @@ def parse():
     ap.add_argument("--nt", type=int, default=100, help="forward (and adjoint) time steps per bench step")
     ap.add_argument("--k", type=int, default=4, help="snapshot / imaging interval (xcorr_step)")
     ap.add_argument("--snap", choices=["fp16", "bf16", "fp32"], default="fp16")
-    ap.add_argument("--zblock", type=int, default=0, help="z planes per block (0: autotuned with the strip)")
+    ap.add_argument("--zblock", type=int, default=0, help="most z planes per block (0: autotuned with the strip)")
     ap.add_argument("--strip", type=int, default=0, help="x tiles per strip of the block schedule (0: full rows)")
     ap.add_argument("--no-plain", action="store_true")
     ap.add_argument("--no-cpu", action="store_true")
@@ -186,7 +186,7 @@ def batched(torch, dev, args):
         passes()
     torch.cuda.synchronize()
     tb = (time.perf_counter() - t0) / reps
-    # the same shots one at a time (one launch per shot and step), z depth 32 for better fill of small volumes
+    # the same shots one at a time (one launch per shot and step), zblock 32 for better fill of small volumes
     descs = B._descs
     handles = []
     for i in range(len(descs)):

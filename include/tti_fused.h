@@ -52,8 +52,8 @@ typedef struct
  * plane are stored into it. free_surface != 0 applies the stress-free surface at plane izbeg as the reference's
  * mirrors do (kernel_loop4_derivatives on the z derivatives inside the sweep, then kernel_loop4_inner on field*_out;
  * field1/field2 must already be mirrored, as the previous step or kernel_loop4_inner leaves them). zblock = most z
- * planes per thread block (0 = 128; blocks take fewer where that fills the GPU better); strip = block schedule: the x-y tiles of a z chunk are visited in vertical strips
- * of `strip` tiles of 64 columns (0 = full rows). zblock and strip change the speed, never the result.
+ * planes per thread block (0 = 128; blocks take fewer where that fills the GPU better); strip = block schedule: the x-y
+ * tiles of a z chunk are visited in vertical strips of `strip` tiles of 64 columns (0 = full rows). zblock and strip change the speed, never the result.
  * Replaces the forward sequence of simulator2SetUp::execute (simulator2/simulator2SetUp.cu:536-599) on one volume. */
 int tti_fused_fwd_step(const float* field1, const float* field2, float* field1_out, float* field2_out, float* field3,
                        float* field4, const float* model1, const float* model2, const float* model3,

@@ -1,11 +1,10 @@
-"""Autotuner for the fused time steps: picks the z depth of the thread blocks (planes per block, the length of the
-register queue's march) and the block schedule (x tiles per strip) by timing candidate launches on the caller's own
-volumes.
+"""Autotuner for the fused time steps: picks the most z planes a thread block may hold (zblock, the longest march of the
+register queues) and the block schedule (x tiles per strip) by timing candidate launches on the caller's own volumes.
 
-The tile shape in x-y is fixed by the kernels (64 x 4 rows forward, 64 x 8 rows adjoint, two and one blocks per CU).
-The z depth trades the 8 halo planes every block re-reads and recomputes against the number of blocks that fill the
-256 CUs: a 512^3 volume runs best at 256 planes, a batch of small apertures or a single small volume may want fewer.
-The strip width decides which tiles run at the same time on one XCD: full rows share x halos perfectly, narrower
+The tile shape in x-y is fixed by the kernels (64 x 8 columns of 2 threads each, one block per CU). Within zblock the
+launchers take the depth that best trades the 8 (forward) or 11 (adjoint) planes every block recomputes against the
+number of blocks that fill the 256 CUs, so zblock matters for large volumes (512^3 runs best at 256 planes); on small
+ones several candidates are the same launch, and which of them is kept makes no difference. The strip width decides which tiles run at the same time on one XCD: full rows share x halos perfectly, narrower
 strips bring more y neighbours into the same L2 at once. Timing is by HIP events on the current stream around a few
 forward and adjoint steps (no snapshots, no imaging: those add the same cost to every candidate). Neither knob
 changes a result bit (each point is computed by the same code whichever block computes it).
@@ -52,7 +51,7 @@ def tune_propagator(P, zblocks=ZBLOCKS, strips=STRIPS, reps: int = 3) -> dict:
 
 
 def tune_batch(B, zblocks=ZBLOCKS, strips=STRIPS, reps: int = 2) -> dict:
-    """Rebuilds the batch with the fastest (z depth, strip) for one batched forward + adjoint step (all shots in one
+    """Rebuilds the batch with the fastest (zblock, strip) for one batched forward + adjoint step (all shots in one
     launch each). The shots' state is left at rest. Returns {"zblock", "strip", "ms": {...}}."""
     from ._lib import call
 

@@ -178,8 +178,8 @@ class BatchFWI:
         self.retile(zblock, strip)
 
     def retile(self, zblock: int, strip: int = 0):
-        """Rebuilds the shot table with `zblock` z planes per thread block and the block schedule `strip` (x tiles per
-        strip, 0 = full rows); captured graphs are dropped."""
+        """Rebuilds the shot table with at most `zblock` z planes per thread block and the block schedule `strip`
+        (x tiles per strip, 0 = full rows); captured graphs are dropped."""
         self.close()
         self.zblock, self.strip = zblock, strip
         self._descs = (TTIShot * len(self.shots))(*[s.desc(self.nt, zblock, strip) for s in self.shots])

@@ -6,7 +6,7 @@ FP64 images summed into the model-sized gradient in FP64.
 
 Defaults are the workload: 64 apertures of 128-320 cells per axis (seed 1004) from a 1024 x 1024 x 400 layered TTI
 model, 1500 steps, 12 Hz Ricker sources 8 planes below each aperture's top, 64 receivers per shot, observed data =
-0.8 x each shot's synthetic data (made beforehand by a forward pass without snapshots). The block schedule (z depth,
+0.8 x each shot's synthetic data (made beforehand by a forward pass without snapshots). The block schedule (zblock,
 strip width) is chosen by the autotuner. `--snap-budget-gb` bounds the checkpoints plus snapshot slots of all shots
 together; the rest of the device footprint (models, two state sets, images) is fixed by the apertures.
 Prints one JSON line: plan, timings of the gradient (first forward, re-run forwards, adjoint) and updates/s.

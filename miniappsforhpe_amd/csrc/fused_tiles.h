@@ -73,20 +73,6 @@ mirror_dz(float (&q)[N])
         q[C + k] = q[C + 7 - k];
 }
 
-__device__ __forceinline__ bool
-interior(const Box& g, int x, int y, int z)
-{
-    return x >= g.ixbeg && x <= g.ixend && y >= g.iybeg && y <= g.iyend && z >= g.izbeg && z <= g.izend;
-}
-
-// valid (allocated) region: interior plus a 4-point ghost rim
-__device__ __forceinline__ bool
-allocated(const Box& g, int x, int y, int z)
-{
-    return x >= g.ixbeg - R && x <= g.ixend + R && y >= g.iybeg - R && y <= g.iyend + R && z >= g.izbeg - R &&
-           z <= g.izend + R;
-}
-
 // Block schedule within one z chunk: tile r -> (bxi, byi). strip <= 0 or >= ntx: x fastest over full rows; otherwise
 // the chunk is cut into vertical strips of `strip` x tiles (the last one narrower), x fastest within a strip, then y,
 // strip after strip. Narrow strips keep the blocks that run at the same time on one XCD closer together in x-y
@@ -220,27 +206,6 @@ snap_decode(int mode, SnapWord r)
     return 0.0f;
 }
 
-// Masked float4 load of 4 consecutive x points starting at gx (gx = 0 mod 4). Points outside the allocated
-// x range [ixbeg-4, ixend+4] read as zero; quads wholly outside are not loaded. With ixbeg = 0 mod 4 and
-// ldx = 0 mod 4 (checked by the launchers) a quad that overlaps the allocated range lies inside [0, ldx).
-__device__ __forceinline__ float4
-load_quad(const float* __restrict__ base, long idx, int gx, const Box& g, bool rowok)
-{
-    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (rowok && gx + 3 >= g.ixbeg - R && gx <= g.ixend + R) {
-        v = *reinterpret_cast<const float4*>(base + idx);
-        const int lim = g.ixend + R - gx; // last valid element offset within the quad
-        if (lim < 3) {
-            if (lim < 1)
-                v.y = 0.0f;
-            if (lim < 2)
-                v.z = 0.0f;
-            v.w = 0.0f;
-        }
-    }
-    return v;
-}
-
 constexpr int TQ_PER_ROW = TW / 4, BQ_PER_ROW = BW / 4; // quads per row of the two tile shapes
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -258,12 +223,12 @@ constexpr int TQ_PER_ROW = TW / 4, BQ_PER_ROW = BW / 4; // quads per row of the 
 //   D  D+ of d_x, d_y; update and store plane o, load the pointwise words of plane o + 1
 // Planes p outside the chunk feed only z stencils, so their bodies leave d_x, d_y and the x-y term out.
 //
-// What bounds it (512^3, 2.2 GHz under load): VALU issue 58% and LDS 50% of the time in lock-step phases, 11.0 GB moved
-// (4.1 of the 4.97 TB/s of a copy; with six model volumes aliased, 3.2 GB less, it runs 8% faster). One thread per column
-// needed 253 VGPRs (8 waves a CU) where one per column and field takes 120 (16 waves); the tile of 8 rows instead of 4
-// reads 40% fewer halo quads and computes 2 instead of 3 d_y per column, the second barrier went, and the partial sums
-// shift as they are summed. Together 2.82 -> 2.67 ms per step, 2.98 -> 2.90 ms with the FP16 snapshot, and with the
-// shortened rim planes 27 -> 17 us at 64^3. Blocks of 4 rows, two a CU: 2.83 ms.
+// What bounds it (512^3): VALU issue 66% and LDS 58% of the busy cycles in lock-step phases, and 11.1 GB moved, at 2.34 ms
+// 4.7 TB/s, about what a copy reaches (with one volume in the place of seven models it runs 12% faster). One thread per
+// column needed 253 VGPRs (8 waves a CU) where one per column and field takes 122 (16 waves); the tile of 8 rows instead of
+// 4 reads 40% fewer halo quads and computes 2 instead of 3 d_y per column, the second barrier went, and the partial sums
+// shift as they are summed. With the loads below, 2.78 -> 2.48 ms per step, 2.98 -> 2.74 ms with the FP16 snapshot (one
+// box, in turn; other boxes take 2.3), and with the shortened rim planes 64^3 27 -> 17 us.
 //
 // Global addresses are 32-bit byte offsets from the (scalar) base pointers: the launcher checks that every volume is
 // smaller than 4 GiB.
@@ -321,15 +286,8 @@ stg8(F&& v)
     return a;
 }
 
-#ifndef TTI_FWD_BY
-#define TTI_FWD_BY 8
-#endif
-constexpr int FWD_BY = TTI_FWD_BY; // rows per forward block
-#ifndef TTI_FWD_SETPRIO
-#define TTI_FWD_SETPRIO 1
-#endif
-constexpr int FU = 2; // forward planes per loop iteration
-constexpr bool FWD_SETPRIO = TTI_FWD_SETPRIO != 0;
+constexpr int FWD_BY = 8; // rows per forward block (STEP_SLOTS, STEP_WARM and the launch bounds hold for these)
+constexpr int FU = 2;     // forward planes per loop iteration
 
 // One block's tile (bxi, byi, bzi) of a forward step; called by the single-volume kernel and the batched one. One thread
 // per column and field (threadIdx.z: 0 sigma_H and u, 1 sigma_V and w).
@@ -485,15 +443,13 @@ fwd_tile(const float* __restrict__ s1, const float* __restrict__ s2, float* __re
         // ---- A: this plane's loads first, so that waiting for them never waits for the stores below (one counter covers
         // loads and stores): the column word of plane o + 8; the tile of plane p + 1 goes to the other buffer (last read
         // before the previous plane's barrier) and the tile of plane p + 2 is fetched
-        if (FWD_SETPRIO)
-            __builtin_amdgcn_s_setprio(3);
+        __builtin_amdgcn_s_setprio(3);
         sq[cur + 8] = col(o + 8);
         if (own || p + 1 <= z1 + R - 1)
             commit(par ^ 1);
         if (own || p + 2 <= z1 + R - 1)
             fetch(p + 2);
-        if (FWD_SETPRIO)
-            __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_s_setprio(0);
         const float(*t)[TW] = T[par][F];
         // ---- B: the z-mixed partial sums; from the planes whose own outputs this block computes also the x-y mixed term,
         // d_x on rows of the tile (x' in [x0-4, x0+68)) and d_y on columns (y' in [y0-4, y0+BY+4)) (the scale is zero for
@@ -719,9 +675,11 @@ adj_half(int t, int& row, int& lx)
 }
 
 // One block's tile of an adjoint step; SNAP = snapshot mode of the imaging condition (TTI_SNAP_NONE: no imaging). One
-// thread per column and field (threadIdx.z: 0 sigma_H and u, 1 sigma_V and w): VALU, LDS and the latency between them
-// bound it together (57 B/pt at the copy rate are 1.5 of 3.4 ms at 512^3), so what counts is waves to fill the gaps: one
-// thread per column held both fields' queues in 256 registers, 8 waves per CU; this holds 16. Each temporary is formed
+// thread per column and field (threadIdx.z: 0 sigma_H and u, 1 sigma_V and w). At 512^3 it moves 96 B a point (12.9 GB of
+// the 8.6 it needs: 10 words per footprint point), 3.8 TB/s or 0.8 of a copy's rate; VALU is busy 51% and LDS 43% of the
+// cycles. With one volume in the place of seven models it takes 2.74 instead of 3.39 ms: a fifth of the time is the models'
+// reads, the rest VALU, LDS and the latency between barriers, where what counts is waves to fill the gaps: one thread per
+// column held both fields' queues in 256 registers, 8 waves per CU; this holds 16. Each temporary is formed
 // once, by the thread that loaded its half-quad, for both fields. S_z comes with the tile, so no second stream of 6
 // volumes runs 7 planes ahead, at the price of 3 more recomputed planes per chunk, which form S_z alone. One barrier per
 // plane: X and Y are written before it and read after it, the tiles of the next plane go into the other buffer.

@@ -10,8 +10,8 @@
 
 namespace tti {
 
-// both kernels: one block per CU; 8 halo planes and the prologue (64^3: forward 98 -> 17 us, adjoint 134 -> 23 us
-// against 64-plane chunks)
+// both kernels: one block per CU (196 and 240 VGPRs); 8 halo planes and the prologue (64^3: forward 98 -> 17 us, adjoint
+// 134 -> 23 us against 64-plane chunks)
 constexpr Chunk T1_CHUNK{ 1, 9.0f };
 
 

@@ -16,21 +16,22 @@
 
 namespace tti {
 
-// {resident blocks per CU, planes' worth of a chunk's prologue and halo, deepest chunk} of the launchers below. Against
-// chunks of 64 planes on grids too small for 512 deeper ones, at 64^3: derivatives 70 -> 30 us (then host time), update
-// 122 -> 21, adjoint derivatives 143 -> 36, adjoint update 70 -> 15, density gradient 149 -> 19 us.
+// {blocks per CU that make a round, planes' worth of a chunk's prologue and halo, deepest chunk} of the launchers below.
+// Against chunks of 64 planes on grids too small for 512 deeper ones, at 64^3: derivatives 70 -> 7 us, update 122 -> 15,
+// adjoint derivatives 143 -> 20, adjoint update 69 -> 6, density gradient 147 -> 12 us.
 constexpr Chunk FWD_DRV_CHUNK{ 1, 4.0f }, FWD_UPDATE_CHUNK{ 1, 9.5f }, ADJ_DRV_CHUNK{ 1, 9.0f },
     RHO_GRAD_CHUNK{ 1, 3.0f };
 // Points below which the order-8 forward update takes a thread per column and field. One thread per column against two:
 // 64^3 16.7 and 15.1 us, 128^3 45.6 and 41.0, 150 x 203 x 117 89.9 and 81.3, 200 x 300 x 100 157.0 and 157.0, 192^3 150.8
 // and 153.8, 301 x 217 x 190 277 and 282, 400^3 1321 and 1405, 480^3 2174 and 2397, 512^3 2504 and 2552.
 constexpr long FWD_UPDATE_SPLIT_BELOW = 6000000;
-// the adjoint update runs in dispatch order, where chunks over 64 planes read more (1.37 ms at 64, 1.43 at 256, 512^3)
+// the adjoint update runs in dispatch order, where chunks over 64 planes gain nothing (512^3 1.43 ms at 64 and at 256
+// planes, 640 x 480 x 300 1.06 ms at 60 and 1.10 at 150)
 constexpr Chunk ADJ_UPDATE_CHUNK{ 1, 4.0f, 64 };
-// order 16: 16 halo planes
+// order 16: 16 halo planes. Two blocks of the adjoint update fit a CU, but priced so, with chunks half as deep, it is 3%
+// slower on average over 18 volumes of 42 to 224 points a side (155 x 206 x 49: 28.3 -> 32.0 us, 224 x 43 x 42: 9.6 -> 8.7)
 constexpr Chunk FWD_DRV16_CHUNK{ 1, 6.0f }, FWD_UPDATE16_CHUNK{ 1, 17.5f }, ADJ_DRV16_CHUNK{ 1, 17.0f },
     ADJ_UPDATE16_CHUNK{ 1, 6.0f, 64 };
-
 
 // ------------------------------------------------------------------------------------------------------------------
 // a2: d_a f = b * D-_a f  (kernels/kernel_type2_fwd_drv.cu:148-362; launcher :368-409)

@@ -108,7 +108,7 @@ class TTIPropagator:
         else:
             self.sponge = tuple(t.to(self.device, torch.float32).contiguous() for t in sponge)
         self._unit = None
-        self.zblock = zblock  # z planes per thread block of the fused steps
+        self.zblock = zblock  # most z planes per thread block of the fused steps
         self.strip = strip    # block schedule: x tiles per strip (0 = full rows); see miniappsforhpe_amd.autotune
         # stress-free surface at the top interior plane: the reference's mirrors (kernel_loop4_inner on sigma after
         # each time update, kernel_loop4_derivatives on the derivatives) on both paths
